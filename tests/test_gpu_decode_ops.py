@@ -132,3 +132,25 @@ def test_masked_argmax(cuda, dtype):
         want = _reference_sampling(logits, b, p)
         torch.cuda.synchronize()
         assert torch.equal(got, want), (got != want).nonzero()[:5].tolist()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("V", [1, 7, 8, 9, 8191, 8193, 57344, 57353])
+def test_masked_argmax_vector_edges(cuda, dtype, V):
+    """Row lengths around the 8-token loads and one round of them (57344), rows and mask rows at
+    odd offsets (unaligned loads), the maximum at the first, last and last vectorised token; whole
+    numbers compared exactly."""
+    from whisperdrz_amd import masked_argmax
+
+    g = torch.Generator(device=cuda).manual_seed(V)
+    rows = 5
+    logits = torch.randn(rows, V + 3, generator=g, device=cuda).to(dtype)[:, 1 : V + 1]
+    blocked = (torch.rand(rows, V + 5, generator=g, device=cuda) < 0.2)[:, 3:]
+    penalty = (torch.rand(rows, V + 2, generator=g, device=cuda) < 0.2)[:, 1:]
+    for row, i in ((0, 0), (1, V - 1), (2, V // 8 * 8 - 1), (3, V // 2)):
+        logits[row, max(i, 0)] = 9.0
+    logits[4] = float("-inf")
+    for b, p in [(blocked, penalty), (None, None)]:
+        got = masked_argmax(logits, b, p)
+        want = _reference_sampling(logits, b[:, :V] if b is not None else None, p[:, :V] if p is not None else None)
+        assert torch.equal(got, want), (V, got.tolist(), want.tolist())
