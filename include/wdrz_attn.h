@@ -243,7 +243,7 @@ int wdrz_masked_argmax(int dtype, const void* logits, int64_t logits_stride,
                        int64_t penalty_stride, int64_t* out, int64_t rows, int64_t V, void* stream);
 
 /*
- * Workspace (bytes) for wdrz_log_mel: the [202, n_mels] filterbank and one maximum per window.
+ * Workspace (bytes) for wdrz_log_mel: the partial maxima of each window.
  * No counterpart in the reference (torchaudio keeps the filterbank in a module buffer).
  */
 size_t wdrz_log_mel_workspace_size(int64_t B, int64_t n_mels);

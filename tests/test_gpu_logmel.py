@@ -56,6 +56,22 @@ def test_lengths_padding_truncation(cuda, n, target):
     _check(got, log_mel_ref(x, 128, target), f"n={n} target={target}")
 
 
+@pytest.mark.parametrize("n_mels", [1, 2, 79, 128])
+@pytest.mark.parametrize("frames", [1, 6, 29, 30, 31, 61, 3842])
+def test_tile_edges(cuda, n_mels, frames):
+    """Frame counts around the 30-frame workgroups and past 128 of them (a workgroup then takes
+    several), filter counts at the ends of their range, rows that do not start 16-byte aligned.
+    fp32 rounding (6e-8 a step, some ten steps) on the weakest of ~1e6 noise bins (1e-3 of the mean
+    amplitude) is 6e-4 of that bin, 1.3e-4 after the log: the file's tolerance."""
+    from whisperdrz_amd import log_mel_spectrogram
+
+    n = max(201, frames * 160 + 37)
+    x = np.stack([_noise(n, frames), _noise(n, frames + 1)])
+    got = log_mel_spectrogram(torch.from_numpy(x).to(cuda), n_mels)
+    for i in range(2):
+        _check(got[i], log_mel_ref(x[i], n_mels), f"frames={frames} window {i}")
+
+
 def test_list_and_silence(cuda):
     # the transcriber's call shape: a list of CPU windows of different lengths, padded to 3000
     from whisperdrz_amd import LogMelSpectrogram

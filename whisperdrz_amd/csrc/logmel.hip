@@ -7,21 +7,25 @@
 //   log10(max(mel, 1e-10)) -> max(log, max_over_window - 8) -> (x + 4) / 4 -> pad with -1.5 /
 //   truncate to target_frames.
 //
-// Three launches:
-//   logmel_init_kernel   the [201, n_mels] filterbank and the cosine / Hann tables (computed in
-//                        double, stored fp32) and each window's running maximum, into the
-//                        workspace
-//   logmel_spec_kernel   one workgroup per (32 frames, window), 4 wavefronts. The frames' samples
-//                        (overlapping by 240) are staged once in LDS with the reflect padding;
-//                        the windowed DFT is a [32 frames x 400 samples] x [400 x 256 bins]
-//                        product on the fp32 matrix cores (v_mfma_f32_32x32x2_f32: real and
-//                        imaginary parts as two accumulators over the same A operand; cosines
-//                        from a 400-entry LDS table indexed by i*k mod 400). The power spectrum
-//                        goes to LDS, a second product [32 x 202] x [202 x n_mels] applies the
-//                        filterbank, and log10 is stored with the window maximum folded in by
-//                        an atomic max.
+// Two launches:
+//   logmel_spec_kernel   one workgroup per (30 frames, window), 5 wavefronts of 6 frames. The
+//                        frames' samples (overlapping by 240) are staged once in LDS with the
+//                        reflect padding; each wavefront runs its frames' real 400-point
+//                        transforms as complex 200-point ones (even samples + i odd samples) in
+//                        registers and LDS, the powers go to LDS, and the filterbank is applied
+//                        as the two weights each bin has; log10 is stored, and the workgroup's
+//                        maximum of its window goes to the workspace.
 //   logmel_finish_kernel (max(x, max - 8) + 4) / 4, and -1.5 past the last frame.
-// fp32 throughout, like the reference; the DFT sums 400 products per bin in fp32.
+// fp32 throughout, like the reference; window, twiddles and filterbank are computed in double and
+// rounded once.
+//
+// Why an FFT: the direct transform on the fp32 matrix cores (a [32 x 400] x [400 x 512] product
+// per 32 frames, the form before this one) took 240 us for 16 windows of 30 s and 50 us for one,
+// after an init launch that rebuilt its tables (3.3 us); the 55 MB this must move take 11 us. Now
+// 63 us for 16 windows and 14.5 us for one (a whole call 237 -> 76 and 53.6 -> 17 us), and nearer
+// to 64-bit results (3.7e-7 against 4.9e-7). What bounds it is the sum of VALU and LDS issue per
+// wavefront (the phases of a workgroup's wavefronts coincide): without the transforms' arithmetic
+// 60 us, without the filterbank's loop 51 us, without building the filter weights 60 us.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -33,216 +37,384 @@ namespace {
 
 constexpr int kNfft = 400;
 constexpr int kHop = 160;
-constexpr int kBins = kNfft / 2 + 1;     // 201
-constexpr int kBinTiles = 8;             // 256 bins computed (2 tiles per wavefront), 201 kept
-constexpr int kFrames = 32;              // frames per workgroup
-constexpr int kSeg = (kFrames - 1) * kHop + kNfft;  // 5360 samples
-constexpr int kPPitch = 225;             // power tile pitch (odd: conflict-free column reads)
-constexpr int kKMel = 202;               // filterbank rows incl. one zero row (K multiple of 2)
-// Samples are stored with one pad float per 32 (position j + j/32): the 32 frames a wavefront
-// reads at once are 160 samples apart, which would otherwise fall into 2 of the 64 LDS banks.
-constexpr int kSegStored = kSeg + kSeg / 32 + 1;
-__device__ __forceinline__ int seg_pos(int j) { return j + (j >> 5); }
-
-typedef float f32x16v __attribute__((ext_vector_type(16)));
-
-__device__ __forceinline__ f32x16v mfma32x2(float a, float b, f32x16v c) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+constexpr int kBins = kNfft / 2 + 1;  // 201
+constexpr int kHalf = kNfft / 2;      // length of the complex transform
+constexpr int kWaveFrames = 6;        // 60 of 64 lanes: 10 lanes a frame, then 20 lanes two frames
+constexpr int kWaves = 5;
+constexpr int kThreads = 64 * kWaves;
+constexpr int kFrames = kWaveFrames * kWaves;  // 30 a workgroup: 100 workgroups a 30-s window
+constexpr int kSeg = (kFrames - 1) * kHop + kNfft;  // samples a workgroup stages
+constexpr int kSegLoads = (kSeg + kThreads - 1) / kThreads;
+// Samples are stored with 52 floats of padding per hop: the frames of a wavefront then start 20
+// banks apart, so the 10 float2 each reads at once fall in different banks.
+constexpr int kHopPad = 52;
+__device__ __forceinline__ int seg_pos(int j) { return j + kHopPad * (j / kHop); }
+// A frame's 200 complex values, and 2 of padding (202 = 10 mod 32: the 10-lane groups of the first
+// stage write different banks). A wavefront's 6 frames are its own region, reused for the powers.
+constexpr int kFramePitch = kHalf + 2;                   // float2
+constexpr int kWaveFloats = 2 * kWaveFrames * kFramePitch;
+// Powers: four bins of a frame together, [bin / 4][frame][4] within the wavefront's region, so that
+// the filterbank reads four bins per lane at once. Odd wavefronts' powers start 32 floats in: the
+// 30 frames' reads then spread evenly over the banks.
+constexpr int kPGroups = (kBins + 3) / 4;  // the last 3 of 204 stay zero
+__device__ __forceinline__ int power_pos(int wave, int fr, int k) {
+  return wave * kWaveFloats + 32 * (wave & 1) + ((k >> 2) * kWaveFrames + fr) * 4 + (k & 3);
 }
+constexpr int kMaxMels = 128;
+// filter m's weights, in groups of four bins aligned like the powers: the groups from bin
+// start[m] / 4 * 4 on, at group (start[m] + start[m + 1] + 6 m) / 4. A filter of n bins touches at
+// most (n + 6) / 4 groups, which is what the next filter's place is further on.
+constexpr int kWeights = ((2 * kBins + 6 * kMaxMels) / 4 + 4) * 4;
+constexpr int kMaxParts = 128;  // workgroups a window (= maxima in the workspace)
+static_assert(kSeg + kHopPad * (kSeg / kHop) + 1 <= kWaves * kWaveFloats, "sample buffer");
+static_assert(32 + 4 * kWaveFrames * kPGroups <= kWaveFloats, "power tile");
 
-// Ordered encoding of floats so that an unsigned max is a float max (negative values reversed).
-__device__ __forceinline__ uint32_t order_key(float f) {
-  const uint32_t u = __float_as_uint(f);
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-__device__ __forceinline__ float order_val(uint32_t k) {
-  return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
-}
-
-// Slaney mel scale (3 mels per 200 Hz below 1 kHz, 27 mels per factor 6.4 above).
-__device__ double hz_to_mel(double f) {
-  const double f_sp = 200.0 / 3.0;
-  if (f < 1000.0) return f / f_sp;
-  return 1000.0 / f_sp + log(f / 1000.0) / (log(6.4) / 27.0);
-}
-__device__ double mel_to_hz(double m) {
-  const double f_sp = 200.0 / 3.0, min_log_mel = 1000.0 / f_sp;
-  if (m < min_log_mel) return f_sp * m;
-  return 1000.0 * exp(log(6.4) / 27.0 * (m - min_log_mel));
-}
-
-// fb[k][m] (row k = frequency bin, kKMel rows, row 201 zero), the window maxima, and the
-// cosine / Hann tables (400 entries each, computed in double).
-__global__ __launch_bounds__(256) void logmel_init_kernel(LogMelArgs a) {
-  const int idx = blockIdx.x * 256 + threadIdx.x;
-  if (idx < a.B) a.gmax[idx] = order_key(-INFINITY);
-  if (idx < kNfft) {
-    double sn, c;
-    sincospi(2.0 * idx / kNfft, &sn, &c);
-    a.tables[idx] = (float)c;
-    a.tables[kNfft + idx] = (float)(0.5 - 0.5 * c);  // periodic Hann
+// ---- tables, computed at compile time in double -------------------------------------------------
+constexpr double kPi = 3.14159265358979323846;
+// Taylor series on |x| <= pi/4 (the next term is below 1e-20)
+constexpr double sin_series(double x) {
+  double t = x, s = x;
+  for (int i = 1; i < 10; ++i) {
+    t *= -x * x / ((2 * i) * (2 * i + 1));
+    s += t;
   }
-  if (idx >= kKMel * a.n_mels) return;
-  const int k = idx / a.n_mels, m = idx % a.n_mels;
-  float v = 0.f;
-  if (k < kBins) {
-    const double mel_max = hz_to_mel(8000.0);
-    const double f0 = mel_to_hz(mel_max * m / (a.n_mels + 1));
-    const double f1 = mel_to_hz(mel_max * (m + 1) / (a.n_mels + 1));
-    const double f2 = mel_to_hz(mel_max * (m + 2) / (a.n_mels + 1));
-    const double f = 8000.0 * k / (kBins - 1);
-    const double down = (f - f0) / (f1 - f0), up = (f2 - f) / (f2 - f1);
-    double t = down < up ? down : up;
-    t = t > 0.0 ? t : 0.0;
-    v = (float)(t * 2.0 / (f2 - f0));
+  return s;
+}
+constexpr double cos_series(double x) {
+  double t = 1.0, s = 1.0;
+  for (int i = 1; i < 10; ++i) {
+    t *= -x * x / ((2 * i - 1) * (2 * i));
+    s += t;
   }
-  a.fb[idx] = v;
+  return s;
+}
+// cos(2 pi t / n) for 0 <= t <= n, n a multiple of 8, folded to the first eighth of a turn
+constexpr double cos_turn(int t, int n) {
+  if (2 * t > n) t = n - t;
+  if (4 * t > n) return -cos_turn(n / 2 - t, n);
+  if (8 * t > n) return sin_series(2.0 * kPi * (n / 4 - t) / n);
+  return cos_series(2.0 * kPi * t / n);
+}
+constexpr double sin_turn(int t, int n) { return 4 * t >= n ? cos_turn(t - n / 4, n) : cos_turn(t + 3 * n / 4, n); }
+
+struct MelTables {
+  float window[kNfft];      // periodic Hann, halved (the even / odd split's 1/2)
+  float2 tw[20 * 10];       // e^(-2 pi i n1 k1 / 200) at [k1][n1]
+  float2 split[kHalf / 2 + 1];  // e^(-2 pi i k / 400)
+};
+constexpr MelTables make_tables() {
+  MelTables m{};
+  for (int i = 0; i < kNfft; ++i) m.window[i] = 0.5f * (float)(0.5 - 0.5 * cos_turn(i, kNfft));
+  for (int k1 = 0; k1 < 20; ++k1)
+    for (int n1 = 0; n1 < 10; ++n1) {
+      m.tw[k1 * 10 + n1].x = (float)cos_turn(n1 * k1, kHalf);
+      m.tw[k1 * 10 + n1].y = (float)-sin_turn(n1 * k1, kHalf);
+    }
+  for (int k = 0; k <= kHalf / 2; ++k) {
+    m.split[k].x = (float)cos_turn(k, kNfft);
+    m.split[k].y = (float)-sin_turn(k, kNfft);
+  }
+  return m;
+}
+__device__ constexpr MelTables kTables = make_tables();
+
+// ---- small transforms (forward, e^(-i)) -----------------------------------------------------------
+struct Cplx {
+  float r, i;
+};
+__device__ __forceinline__ Cplx operator+(Cplx a, Cplx b) { return {a.r + b.r, a.i + b.i}; }
+__device__ __forceinline__ Cplx operator-(Cplx a, Cplx b) { return {a.r - b.r, a.i - b.i}; }
+
+__device__ __forceinline__ void dft5(const Cplx* x, Cplx* y) {
+  constexpr float c1 = (float)cos_turn(8, 40), c2 = (float)cos_turn(16, 40);
+  constexpr float s1 = (float)sin_turn(8, 40), s2 = (float)sin_turn(16, 40);
+  const Cplx t1 = x[1] + x[4], t2 = x[2] + x[3], t3 = x[1] - x[4], t4 = x[2] - x[3];
+  y[0] = x[0] + t1 + t2;
+  const Cplx m1 = {x[0].r + c1 * t1.r + c2 * t2.r, x[0].i + c1 * t1.i + c2 * t2.i};
+  const Cplx m2 = {x[0].r + c2 * t1.r + c1 * t2.r, x[0].i + c2 * t1.i + c1 * t2.i};
+  const Cplx n1 = {s1 * t3.r + s2 * t4.r, s1 * t3.i + s2 * t4.i};
+  const Cplx n2 = {s2 * t3.r - s1 * t4.r, s2 * t3.i - s1 * t4.i};
+  y[1] = {m1.r + n1.i, m1.i - n1.r};  // m1 - i n1
+  y[4] = {m1.r - n1.i, m1.i + n1.r};
+  y[2] = {m2.r + n2.i, m2.i - n2.r};
+  y[3] = {m2.r - n2.i, m2.i + n2.r};
 }
 
-__global__ __launch_bounds__(256) void logmel_spec_kernel(LogMelArgs a) {
+// 20 and 10 points by the prime-factor map (n = 5a + 4b, k = 5q + 16r mod 20; n = 5a + 2b,
+// k = 5q + 6r mod 10): no twiddles between the factors.
+__device__ __forceinline__ void dft20(Cplx* v) {
+  Cplx f[4][5];
+#pragma unroll
+  for (int b = 0; b < 5; ++b) {
+    const Cplx x0 = v[(4 * b) % 20], x1 = v[(5 + 4 * b) % 20], x2 = v[(10 + 4 * b) % 20], x3 = v[(15 + 4 * b) % 20];
+    const Cplx p = x0 + x2, m = x0 - x2, q = x1 + x3, n = x1 - x3;
+    f[0][b] = p + q;
+    f[2][b] = p - q;
+    f[1][b] = {m.r + n.i, m.i - n.r};  // m - i n
+    f[3][b] = {m.r - n.i, m.i + n.r};
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    Cplx y[5];
+    dft5(f[q], y);
+#pragma unroll
+    for (int r = 0; r < 5; ++r) v[(5 * q + 16 * r) % 20] = y[r];
+  }
+}
+__device__ __forceinline__ void dft10(Cplx* v) {
+  Cplx f[2][5];
+#pragma unroll
+  for (int b = 0; b < 5; ++b) {
+    const Cplx x0 = v[(2 * b) % 10], x1 = v[(5 + 2 * b) % 10];
+    f[0][b] = x0 + x1;
+    f[1][b] = x0 - x1;
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    Cplx y[5];
+    dft5(f[q], y);
+#pragma unroll
+    for (int r = 0; r < 5; ++r) v[(5 * q + 6 * r) % 10] = y[r];
+  }
+}
+
+// Edge j of the slaney mel filters (3 mels per 200 Hz below 1 kHz, 27 mels per factor 6.4 above):
+// n_mels + 2 points evenly spaced in mels over [0, 8 kHz].
+__device__ __forceinline__ double mel_edge(int j, int n_mels) {
+  const double f_sp = 200.0 / 3.0, logstep = 0.068751777420949123;  // log(6.4) / 27
+  const double mel_max = 15.0 + 2.0794415416798357 / logstep;       // log(8000 / 1000) = 2.079...
+  const double m = mel_max * j / (n_mels + 1);
+  return m < 15.0 ? f_sp * m : 1000.0 * exp(logstep * (m - 15.0));
+}
+
+// LDS ops of one wavefront run in order: between its own writes and reads only the compiler has to
+// be kept from moving them.
+__device__ __forceinline__ void wave_fence() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront"); }
+
+__global__ __launch_bounds__(kThreads) void logmel_spec_kernel(LogMelArgs a) {
   const int b = blockIdx.y;
-  const int f0 = blockIdx.x * kFrames;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int tid = threadIdx.x;
   const int N = a.n_samples;
 
-  static_assert(kSegStored <= kFrames * kPPitch, "sample buffer");
-  __shared__ float seg_p[kFrames * kPPitch];  // samples during the DFT, then the power tile
-  __shared__ float win[kNfft];
-  __shared__ float ctab[kNfft];
-  __shared__ uint32_t wmax[4];
+  __shared__ __align__(16) float buf[kWaves * kWaveFloats];  // samples, then transforms and powers
+  __shared__ __align__(16) float wts[kWeights];
+  __shared__ uint8_t start[kMaxMels + 2];  // first bin at or above each edge
+  __shared__ float wmax[kWaves];
+  double* edges = reinterpret_cast<double*>(buf);  // until the first samples are stored
+  auto wt_base = [&](int m) { return (start[m] + start[m + 1] + 6 * m) / 4 * 4; };
 
   const float* x = a.audio + (int64_t)b * a.audio_stride;
-  // Padded sample j of this tile is original sample 160*f0 + j - 200, reflected at both ends.
-  for (int j = tid; j < kSeg; j += 256) {
-    int o = kHop * f0 + j - kNfft / 2;
-    if (o < 0) o = -o;
-    if (o >= N) o = 2 * (N - 1) - o;
-    o = o < 0 ? 0 : (o >= N ? N - 1 : o);  // frames past the end only
-    seg_p[seg_pos(j)] = x[o];
-  }
-  for (int j = tid; j < kNfft; j += 256) {
-    ctab[j] = a.tables[j];
-    win[j] = a.tables[kNfft + j];
-  }
-  __syncthreads();
-
-  // ---- windowed DFT: wave w computes bin tiles w and w + 4 for the 32 frames (tile 7 is past
-  // the 201 bins; computing it keeps every wavefront on the same straight-line code) ----
-  const int fr = lane & 31;  // frame of this lane's A element / bin of its B element
-  const int kk = lane >> 5;  // which of the 2 samples of a step
-  f32x16v re[2], im[2];
-#pragma unroll
-  for (int u = 0; u < 2; ++u) re[u] = im[u] = f32x16v{};
-  int idx[2], step[2];
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int n = 32 * (wave + 4 * u) + fr;  // bin
-    idx[u] = (kk * n) % kNfft;               // (i * n) mod 400 for i = kk
-    step[u] = (2 * n) % kNfft;
-  }
-#pragma unroll 8
-  for (int s = 0; s < kNfft / 2; ++s) {
-    const int i = 2 * s + kk;
-    const float av = seg_p[seg_pos(kHop * fr + i)] * win[i];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const float c = ctab[idx[u]];
-      int is = idx[u] + 300;  // sin(t) = cos(t - pi/2): index - 100 mod 400
-      is = is >= kNfft ? is - kNfft : is;
-      const float sn = ctab[is];
-      re[u] = mfma32x2(av, c, re[u]);
-      im[u] = mfma32x2(av, sn, im[u]);
-      idx[u] += step[u];
-      idx[u] = idx[u] >= kNfft ? idx[u] - kNfft : idx[u];
-    }
-  }
-  __syncthreads();  // every wavefront is done with the samples: the buffer becomes the power tile
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int n = 32 * (wave + 4 * u) + fr;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int row = 8 * (e / 4) + 4 * kk + (e % 4);  // frame within the tile
-      const float p = re[u][e] * re[u][e] + im[u][e] * im[u][e];
-      if (n < kKMel) seg_p[row * kPPitch + n] = n < kBins ? p : 0.f;
-    }
-  }
-  __syncthreads();
-
-  // ---- filterbank: wave w computes mel tile w, [32 frames] x [32 mels] over 202 bins ----
-  const int n_tiles = (a.n_mels + 31) / 32;
+  const int n_tiles = (a.n_frames + kFrames - 1) / kFrames;
   float vmax = -INFINITY;
-  if (wave < n_tiles) {
-    const int mel = 32 * wave + fr;
-    const int melc = mel < a.n_mels ? mel : a.n_mels - 1;
-    f32x16v acc = f32x16v{};
-#pragma unroll 8
-    for (int s = 0; s < kKMel / 2; ++s) {
-      const int k = 2 * s + kk;
-      const float av = seg_p[fr * kPPitch + k];
-      const float bv = a.fb[k * a.n_mels + melc];
-      acc = mfma32x2(av, bv, acc);
-    }
-    float* out = a.out + (int64_t)b * a.os[0] + (int64_t)mel * a.os[1];
+  for (int tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
+    const int f0 = tile * kFrames;
+    // tables and addresses are formed again for each tile: kept across tiles they would spill
+    const MelTables* tab = &kTables;
+    int tid = threadIdx.x;
+    asm volatile("" : "+s"(tab), "+v"(tid));
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // Padded sample j of this tile is original sample 160 f0 + j - 200, reflected at both ends.
+    float smp[kSegLoads];
+    const int o0 = kHop * f0 - kNfft / 2;
+    const bool inside = o0 >= 0 && o0 + kSeg <= N;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int f = f0 + 8 * (e / 4) + 4 * kk + (e % 4);
-      const float lv = log10f(fmaxf(acc[e], 1e-10f));
-      if (mel < a.n_mels && f < a.n_frames) {
-        vmax = fmaxf(vmax, lv);
-        if (f < a.out_frames) out[f] = lv;
+    for (int i = 0; i < kSegLoads; ++i) {
+      const int j = tid + kThreads * i;
+      int o = o0 + j;
+      if (!inside) {
+        o = o < 0 ? -o : o;
+        o = o >= N ? 2 * (N - 1) - o : o;
+        o = o < 0 ? 0 : o;  // frames past the end only
+      }
+      smp[i] = j < kSeg ? x[o] : 0.f;
+    }
+    if (tile == (int)blockIdx.x) {
+      // the filterbank, while the samples are on their way: bin k lies between edges j and j + 1,
+      // so it is on the rising side of filter j and on the falling side of filter j - 1
+      for (int j = tid; j < a.n_mels + 2; j += kThreads) {
+        const double f = mel_edge(j, a.n_mels);
+        edges[j] = f;
+        start[j] = j == a.n_mels + 1 ? kBins : (int)ceil(f / 40.0);  // bins are 40 Hz apart
+      }
+      for (int i = tid; i < kWeights; i += kThreads) wts[i] = 0.f;
+      __syncthreads();
+      for (int k = tid; k < kBins; k += kThreads) {
+        int lo = 0, hi = a.n_mels + 1;  // the last edge interval whose first bin is <= k
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) >> 1;
+          if (start[mid] <= k) lo = mid;
+          else hi = mid;
+        }
+        const double f = 40.0 * k, e0 = edges[lo], e1 = edges[lo + 1];
+        const double down = (f - e0) / (e1 - e0), up = (e1 - f) / (e1 - e0);
+        if (lo < a.n_mels)
+          wts[wt_base(lo) + k - (start[lo] & ~3)] = (float)((down > 0.0 ? down : 0.0) * 2.0 / (edges[lo + 2] - e0));
+        if (lo > 0)
+          wts[wt_base(lo - 1) + k - (start[lo - 1] & ~3)] = (float)((up > 0.0 ? up : 0.0) * 2.0 / (e1 - edges[lo - 1]));
+      }
+      __syncthreads();  // the samples take the edges' place
+    }
+#pragma unroll
+    for (int i = 0; i < kSegLoads; ++i) {
+      const int j = tid + kThreads * i;
+      if (j < kSeg) buf[seg_pos(j)] = smp[i];
+    }
+    __syncthreads();
+
+    // ---- stage 1: lane (frame, n1) transforms z[n1 + 10 n2] over n2, z[n] = x[2n] + i x[2n + 1] ----
+    const int l = lane < 60 ? lane : 59;  // the last four lanes repeat lane 59
+    Cplx v[20];
+    {
+      const int fr = l / 10, n1 = l % 10;
+      const float* s = buf + (kHop + kHopPad) * (kWaveFrames * wave + fr) + 2 * n1;
+#pragma unroll
+      for (int n2 = 0; n2 < 20; ++n2) {
+        const float2 z = *reinterpret_cast<const float2*>(s + 20 * n2 + kHopPad * (n2 / 8));
+        const float2 w = *reinterpret_cast<const float2*>(&tab->window[2 * n1 + 20 * n2]);
+        v[n2] = {z.x * w.x, z.y * w.y};
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      dft20(v);
+      __builtin_amdgcn_sched_barrier(0);  // the twiddles' loads above would take 40 registers more
+      __syncthreads();  // every wavefront has read its samples: the buffer becomes the transforms'
+      float2* A = reinterpret_cast<float2*>(buf + wave * kWaveFloats) + fr * kFramePitch + n1;
+#pragma unroll
+      for (int k1 = 0; k1 < 20; ++k1) {
+        const float2 t = tab->tw[k1 * 10 + n1];
+        A[10 * k1] = make_float2(v[k1].r * t.x - v[k1].i * t.y, v[k1].r * t.y + v[k1].i * t.x);
       }
     }
+    wave_fence();
+    // ---- stage 2: lane (frame pair, k1) transforms over n1, for both frames: Z[k1 + 20 k2] ----
+    {
+      const int k1 = l % 20;
+      float2* A = reinterpret_cast<float2*>(buf + wave * kWaveFloats) + 2 * (l / 20) * kFramePitch;
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int n = 0; n < 10; n += 2) {
+          const float4 z = *reinterpret_cast<const float4*>(A + u * kFramePitch + 10 * k1 + n);
+          v[10 * u + n] = {z.x, z.y};
+          v[10 * u + n + 1] = {z.z, z.w};
+        }
+      wave_fence();
+      dft10(v);
+      dft10(v + 10);
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int k2 = 0; k2 < 10; ++k2)
+          A[u * kFramePitch + k1 + 20 * k2] = make_float2(v[10 * u + k2].r, v[10 * u + k2].i);
+    }
+    wave_fence();
+    // ---- powers of bins k and 200 - k from Z[k] and Z[200 - k] (even +- e^(-2 pi i k / 400) odd) ----
+    {
+      constexpr int kPairs = kHalf / 2 + 1, kAll = kWaveFrames * kPairs, kRounds = (kAll + 63) / 64;
+      const float2* Z = reinterpret_cast<const float2*>(buf + wave * kWaveFloats);
+      float lo[kRounds], hi[kRounds];
+#pragma unroll
+      for (int i = 0; i < kRounds; ++i) {
+        const int q = min(lane + 64 * i, kAll - 1);
+        const int fr = q / kPairs, k = q % kPairs;
+        const float2 z = Z[fr * kFramePitch + k];
+        const float2 y = Z[fr * kFramePitch + (k ? kHalf - k : 0)];
+        const float2 w = tab->split[k];
+        const float er = z.x + y.x, ei = z.y - y.y;     // even part (of the halved samples)
+        const float od = z.y + y.y, oi = y.x - z.x;     // odd part
+        const float tr = w.x * od - w.y * oi, ti = w.x * oi + w.y * od;
+        lo[i] = (er + tr) * (er + tr) + (ei + ti) * (ei + ti);
+        hi[i] = (er - tr) * (er - tr) + (ei - ti) * (ei - ti);
+      }
+      wave_fence();
+#pragma unroll
+      for (int i = 0; i < kRounds; ++i) {
+        const int q = min(lane + 64 * i, kAll - 1);
+        const int fr = q / kPairs, k = q % kPairs;
+        buf[power_pos(wave, fr, k)] = lo[i];
+        buf[power_pos(wave, fr, kHalf - k)] = hi[i];
+      }
+      if (lane < 3 * kWaveFrames) buf[power_pos(wave, lane / 3, kBins + lane % 3)] = 0.f;
+    }
+    __syncthreads();
+
+    // ---- filterbank and log10: half-wavefront = one mel, lane = frame; mels 2p and 2p + 1 are
+    // about equally wide, so the halves' loops end together ----
+    {
+      const int fr = min(lane & 31, kFrames - 1), f = f0 + fr;
+      const float* P = buf + power_pos(fr / kWaveFrames, fr % kWaveFrames, 0);
+      for (int p = wave; 2 * p < a.n_mels; p += kWaves) {
+        const int mel = 2 * p + (lane >> 5), melc = min(mel, a.n_mels - 1);
+        const int g0 = start[melc] >> 2, g1 = (start[melc + 2] + 3) >> 2;
+        const float* w = wts + wt_base(melc);
+        float acc = 0.f;
+        for (int g = g0; g < g1; ++g) {  // weights of the bins outside the filter are zero
+          const f32x4 pv = *reinterpret_cast<const f32x4*>(P + 4 * kWaveFrames * g);
+          const f32x4 wv = *reinterpret_cast<const f32x4*>(w + 4 * (g - g0));
+          acc += (pv[0] * wv[0] + pv[1] * wv[1]) + (pv[2] * wv[2] + pv[3] * wv[3]);
+        }
+        const float lv = log10f(fmaxf(acc, 1e-10f));
+        if (mel < a.n_mels && f < a.n_frames && (lane & 31) < kFrames) {
+          vmax = fmaxf(vmax, lv);
+          if (f < a.out_frames) a.out[(int64_t)b * a.os[0] + (int64_t)mel * a.os[1] + f] = lv;
+        }
+      }
+    }
+    __syncthreads();  // the next tile's samples overwrite the powers
   }
-  // window maximum: wave, then workgroup, then one atomic (vector) per workgroup
+  // this workgroup's maximum of the window
+  const int tid = threadIdx.x;
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, o));
-  if (lane == 0) wmax[wave] = order_key(vmax);
+  if ((tid & 63) == 0) wmax[tid >> 6] = vmax;
   __syncthreads();
   if (tid == 0) {
-    uint32_t k = wmax[0];
 #pragma unroll
-    for (int w = 1; w < 4; ++w) k = k > wmax[w] ? k : wmax[w];
-    atomicMax(a.gmax + b, k);
+    for (int w = 1; w < kWaves; ++w) vmax = fmaxf(vmax, wmax[w]);
+    a.part_max[(int64_t)b * kMaxParts + blockIdx.x] = vmax;
   }
 }
 
+// One row (window, mel) piece of 256 VEC frames per workgroup. VEC 4: 16-byte accesses, for rows
+// that start 16-byte aligned and hold whole groups of four.
+template <int VEC>
 __global__ __launch_bounds__(256) void logmel_finish_kernel(LogMelArgs a) {
   const int b = blockIdx.z, m = blockIdx.y;
-  const int f = blockIdx.x * 256 + threadIdx.x;
-  if (f >= a.out_frames) return;
+  const int f = (blockIdx.x * 256 + threadIdx.x) * VEC;
   float* p = a.out + (int64_t)b * a.os[0] + (int64_t)m * a.os[1] + f;
-  if (f >= a.n_frames) {
-    *p = -1.5f;  // audio.py:133-137
-    return;
-  }
-  const float floor_v = order_val(a.gmax[b]) - 8.0f;
-  *p = (fmaxf(*p, floor_v) + 4.0f) / 4.0f;
+  float v[VEC];
+  const bool any = f < a.n_frames && f < a.out_frames;
+  if (any) __builtin_memcpy(v, p, sizeof(v));
+  // the window's maximum: every wavefront reduces the workgroups' maxima
+  float vmax = -INFINITY;
+  for (int i = threadIdx.x & 63; i < a.parts; i += 64) vmax = fmaxf(vmax, a.part_max[(int64_t)b * kMaxParts + i]);
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, o));
+  if (f >= a.out_frames) return;
+  const float floor_v = vmax - 8.0f;
+#pragma unroll
+  for (int i = 0; i < VEC; ++i)
+    v[i] = f + i < a.n_frames ? (fmaxf(v[i], floor_v) + 4.0f) / 4.0f : -1.5f;  // audio.py:133-137
+  __builtin_memcpy(p, v, sizeof(v));
 }
 
 }  // namespace
 
-// Workspace: filterbank [202, n_mels], cosine + Hann tables [2, 400], window maxima [B].
-namespace {
-size_t fb_bytes(int64_t n_mels) { return ((size_t)(kKMel * n_mels) * sizeof(float) + 255) / 256 * 256; }
-constexpr size_t kTableBytes = 2 * kNfft * sizeof(float);
-}  // namespace
-
+// Workspace: kMaxParts maxima per window.
 size_t logmel_workspace_bytes(int64_t B, int64_t n_mels) {
-  return fb_bytes(n_mels) + kTableBytes + (size_t)B * sizeof(uint32_t);
+  (void)n_mels;
+  return (size_t)B * kMaxParts * sizeof(float);
 }
 
 hipError_t launch_logmel(LogMelArgs a, void* ws, hipStream_t stream) {
-  char* p = static_cast<char*>(ws);
-  a.fb = reinterpret_cast<float*>(p);
-  a.tables = reinterpret_cast<float*>(p + fb_bytes(a.n_mels));
-  a.gmax = reinterpret_cast<uint32_t*>(p + fb_bytes(a.n_mels) + kTableBytes);
-  int init_n = kKMel * a.n_mels > a.B ? kKMel * a.n_mels : a.B;
-  init_n = init_n > kNfft ? init_n : kNfft;
-  hipLaunchKernelGGL(logmel_init_kernel, dim3((init_n + 255) / 256), dim3(256), 0, stream, a);
-  hipLaunchKernelGGL(logmel_spec_kernel, dim3((a.n_frames + kFrames - 1) / kFrames, a.B), dim3(256), 0, stream, a);
-  hipLaunchKernelGGL(logmel_finish_kernel, dim3((a.out_frames + 255) / 256, a.n_mels, a.B), dim3(256), 0, stream, a);
+  a.part_max = static_cast<float*>(ws);
+  const int tiles = (a.n_frames + kFrames - 1) / kFrames;
+  a.parts = tiles < kMaxParts ? tiles : kMaxParts;
+  hipLaunchKernelGGL(logmel_spec_kernel, dim3(a.parts, a.B), dim3(kThreads), 0, stream, a);
+  const bool vec = (reinterpret_cast<uintptr_t>(a.out) & 15u) == 0 && a.out_frames % 4 == 0 && a.os[0] % 4 == 0 &&
+                   a.os[1] % 4 == 0;
+  if (vec)
+    hipLaunchKernelGGL(logmel_finish_kernel<4>, dim3((a.out_frames + 1023) / 1024, a.n_mels, a.B), dim3(256), 0, stream, a);
+  else
+    hipLaunchKernelGGL(logmel_finish_kernel<1>, dim3((a.out_frames + 255) / 256, a.n_mels, a.B), dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 

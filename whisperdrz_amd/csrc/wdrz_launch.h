@@ -176,10 +176,9 @@ struct LogMelArgs {
   int64_t audio_stride;
   float* out;         // [B, n_mels, out_frames], frames contiguous
   int64_t os[2];      // b, mel strides of out
-  float* fb;          // workspace: [202, n_mels] filterbank
-  float* tables;      // workspace: cos(2 pi j / 400), then the periodic Hann window
-  uint32_t* gmax;     // workspace: [B] ordered-encoded window maxima
+  float* part_max;    // workspace: [B, 128], each workgroup's maximum of its window
   int B, n_samples, n_mels, n_frames, out_frames;
+  int parts;          // workgroups (maxima) per window (set by the launcher)
 };
 size_t logmel_workspace_bytes(int64_t B, int64_t n_mels);
 hipError_t launch_logmel(LogMelArgs a, void* ws, hipStream_t stream);
