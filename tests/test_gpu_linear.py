@@ -58,6 +58,24 @@ def test_linear_gelu(cuda, dtype, M, N, K, gelu):
     _check(y, mod, "vs torch modules")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [1, 2, 15, 16, 17])
+@pytest.mark.parametrize("N,K", [(8, 128), (24, 1280), (1280, 1408), (40, 5120)])
+def test_linear_few_rows(cuda, dtype, M, N, K):
+    """Both sides of the 16-row rule; half a feature tile, one K step per wavefront, K past one
+    batch of loads (1280) and a part of one; rows and weights taken from wider buffers. The bound is
+    the file's: two 16-bit ulps of the fp32 restatement."""
+    from whisperdrz_amd import linear
+
+    g = torch.Generator(device=cuda).manual_seed(M + N + K)
+    x = torch.randn(M, K + 64, generator=g, device=cuda).to(dtype)[:, 8 : K + 8]
+    w = (torch.randn(N, K + 16, generator=g, device=cuda) / K ** 0.5).to(dtype)[:, :K]
+    b = torch.randn(N, generator=g, device=cuda).to(dtype)
+    for gelu in (False, True):
+        pre = (x.float() @ w.float().T + b.float()).to(dtype)
+        _check(linear(x, w, b, gelu), F.gelu(pre.float()).to(dtype) if gelu else pre, f"gelu={gelu}")
+
+
 def test_linear_strided_rows_and_no_bias(cuda):
     """x rows taken from a wider buffer (a view, row stride > K) and a Linear without bias."""
     from whisperdrz_amd import linear_gelu
@@ -96,7 +114,8 @@ def test_linear_zero_rows_and_errors(cuda):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,N,K,n_split", [(64, 1280, 5120, 4), (1, 1280, 5120, 4), (5, 1280, 5120, 2),
-                                           (65, 1024, 4096, 4), (130, 40, 1024, 2), (3, 8, 512, 4)])
+                                           (65, 1024, 4096, 4), (130, 40, 1024, 2), (3, 8, 512, 4),
+                                           (16, 1280, 1280, 2), (17, 24, 6144, 4), (9, 24, 6144, 4)])
 def test_linear_partials(cuda, dtype, M, N, K, n_split):
     from whisperdrz_amd import linear_partials
 

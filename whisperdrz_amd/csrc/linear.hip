@@ -47,6 +47,25 @@ template <> struct LinMfma<F16> {
 
 __device__ __forceinline__ float gelu_erf(float v) { return 0.5f * v * (1.f + erff(v * 0.70710678118654752f)); }
 
+// Four features nb .. nb + 3 of row m: bias, rounding to the storage type as the Linear's output,
+// then the activation.
+template <typename T, int ACT>
+__device__ __forceinline__ void linear_store(const LinearArgs& a, int m, int nb, f32x4 acc) {
+  const uint16_t* B = static_cast<const uint16_t*>(a.bias);
+  float v[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    float s = acc[r];
+    if (B) s += __is_same(T, Bf16) ? bf16_lo(B[nb + r]) : f16_lo(B[nb + r]);
+    s = LinMfma<T>::round(s);
+    v[r] = ACT ? gelu_erf(s) : s;
+  }
+  uint2 out;
+  out.x = LinMfma<T>::pack(v[0], v[1]);
+  out.y = LinMfma<T>::pack(v[2], v[3]);
+  *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.y) + (int64_t)m * a.y_stride + nb) = out;
+}
+
 constexpr int kLinRows = 64;    // rows (M) per workgroup
 constexpr int kLinChunk = 128;  // K per LDS stage
 constexpr int kLinPad = 8;      // 16-bit elements of row padding in LDS (16 bytes)
@@ -154,27 +173,83 @@ __global__ __launch_bounds__(256) void linear_act_kernel(LinearArgs a) {
     }
     return;
   }
-  const uint16_t* B = static_cast<const uint16_t*>(a.bias);
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     const int nb = n0 + 16 * j + (lane >> 4) * 4;
-    if (nb >= a.N) continue;
-    float v[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float s = acc[j][r];
-      if (B) s += __is_same(T, Bf16) ? bf16_lo(B[nb + r]) : f16_lo(B[nb + r]);
-      s = LinMfma<T>::round(s);  // the Linear's output in the storage type, as the reference has it
-      v[r] = ACT ? gelu_erf(s) : s;
-    }
-    uint2 out;
-    out.x = LinMfma<T>::pack(v[0], v[1]);
-    out.y = LinMfma<T>::pack(v[2], v[3]);
-    *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.y) + (int64_t)m * a.y_stride + nb) = out;
+    if (nb < a.N) linear_store<T, ACT>(a, m, nb, acc[j]);
   }
 }
 
+// Few rows (M <= 16, one MFMA tile of activations): a workgroup of kRowWaves wavefronts takes 16
+// features, the wavefronts split K, and each reads its part of the 16 weight rows and of the
+// activations straight into MFMA operands. Every load of the workgroup is requested at kernel
+// start, nothing is staged, and one barrier (the sum over the wavefronts) remains; the 64-row form
+// above walks ten LDS stages with a barrier each for the same weights. Bound: launch, one trip to
+// memory and the weight stream (1280 x 1280: 4.1 us, of which an empty launch is 1.8). The weight
+// loads take 64 bytes of a row each, so they are cached loads: as streaming loads the other half of
+// the line is fetched twice. Cold weights in a graph, us at 1 / 16 rows (64-row form -> this):
+// 3840 x 1280 6.1 -> 4.6 / 6.3 -> 5.5, 1280 x 1280 5.6 -> 4.1 / 5.7 -> 4.9, fc1 with GELU 8.9 ->
+// 6.8 / 9.1 -> 8.4, output halves 4.0 -> 3.2 / 4.0 -> 3.6, fc2 quarters 7.9 -> 6.1 / 7.7 -> 7.8.
+// From 17 rows on the activations' own operand reads (64 bytes a row too, from every workgroup)
+// cost more than the stages: 24 rows fc1 9.4 -> 10.3, fc2 8.0 -> 9.5.
+constexpr int kRowMax = 16;
+constexpr int kRowWaves = 4;
+constexpr int kRowBatch = 10;  // 32-value K steps requested together (K = 1280 over 4 wavefronts)
+
+template <typename T, int ACT, bool PART>
+__global__ __launch_bounds__(64 * kRowWaves) void linear_rows_kernel(LinearArgs a) {
+  typedef typename LinMfma<T>::op_t op_t;
+  __shared__ __align__(16) f32x4 red[kRowWaves][64];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n0 = blockIdx.x * 16;
+  const int k_len = PART ? a.K / a.n_split : a.K;  // a multiple of 128
+  const int steps = k_len / (32 * kRowWaves);
+  const int k0 = (PART ? (int)blockIdx.z * k_len : 0) + wave * steps * 32;
+  // MFMA operands: lane holds 8 K values of row lane % 16 at K offset 8 (lane / 16)
+  const int li = lane & 15, lq = (lane >> 4) * 8;
+  const uint16_t* w = static_cast<const uint16_t*>(a.w) + (int64_t)min(n0 + li, a.N - 1) * a.w_stride + k0 + lq;
+  const uint16_t* x = static_cast<const uint16_t*>(a.x) + (int64_t)li * a.x_stride + k0 + lq;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < steps; s0 += kRowBatch) {
+    u32x4 rw[kRowBatch], rx[kRowBatch];
+#pragma unroll
+    for (int i = 0; i < kRowBatch; ++i) {
+      rx[i] = u32x4{0, 0, 0, 0};
+      if (s0 + i < steps) rw[i] = load16(w + 32 * (s0 + i));
+    }
+    if (li < a.M) {  // rows past M: zero operands, no loads
+#pragma unroll
+      for (int i = 0; i < kRowBatch; ++i)
+        if (s0 + i < steps) rx[i] = load16(x + 32 * (s0 + i));
+    }
+#pragma unroll
+    for (int i = 0; i < kRowBatch; ++i)
+      if (s0 + i < steps)
+        acc = LinMfma<T>::run(__builtin_bit_cast(op_t, rw[i]), __builtin_bit_cast(op_t, rx[i]), acc);
+  }
+  red[wave][lane] = acc;
+  __syncthreads();
+  // red[w][lane][r] = C[n = 4 (lane / 16) + r][m = lane % 16] over wavefront w's K range
+  if (wave != 0) return;
+  f32x4 c = red[0][lane];
+#pragma unroll
+  for (int v = 1; v < kRowWaves; ++v) c += red[v][lane];
+  const int m = li, nb = n0 + (lane >> 4) * 4;
+  if (m >= a.M || nb >= a.N) return;
+  if constexpr (PART) *reinterpret_cast<f32x4*>(a.part + ((int64_t)blockIdx.z * a.M + m) * a.N + nb) = c;
+  else linear_store<T, ACT>(a, m, nb, c);
+}
+
 }  // namespace
+
+template <typename T>
+void launch_rows(const LinearArgs& a, hipStream_t stream) {
+  const dim3 grid((unsigned)((a.N + 15) / 16), 1, (unsigned)(a.part ? a.n_split : 1)), block(64 * kRowWaves);
+  if (a.part) hipLaunchKernelGGL((linear_rows_kernel<T, 0, true>), grid, block, 0, stream, a);
+  else if (a.act) hipLaunchKernelGGL((linear_rows_kernel<T, 1, false>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((linear_rows_kernel<T, 0, false>), grid, block, 0, stream, a);
+}
 
 template <typename T, int NJ, int PF>
 void launch_t(const LinearArgs& a, hipStream_t stream) {
@@ -187,6 +262,11 @@ void launch_t(const LinearArgs& a, hipStream_t stream) {
 
 hipError_t launch_linear(int dtype, const LinearArgs& a, hipStream_t stream) {
   if (a.M == 0 || a.N == 0) return hipSuccess;
+  if (a.M <= kRowMax) {
+    if (dtype == 2) launch_rows<Bf16>(a, stream);
+    else launch_rows<F16>(a, stream);
+    return hipGetLastError();
+  }
   // 16 features per workgroup, X two chunks ahead; 32 features once 16 would give 320 or more
   // workgroups (more than one per CU). Measured at 64 rows, 32 cold weights in a graph: fc1
   // (5120 x 1280) 10.8 -> 10.1 us and fc2's split-K quarters (1280 x 5120) 10.3 -> 9.5 us with 32;
