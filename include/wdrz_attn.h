@@ -227,6 +227,27 @@ int wdrz_add_layernorm_partials(int dtype, void* x, int64_t x_stride, const floa
                                 int64_t n, float eps, void* stream);
 
 /*
+ * Residual add + LayerNorm + the Linear that follows, for the few rows of a decode step with one to
+ * four streams.
+ *
+ * Replaces: the residual add closing a sub-layer, the LayerNorm opening the next and that
+ *           sub-layer's first projection (src/whisperdrz/model.py:420-434: attn_ln + query / key /
+ *           value, cross_attn_ln + query, mlp_ln + the MLP's first Linear and GELU).
+ * With partials (fp32 [n_split][M][K], wdrz_linear_partials' output) and delta_bias:
+ *   r = round(x + round(sum of the partials + delta_bias)), stored to x_out [M, K] (a buffer other
+ *   than x); without (partials NULL): r = x and x_out is not used.
+ * y = act(LayerNorm(r) w^T + bias) [M, N], rounded as wdrz_add_layernorm_partials and wdrz_linear
+ *   round. w: [N, K] rows; bias may be NULL; activation as in wdrz_linear.
+ * M <= 4, K <= 1536, K % 128 == 0, N % 8 == 0, n_split 2 or 4; 16-byte aligned pointers (bias and
+ * y's features excepted as in wdrz_linear) and row strides.
+ */
+int wdrz_ln_linear(int dtype, const void* x, int64_t x_stride, const float* partials, int n_split,
+                   const void* delta_bias, void* x_out, int64_t x_out_stride, const void* ln_weight,
+                   const void* ln_bias, float eps, const void* w, int64_t w_stride,
+                   const void* bias, void* y, int64_t y_stride, int64_t M, int64_t N, int64_t K,
+                   int activation, void* stream);
+
+/*
  * Greedy sampling with the decode step's token constraints.
  *
  * Replaces: decode_batch's sampling tail (src/whisperdrz/decoding.py:1729-1761):

@@ -15,7 +15,7 @@ from .attention import (
 )
 from .audio import LogMelSpectrogram, log_mel_spectrogram
 from .decode_ops import (add_layernorm_, add_layernorm_partials_, layer_norm, linear, linear_gelu, linear_partials,
-                         masked_argmax)
+                         ln_linear, masked_argmax)
 from .dtw import (compute_attention, dtw_attention_prep, dtw_prep, dtw_prep_batch, dtw_prep_workspace_size,
                   median_filter)
 
@@ -37,6 +37,7 @@ __all__ = [
     "linear",
     "linear_gelu",
     "linear_partials",
+    "ln_linear",
     "masked_argmax",
     "log_mel_spectrogram",
     "compute_attention",

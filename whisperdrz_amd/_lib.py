@@ -39,6 +39,7 @@ EXPORTED_SYMBOLS = (
     "wdrz_linear",
     "wdrz_linear_partials",
     "wdrz_add_layernorm_partials",
+    "wdrz_ln_linear",
     "wdrz_log_mel_workspace_size",
     "wdrz_log_mel",
     "wdrz_dtw_qk",
@@ -106,6 +107,12 @@ def _declare(lib: ctypes.CDLL) -> None:
         ctypes.c_int, _p, _i64, _p, ctypes.c_int, _p,  # dtype, x, x stride, partials, n_split, delta bias
         _p, _p, _p, _i64, _i64, _i64,  # weight, bias, y, y stride, rows, n
         ctypes.c_float, _p,  # eps, stream
+    ]
+    lib.wdrz_ln_linear.restype = ctypes.c_int
+    lib.wdrz_ln_linear.argtypes = [
+        ctypes.c_int, _p, _i64, _p, ctypes.c_int, _p, _p, _i64,  # dtype, x, stride, partials, n_split, delta bias, x_out, stride
+        _p, _p, ctypes.c_float, _p, _i64, _p,  # LayerNorm weight, bias, eps; w, stride, bias
+        _p, _i64, _i64, _i64, _i64, ctypes.c_int, _p,  # y, stride, M, N, K, activation, stream
     ]
     lib.wdrz_masked_argmax.restype = ctypes.c_int
     lib.wdrz_masked_argmax.argtypes = [

@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "layernorm.h"
 #include "wdrz_common.h"
 #include "wdrz_launch.h"
 
@@ -241,6 +242,65 @@ __global__ __launch_bounds__(64 * kRowWaves) void linear_rows_kernel(LinearArgs 
   else linear_store<T, ACT>(a, m, nb, c);
 }
 
+// The same with the activations computed on the way: rows = LayerNorm(x + delta), as
+// wdrz_add_layernorm_partials gives them, for up to kLnRowMax rows of n = K <= 1536. Wavefront r of
+// every workgroup adds and normalises row r into LDS while the workgroup's weights are in flight
+// (the row's loads are issued first: loads return in order); workgroup 0 stores the new residual to
+// a buffer of its own, since the other workgroups still read the old one. Bound: the launch and two
+// trips to memory side by side. Cold weights in a graph, 1 / 4 rows, separate launches -> this (the
+// Linear alone): q/k/v behind 4 partials 8.1 -> 6.0 (4.6) / 9.4 -> 6.9 us, 1280 x 1280 behind 2
+// 7.3 -> 5.3 (4.1) / 8.0 -> 5.9, fc1 with GELU 10.3 -> 8.1 (7.1) / 11.3 -> 9.1. A wavefront takes
+// one row, hence the limit of 4: every workgroup repeats the rows' work and their NP + 1 reads.
+constexpr int kLnRowMax = kRowWaves;
+constexpr int kLnMaxK = 1536;
+
+template <typename T, int ACT, int NP>
+__global__ __launch_bounds__(64 * kRowWaves) void ln_linear_kernel(LinearArgs a, AddLnArgs ln, void* x_out,
+                                                                   int64_t xo_stride) {
+  typedef typename LinMfma<T>::op_t op_t;
+  constexpr int kSteps = kLnMaxK / (32 * kRowWaves);
+  __shared__ __align__(16) uint16_t sx[kLnRowMax][kLnMaxK + 8];
+  __shared__ __align__(16) f32x4 red[kRowWaves][64];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n0 = blockIdx.x * 16;
+  const int steps = a.K / (32 * kRowWaves);
+  const int k0 = wave * steps * 32;
+  const int li = lane & 15, lq = (lane >> 4) * 8;
+  const uint16_t* w = static_cast<const uint16_t*>(a.w) + (int64_t)min(n0 + li, a.N - 1) * a.w_stride + k0 + lq;
+  LnRow<T, kLnMaxK / 512, NP> row;
+  if (wave < a.M) row.load(ln, wave, lane);
+  u32x4 rw[kSteps];
+#pragma unroll
+  for (int i = 0; i < kSteps; ++i)
+    if (i < steps) rw[i] = load16(w + 32 * i);
+  if (wave < a.M) {
+    char* xo = static_cast<char*>(x_out) + wave * xo_stride * 2;
+    row.finish(ln, lane,
+               [&](int c, u32x4 v) {
+                 if (blockIdx.x == 0) *reinterpret_cast<u32x4*>(xo + c * 16) = v;
+               },
+               [&](int c, u32x4 v) { *reinterpret_cast<u32x4*>(&sx[wave][c * 8]) = v; });
+  }
+  __syncthreads();
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < kSteps; ++i)
+    if (i < steps) {
+      u32x4 rx = {0, 0, 0, 0};  // rows past M
+      if (li < a.M) rx = *reinterpret_cast<const u32x4*>(&sx[li][k0 + lq + 32 * i]);
+      acc = LinMfma<T>::run(__builtin_bit_cast(op_t, rw[i]), __builtin_bit_cast(op_t, rx), acc);
+    }
+  red[wave][lane] = acc;
+  __syncthreads();
+  if (wave != 0) return;
+  f32x4 c = red[0][lane];
+#pragma unroll
+  for (int v = 1; v < kRowWaves; ++v) c += red[v][lane];
+  const int nb = n0 + (lane >> 4) * 4;
+  if (li < a.M && nb < a.N) linear_store<T, ACT>(a, li, nb, c);
+}
+
 }  // namespace
 
 template <typename T>
@@ -249,6 +309,27 @@ void launch_rows(const LinearArgs& a, hipStream_t stream) {
   if (a.part) hipLaunchKernelGGL((linear_rows_kernel<T, 0, true>), grid, block, 0, stream, a);
   else if (a.act) hipLaunchKernelGGL((linear_rows_kernel<T, 1, false>), grid, block, 0, stream, a);
   else hipLaunchKernelGGL((linear_rows_kernel<T, 0, false>), grid, block, 0, stream, a);
+}
+
+template <typename T, int ACT>
+void launch_ln_rows(const LinearArgs& a, const AddLnArgs& ln, void* x_out, int64_t xo_stride, hipStream_t stream) {
+  const dim3 grid((unsigned)((a.N + 15) / 16)), block(64 * kRowWaves);
+  if (!ln.dpart) hipLaunchKernelGGL((ln_linear_kernel<T, ACT, 0>), grid, block, 0, stream, a, ln, x_out, xo_stride);
+  else if (ln.n_part == 2) hipLaunchKernelGGL((ln_linear_kernel<T, ACT, 2>), grid, block, 0, stream, a, ln, x_out, xo_stride);
+  else hipLaunchKernelGGL((ln_linear_kernel<T, ACT, 4>), grid, block, 0, stream, a, ln, x_out, xo_stride);
+}
+
+hipError_t launch_ln_linear(int dtype, const LinearArgs& a, const AddLnArgs& ln, void* x_out, int64_t xo_stride,
+                            hipStream_t stream) {
+  if (a.M < 1 || a.M > kLnRowMax || a.K > kLnMaxK || a.K != ln.n) return hipErrorInvalidValue;
+  if (dtype == 2) {
+    if (a.act) launch_ln_rows<Bf16, 1>(a, ln, x_out, xo_stride, stream);
+    else launch_ln_rows<Bf16, 0>(a, ln, x_out, xo_stride, stream);
+  } else {
+    if (a.act) launch_ln_rows<F16, 1>(a, ln, x_out, xo_stride, stream);
+    else launch_ln_rows<F16, 0>(a, ln, x_out, xo_stride, stream);
+  }
+  return hipGetLastError();
 }
 
 template <typename T, int NJ, int PF>

@@ -487,6 +487,61 @@ int wdrz_linear_partials(int dtype, const void* x, int64_t x_stride, const void*
   return WDRZ_OK;
 }
 
+int wdrz_ln_linear(int dtype, const void* x, int64_t x_stride, const float* partials, int n_split,
+                   const void* delta_bias, void* x_out, int64_t x_out_stride, const void* ln_weight,
+                   const void* ln_bias, float eps, const void* w, int64_t w_stride, const void* bias, void* y,
+                   int64_t y_stride, int64_t M, int64_t N, int64_t K, int activation, void* stream) {
+  g_last_error.clear();
+  if (dtype != WDRZ_BF16 && dtype != WDRZ_F16)
+    return fail(dtype == WDRZ_F32 ? WDRZ_EUNSUPPORTED : WDRZ_EINVAL, "dtype %d: only WDRZ_BF16 / WDRZ_F16", dtype);
+  if (activation != 0 && activation != 1) return fail(WDRZ_EINVAL, "activation %d is not 0 (none) or 1 (GELU)", activation);
+  if (M < 0 || N <= 0 || K <= 0) return fail(WDRZ_EINVAL, "bad sizes M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
+  if (M > 4 || K > 1536) return fail(WDRZ_EUNSUPPORTED, "M=%lld exceeds 4 or K=%lld exceeds 1536", (long long)M, (long long)K);
+  if (K % 128 != 0 || N % 8 != 0)
+    return fail(WDRZ_EUNSUPPORTED, "K=%lld must be a multiple of 128 and N=%lld of 8", (long long)K, (long long)N);
+  if (N > (1 << 24)) return fail(WDRZ_EUNSUPPORTED, "sizes too large");
+  if (partials && n_split != 2 && n_split != 4) return fail(WDRZ_EUNSUPPORTED, "n_split %d is not 2 or 4", n_split);
+  if (!(eps >= 0.f)) return fail(WDRZ_EINVAL, "eps must be >= 0");
+  if (M == 0) return WDRZ_OK;
+  int rc;
+  if ((rc = check_ptr("x", x)) || (rc = check_ptr("ln_weight", ln_weight)) || (rc = check_ptr("ln_bias", ln_bias)) ||
+      (rc = check_ptr("w", w)) || (rc = check_ptr("y", y)))
+    return rc;
+  if (partials && ((rc = check_ptr("partials", partials)) || (rc = check_ptr("delta_bias", delta_bias)) ||
+                   (rc = check_ptr("x_out", x_out))))
+    return rc;
+  if (partials && x_out == x) return fail(WDRZ_EINVAL, "x_out must not be x");
+  if (bias && (reinterpret_cast<uintptr_t>(bias) & 1)) return fail(WDRZ_EINVAL, "bias is not 2-byte aligned");
+  if (x_stride < K || w_stride < K || y_stride < N || (partials && x_out_stride < K))
+    return fail(WDRZ_EINVAL, "row strides shorter than the rows");
+  if ((x_stride * 2) % 16 || (w_stride * 2) % 16 || (y_stride * 2) % 16 || (partials && (x_out_stride * 2) % 16))
+    return fail(WDRZ_EINVAL, "row strides are not 16-byte aligned");
+  wdrz::LinearArgs a{};
+  a.w = w;
+  a.bias = bias;
+  a.y = y;
+  a.w_stride = w_stride;
+  a.y_stride = y_stride;
+  a.M = (int)M;
+  a.N = (int)N;
+  a.K = (int)K;
+  a.act = activation;
+  wdrz::AddLnArgs ln{};
+  ln.x = const_cast<void*>(x);
+  ln.x_stride = x_stride;
+  ln.weight = ln_weight;
+  ln.bias = ln_bias;
+  ln.rows = M;
+  ln.n = (int)K;
+  ln.eps = eps;
+  ln.dpart = partials;
+  ln.n_part = n_split;
+  ln.dbias = delta_bias;
+  hipError_t err = wdrz::launch_ln_linear(dtype, a, ln, x_out, x_out_stride, reinterpret_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(WDRZ_ELAUNCH, "kernel launch failed: %s", hipGetErrorString(err));
+  return WDRZ_OK;
+}
+
 int wdrz_add_layernorm_partials(int dtype, void* x, int64_t x_stride, const float* partials, int n_split,
                                 const void* delta_bias, const void* weight, const void* bias, void* y,
                                 int64_t y_stride, int64_t rows, int64_t n, float eps, void* stream) {

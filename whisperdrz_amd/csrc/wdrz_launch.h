@@ -170,6 +170,11 @@ struct LinearArgs {
 };
 hipError_t launch_linear(int dtype, const LinearArgs& a, hipStream_t stream);
 
+// Y = act(LayerNorm(x [+ delta]) W^T + b) for M <= 4 rows of K <= 1536: ln gives x, the partials and
+// the LayerNorm's parameters; the new residual goes to x_out (with partials only).
+hipError_t launch_ln_linear(int dtype, const LinearArgs& a, const AddLnArgs& ln, void* x_out, int64_t xo_stride,
+                            hipStream_t stream);
+
 // Log-mel front end over fp32 waveforms [B, n_samples] (row stride audio_stride elements).
 struct LogMelArgs {
   const float* audio;

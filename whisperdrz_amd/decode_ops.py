@@ -3,6 +3,8 @@
 * :func:`add_layernorm_` — ``x += delta; return ln(x)``: the residual add closing a sub-layer
   and the LayerNorm opening the next (reference ``src/whisperdrz/model.py:420-433``, the final
   ``ln`` at ``model.py:609-613``), one launch instead of two.
+* :func:`ln_linear` — the same add and LayerNorm inside the Linear that takes the result, for the
+  one to four rows of a small step.
 * :func:`masked_argmax` — ``decode_batch``'s greedy sampling tail (``decoding.py:1729-1761``):
   additive -65504 mask, repetition penalty, argmax, one launch instead of six.
 * :func:`linear_gelu` — the MLP's ``Linear(n_state, 4 n_state)`` + ``GELU`` (``model.py:388-391``,
@@ -20,7 +22,7 @@ import torch.nn as nn
 from . import _lib
 from .attention import _check_cuda, _dtype_code, _raise, _stream_handle
 
-__all__ = ["add_layernorm_", "layer_norm", "linear_gelu", "masked_argmax"]
+__all__ = ["add_layernorm_", "layer_norm", "linear_gelu", "ln_linear", "masked_argmax"]
 
 _LN16 = {torch.bfloat16: _lib.WDRZ_BF16, torch.float16: _lib.WDRZ_F16}
 
@@ -179,3 +181,50 @@ def add_layernorm_partials_(x: torch.Tensor, partials: torch.Tensor, lin: nn.Lin
     if rc != _lib.WDRZ_OK:
         _raise(rc, "add_layernorm_partials_")
     return y.view(x.shape)
+
+
+LN_LINEAR_ROWS = 4  # rows ln_linear takes (every workgroup repeats their LayerNorm)
+LN_LINEAR_MAX_K = 1536
+
+
+def ln_linear(x: torch.Tensor, ln: nn.LayerNorm, weight: torch.Tensor, bias: Optional[torch.Tensor],
+              gelu: bool = False, partials: Optional[torch.Tensor] = None,
+              lin: Optional[nn.Linear] = None) -> tuple[torch.Tensor, torch.Tensor]:
+    """``linear(add_layernorm_partials_(x, partials, lin, ln), weight, bias, gelu)`` in one launch,
+    for up to LN_LINEAR_ROWS rows of at most LN_LINEAR_MAX_K; without ``partials``
+    ``linear(layer_norm(x, ln), weight, bias, gelu)``. ``x`` is left as it is: returns the new
+    residual (``x`` itself without ``partials``) and the Linear's output."""
+    _check_cuda("x", x, x.device)
+    if x.dtype not in _LN16:
+        raise TypeError(f"x: dtype {x.dtype} is not supported (bfloat16, float16)")
+    xr = _rows(x, "x")
+    M, K = (int(v) for v in xr.shape)
+    w, b = weight.detach(), bias.detach() if bias is not None else None
+    lw, lb = ln.weight.detach(), ln.bias.detach()
+    if w.dtype != x.dtype or lw.dtype != x.dtype or (b is not None and b.dtype != x.dtype):
+        raise TypeError("the LayerNorm and Linear parameters must have the activations' dtype")
+    if w.stride(-1) != 1 or w.shape[1] != K or tuple(lw.shape) != (K,):
+        raise ValueError("weight must be [N, K] with contiguous rows and K = x.shape[-1] = the LayerNorm's width")
+    if b is not None and not b.is_contiguous():
+        b = b.contiguous()
+    db, x_new = None, x
+    if partials is not None:
+        if partials.dtype != torch.float32 or tuple(partials.shape[1:]) != (M, K) or not partials.is_contiguous():
+            raise ValueError("partials must be contiguous fp32 [n_split, rows, n] matching x")
+        if lin is None or lin.bias is None:
+            raise ValueError("partials need the Linear they come from, with a bias")
+        db = lin.bias.detach()
+        if db.dtype != x.dtype:
+            raise TypeError("the LayerNorm and Linear parameters must have the activations' dtype")
+        x_new = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+    N = int(w.shape[0])
+    y = torch.empty(M, N, dtype=x.dtype, device=x.device)
+    rc = _lib.load().wdrz_ln_linear(
+        _LN16[x.dtype], xr.data_ptr(), xr.stride(0), partials.data_ptr() if partials is not None else None,
+        int(partials.shape[0]) if partials is not None else 0, db.data_ptr() if db is not None else None,
+        x_new.data_ptr(), K, lw.data_ptr(), lb.data_ptr(), float(ln.eps), w.data_ptr(), w.stride(0),
+        b.data_ptr() if b is not None else None, y.data_ptr(), N, M, N, K, 1 if gelu else 0, _stream_handle(),
+    )
+    if rc != _lib.WDRZ_OK:
+        _raise(rc, "ln_linear")
+    return x_new, y.view(*x.shape[:-1], N)

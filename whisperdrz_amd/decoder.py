@@ -37,7 +37,8 @@ import torch.nn.functional as F
 from torch import Tensor
 
 from .attention import flash_attn_with_kvcache, scaled_dot_product_attention
-from .decode_ops import add_layernorm_, add_layernorm_partials_, layer_norm, linear, linear_gelu, linear_partials
+from .decode_ops import (LN_LINEAR_MAX_K, LN_LINEAR_ROWS, add_layernorm_, add_layernorm_partials_, layer_norm, linear,
+                         linear_gelu, linear_partials, ln_linear)
 from .kv_cache import FlashKVCache, KVSlotPool
 
 # Batch buckets of the captured decode step (reference transcriber.py:18).
@@ -134,23 +135,30 @@ class MultiHeadAttention(nn.Module):
         cross-attention's query projection). Same arithmetic per output element.
         ``project_out=False`` returns the attention output before ``out`` (the caller applies it,
         fused with the residual add)."""
-        B, seq_len, _ = x.shape
-        d = self.n_state // self.n_head
         if is_cross_attn:
-            # the query projection on the same 64-row kernel as the others (K % 128 == 0)
-            q = linear(x, self.query.weight, self.query.bias) if self.n_state % 128 == 0 else self.query(x)
-            q = q.view(B, seq_len, self.n_head, d)
-            o = self.attn_kvcache(q, kv_cache.k_cache, kv_cache.v_cache, cache_batch_idx=batch_idx,
-                                  softmax_scale=d ** -0.5, causal=False)
+            # the query projection on the same kernels as the others (K % 128 == 0)
+            proj = linear(x, self.query.weight, self.query.bias) if self.n_state % 128 == 0 else self.query(x)
         else:
             w, b = self.qkv_weight()
-            qkv = linear(x, w, b) if self.n_state % 128 == 0 else F.linear(x, w, b)
-            qkv = qkv.view(B, seq_len, 3, self.n_head, d)
+            proj = linear(x, w, b) if self.n_state % 128 == 0 else F.linear(x, w, b)
+        o = self.attend_step(proj, kv_cache, is_cross_attn, cache_seqlens, batch_idx)
+        return self.out(o) if project_out else o
+
+    def attend_step(self, proj: Tensor, kv_cache: FlashKVCache, is_cross_attn: bool,
+                    cache_seqlens: Optional[Tensor], batch_idx: Optional[Tensor]) -> Tensor:
+        """The cached attention of projected rows: ``proj`` is the query (cross) or the query, key
+        and value next to each other (self)."""
+        B, seq_len, _ = proj.shape
+        d = self.n_state // self.n_head
+        if is_cross_attn:
+            o = self.attn_kvcache(proj.view(B, seq_len, self.n_head, d), kv_cache.k_cache, kv_cache.v_cache,
+                                  cache_batch_idx=batch_idx, softmax_scale=d ** -0.5, causal=False)
+        else:
+            qkv = proj.view(B, seq_len, 3, self.n_head, d)
             o = self.attn_kvcache(qkv[:, :, 0], kv_cache.k_cache, kv_cache.v_cache, k=qkv[:, :, 1], v=qkv[:, :, 2],
                                   cache_seqlens=cache_seqlens, cache_batch_idx=batch_idx, softmax_scale=d ** -0.5,
                                   causal=self.causal)
-        o = o.reshape(B, seq_len, self.n_state)
-        return self.out(o) if project_out else o
+        return o.reshape(B, seq_len, self.n_state)
 
     def forward_flash(self, x: Tensor, kv_cache: FlashKVCache, is_cross_attn: bool = False,
                       slot_indices: Optional[Tensor] = None) -> Tensor:
@@ -257,6 +265,22 @@ class TextDecoderStack(nn.Module):
             layer_lens = [seqlens[i] for i in range(len(blocks))]
         else:
             layer_lens = [s.seq_lens if slot_indices is None else s.seq_lens[slot_indices] for s in self_kv]
+        # a small step: every add + LayerNorm inside the projection that follows it
+        n = self.n_state
+        if (x.numel() // n if n else 0) <= LN_LINEAR_ROWS and n % 256 == 0 and n <= LN_LINEAR_MAX_K and all(
+                m.bias is not None for b in blocks for m in (b.attn.out, b.cross_attn.out, b.mlp[2])):
+            part = lin = None
+            for i, (block, s_kv, c_kv) in enumerate(zip(blocks, self_kv, cross_kv, strict=True)):
+                attn, cross, fc1, fc2 = block.attn, block.cross_attn, block.mlp[0], block.mlp[2]
+                x, qkv = ln_linear(x, block.attn_ln, *attn.qkv_weight(), partials=part, lin=lin)
+                o = attn.attend_step(qkv, s_kv, False, layer_lens[i], batch_idx)
+                x, q = ln_linear(x, block.cross_attn_ln, cross.query.weight, cross.query.bias,
+                                 partials=linear_partials(o, attn.out, 2), lin=attn.out)
+                o = cross.attend_step(q, c_kv, True, None, batch_idx)
+                x, h = ln_linear(x, block.mlp_ln, fc1.weight, fc1.bias, gelu=True,
+                                 partials=linear_partials(o, cross.out, 2), lin=cross.out)
+                part, lin = linear_partials(h, fc2, 4), fc2
+            return add_layernorm_partials_(x, part, lin, self.ln)
         h = layer_norm(x, blocks[0].attn_ln)
         for i, (block, s_kv, c_kv) in enumerate(zip(blocks, self_kv, cross_kv, strict=True)):
             o = block.attn.forward_flash_step(h, s_kv, False, layer_lens[i], batch_idx, project_out=False)
