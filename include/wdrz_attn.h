@@ -233,9 +233,9 @@ int wdrz_add_layernorm_partials(int dtype, void* x, int64_t x_stride, const floa
  * Replaces: the residual add closing a sub-layer, the LayerNorm opening the next and that
  *           sub-layer's first projection (src/whisperdrz/model.py:420-434: attn_ln + query / key /
  *           value, cross_attn_ln + query, mlp_ln + the MLP's first Linear and GELU).
- * With partials (fp32 [n_split][M][K], wdrz_linear_partials' output) and delta_bias:
- *   r = round(x + round(sum of the partials + delta_bias)), stored to x_out [M, K] (a buffer other
- *   than x); without (partials NULL): r = x and x_out is not used.
+ * partials (fp32 [n_split][M][K], wdrz_linear_partials' output) and delta_bias:
+ *   r = round(x + round(sum of the partials + delta_bias)), stored to x_out [M, K], a buffer other
+ *   than x.
  * y = act(LayerNorm(r) w^T + bias) [M, N], rounded as wdrz_add_layernorm_partials and wdrz_linear
  *   round. w: [N, K] rows; bias may be NULL; activation as in wdrz_linear.
  * M <= 4, K <= 1536, K % 128 == 0, N % 8 == 0, n_split 2 or 4; 16-byte aligned pointers (bias and
@@ -246,6 +246,37 @@ int wdrz_ln_linear(int dtype, const void* x, int64_t x_stride, const float* part
                    const void* ln_bias, float eps, const void* w, int64_t w_stride,
                    const void* bias, void* y, int64_t y_stride, int64_t M, int64_t N, int64_t K,
                    int activation, void* stream);
+
+/*
+ * The start of a cached decoder step: embeddings, the first LayerNorm and the step's metadata.
+ *
+ * Replaces: x = token_embedding(tokens) + positional_embedding[positions] and the first block's
+ *           attn_ln (src/whisperdrz/model.py:586-600, 420), and per layer the gather
+ *           seq_lens[slot_indices] and the int32 slot map (model.py:327-334).
+ * tokens, positions: int64 [B, sq], element strides tok_strides[2] / pos_strides[2]; emb: 16-bit
+ *   [n_vocab, n], row stride emb_stride; pos_emb: [n_ctx, n]; x, y: [B * sq, n] contiguous:
+ *   x = round(emb + pos_emb), y = LayerNorm(x) as wdrz_add_layernorm computes it.
+ * slots: int64 [B] or NULL (slot b); slots32: int32 [B] (written when slots is given);
+ * lens: int32 [n_layers, n_slots] contiguous; seqlens: int32 [n_layers, B] = lens[l, slot of b].
+ * Negative positions and slots count from the end. A token or position out of range gives a NaN
+ *   row, a slot out of range the length -1 (which attention turns into NaN).
+ * n a multiple of 8, <= 2048; 16-byte aligned tables, rows and parameters.
+ */
+int wdrz_step_begin(int dtype, const int64_t* tokens, const int64_t* tok_strides,
+                    const int64_t* positions, const int64_t* pos_strides, const void* emb,
+                    int64_t emb_stride, int64_t n_vocab, const void* pos_emb,
+                    int64_t pos_emb_stride, int64_t n_ctx, const void* ln_weight,
+                    const void* ln_bias, float eps, void* x, void* y, const int64_t* slots,
+                    int32_t* slots32, const int32_t* lens, int32_t* seqlens, int64_t B,
+                    int64_t sq, int64_t n, int64_t n_layers, int64_t n_slots, void* stream);
+
+/*
+ * The end of a cached decoder step: lens[l, slot of b] = seqlens[l, b] + sq for every layer, the
+ * bump of seq_lens after all layers (src/whisperdrz/model.py:602-607). Arguments as in
+ * wdrz_step_begin; repeated slots are bumped once, as torch's indexed add does.
+ */
+int wdrz_step_end(int32_t* lens, const int32_t* seqlens, const int64_t* slots, int64_t B,
+                  int64_t sq, int64_t n_layers, int64_t n_slots, void* stream);
 
 /*
  * Greedy sampling with the decode step's token constraints.

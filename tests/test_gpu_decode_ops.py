@@ -154,3 +154,45 @@ def test_masked_argmax_vector_edges(cuda, dtype, V):
         got = masked_argmax(logits, b, p)
         want = _reference_sampling(logits, b[:, :V] if b is not None else None, p[:, :V] if p is not None else None)
         assert torch.equal(got, want), (V, got.tolist(), want.tolist())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,sq,n,with_slots", [(1, 1, 1280, True), (5, 1, 8, True), (3, 7, 520, False), (70, 2, 2048, True)])
+def test_step_begin_end(cuda, dtype, B, sq, n, with_slots):
+    """The prologue against torch's indexing, add and this library's LayerNorm (same bits), and the
+    epilogue's bump: repeated and negative slots, strided indices, ids out of range."""
+    from whisperdrz_amd import layer_norm
+    from whisperdrz_amd.decode_ops import step_begin, step_end_
+
+    g = torch.Generator(device=cuda).manual_seed(B * n + sq)
+    V, ctx, layers, n_slots = 50, 20, 3, B + 4
+    emb, pos = (torch.randn(r, n, generator=g, device=cuda).to(dtype) for r in (V, ctx))
+    ln = torch.nn.LayerNorm(n).to(cuda, dtype)
+    with torch.no_grad():
+        ln.weight.copy_(1 + 0.1 * torch.randn(n, generator=g, device=cuda))
+    tokens = torch.randint(0, V, (B, 2 * sq), generator=g, device=cuda)[:, ::2]
+    positions = torch.randint(-ctx, ctx, (B,), generator=g, device=cuda).unsqueeze(1).expand(B, sq)
+    lens = torch.randint(0, 9, (layers, n_slots), generator=g, device=cuda, dtype=torch.int32)
+    slots = torch.randint(-n_slots, n_slots, (B,), generator=g, device=cuda) if with_slots else None
+    x, h, slots32, seqlens = step_begin(tokens, positions, emb, pos, ln, slots, lens)
+    want = emb[tokens] + pos[positions]
+    assert torch.equal(x, want) and torch.equal(h, layer_norm(want, ln))
+    want_lens = lens.clone()
+    if with_slots:
+        assert torch.equal(slots32, slots.int()) and torch.equal(seqlens, lens[:, slots])
+        want_lens[:, slots] += sq
+    else:
+        assert slots32 is None and torch.equal(seqlens, lens[:, :B])
+        want_lens[:, :B] += sq
+    step_end_(lens, seqlens, slots, sq)
+    assert torch.equal(lens, want_lens)
+    # out of range: NaN rows, length -1, nothing bumped; the other rows as before
+    tokens = tokens.clone()
+    tokens[0, 0] = V
+    if with_slots:
+        slots[0] = n_slots
+    x2, h2, _, seqlens2 = step_begin(tokens, positions, emb, pos, ln, slots, lens)
+    assert x2[0, 0].isnan().all() and h2[0, 0].isnan().all()
+    assert torch.equal(x2.view(B * sq, n)[1:], x.view(B * sq, n)[1:])
+    if with_slots:
+        assert (seqlens2[:, 0] == -1).all()

@@ -153,13 +153,13 @@ def test_linear_partials_errors(cuda):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("n_split", [0, 2, 4])
+@pytest.mark.parametrize("n_split", [2, 4])
 @pytest.mark.parametrize("M,N,K", [(1, 3840, 1280), (4, 40, 128), (3, 8, 1536), (2, 1280, 384)])
 def test_ln_linear_equals_its_parts(cuda, dtype, n_split, M, N, K):
     """add + LayerNorm + Linear in one launch against the two launches: the residual is the same
     bits, and so are the LayerNorm's rows, the Linear's input; its K order is the few-row Linear's,
     so the outputs are the same bits too."""
-    from whisperdrz_amd import add_layernorm_partials_, layer_norm, linear, ln_linear
+    from whisperdrz_amd import add_layernorm_partials_, linear, ln_linear
 
     g = torch.Generator(device=cuda).manual_seed(M + N + K + n_split)
     ln = torch.nn.LayerNorm(K).to(cuda, dtype)
@@ -170,25 +170,29 @@ def test_ln_linear_equals_its_parts(cuda, dtype, n_split, M, N, K):
     w = (torch.randn(N, K, generator=g, device=cuda) / K ** 0.5).to(dtype)
     b = torch.randn(N, generator=g, device=cuda).to(dtype)
     x = torch.randn(M, K + 8, generator=g, device=cuda).to(dtype)[:, :K]
-    part = torch.randn(n_split, M, K, generator=g, device=cuda) if n_split else None
+    part = torch.randn(n_split, M, K, generator=g, device=cuda)
     for gelu, bias in ((True, b), (False, None)):
         want_x = x.clone()
-        h = add_layernorm_partials_(want_x, part, fc, ln) if n_split else layer_norm(want_x, ln)
+        h = add_layernorm_partials_(want_x, part, fc, ln)
         want = linear(h, w, bias, gelu)
         before = x.clone()
-        got_x, got = ln_linear(x, ln, w, bias, gelu, partials=part, lin=fc if n_split else None)
+        got_x, got = ln_linear(x, part, fc, ln, w, bias, gelu)
         assert torch.equal(x, before) and torch.equal(got_x, want_x) and torch.equal(got, want)
 
 
 def test_ln_linear_errors(cuda):
     from whisperdrz_amd import ln_linear
 
-    ln = torch.nn.LayerNorm(128).to(cuda, torch.bfloat16)
-    w = torch.randn(32, 128, device=cuda).to(torch.bfloat16)
+    dt = torch.bfloat16
+    ln, fc = torch.nn.LayerNorm(128).to(cuda, dt), torch.nn.Linear(8, 128).to(cuda, dt)
+    w = torch.randn(32, 128, device=cuda).to(dt)
+    part = torch.zeros(2, 5, 128, device=cuda)
     with pytest.raises(NotImplementedError, match="exceeds 4"):
-        ln_linear(torch.randn(5, 128, device=cuda).to(torch.bfloat16), ln, w, None)
-    x = torch.randn(2, 128, device=cuda).to(torch.bfloat16)
-    with pytest.raises(ValueError, match="Linear they come from"):
-        ln_linear(x, ln, w, None, partials=torch.zeros(2, 2, 128, device=cuda))
+        ln_linear(torch.randn(5, 128, device=cuda).to(dt), part, fc, ln, w, None)
+    x = torch.randn(2, 128, device=cuda).to(dt)
+    with pytest.raises(ValueError, match="partials"):
+        ln_linear(x, part, fc, ln, w, None)
+    with pytest.raises(NotImplementedError, match="n_split 3"):
+        ln_linear(x, torch.zeros(3, 2, 128, device=cuda), fc, ln, w, None)
     with pytest.raises(TypeError):
-        ln_linear(x.float(), ln, w, None)
+        ln_linear(x.float(), part[:, :2].contiguous(), fc, ln, w, None)

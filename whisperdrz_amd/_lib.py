@@ -40,6 +40,8 @@ EXPORTED_SYMBOLS = (
     "wdrz_linear_partials",
     "wdrz_add_layernorm_partials",
     "wdrz_ln_linear",
+    "wdrz_step_begin",
+    "wdrz_step_end",
     "wdrz_log_mel_workspace_size",
     "wdrz_log_mel",
     "wdrz_dtw_qk",
@@ -114,6 +116,16 @@ def _declare(lib: ctypes.CDLL) -> None:
         _p, _p, ctypes.c_float, _p, _i64, _p,  # LayerNorm weight, bias, eps; w, stride, bias
         _p, _i64, _i64, _i64, _i64, ctypes.c_int, _p,  # y, stride, M, N, K, activation, stream
     ]
+    lib.wdrz_step_begin.restype = ctypes.c_int
+    lib.wdrz_step_begin.argtypes = [
+        ctypes.c_int, _p, _i64p, _p, _i64p,  # dtype, tokens, strides, positions, strides
+        _p, _i64, _i64, _p, _i64, _i64,  # emb, stride, n_vocab, pos_emb, stride, n_ctx
+        _p, _p, ctypes.c_float, _p, _p,  # LayerNorm weight, bias, eps, x, y
+        _p, _p, _p, _p,  # slots, slots32, lens, seqlens
+        _i64, _i64, _i64, _i64, _i64, _p,  # B, sq, n, n_layers, n_slots, stream
+    ]
+    lib.wdrz_step_end.restype = ctypes.c_int
+    lib.wdrz_step_end.argtypes = [_p, _p, _p, _i64, _i64, _i64, _i64, _p]  # lens, seqlens, slots, sizes, stream
     lib.wdrz_masked_argmax.restype = ctypes.c_int
     lib.wdrz_masked_argmax.argtypes = [
         ctypes.c_int, _p, _i64, _p, _i64, _p, _i64,  # dtype, logits, stride, blocked, stride, penalty, stride

@@ -7,7 +7,11 @@
 //    the LayerNorm (eps 1e-5, affine) is computed in fp32 from the rounded sum, as torch's
 //    LayerNorm does for 16-bit inputs, and rounded once. One wavefront per row; the row stays in
 //    registers between the mean and the variance pass.
-// 2. wdrz_masked_argmax: decode_batch's greedy sampling tail (src/whisperdrz/decoding.py:
+// 2. wdrz_step_begin / wdrz_step_end: what a cached step does around its blocks (src/whisperdrz/
+//    model.py:586-613): x = token embedding + positional embedding with the first LayerNorm, the
+//    int32 slot map and every layer's gathered cache lengths; after the blocks the lengths' bump.
+//    One launch each instead of six and three of torch's (2-4 us each for a few KB).
+// 3. wdrz_masked_argmax: decode_batch's greedy sampling tail (src/whisperdrz/decoding.py:
 //    1729-1761): masked = logits + (-65504 where blocked), then the repetition penalty
 //    (x > 0 ? x / 1.2 : x * 1.2 where penalised), argmax. Each step rounds to the logits' type
 //    as the torch ops do; ties go to the lowest index, as torch.argmax. One workgroup per row.
@@ -33,6 +37,66 @@ __global__ __launch_bounds__(256) void add_layernorm_kernel(AddLnArgs a) {
   r.load(a, row, lane);
   r.finish(a, lane, [&](int c, u32x4 w) { *reinterpret_cast<u32x4*>(xrow + c * 16) = w; },
            [&](int c, u32x4 w) { *reinterpret_cast<u32x4*>(yrow + c * 16) = w; });
+}
+
+// ---- step prologue and epilogue -------------------------------------------------------------
+// Workgroups [0, ceil(rows / 4)): a wavefront per row (b, t) looks up its two embedding rows, adds
+// them (rounded as torch's add) and normalises the sum. The workgroups behind them: one thread per
+// (layer, batch row) gathers a cache length, one per batch row converts a slot id. Slots and
+// positions count from the end when negative, as in torch's indexing (the slot map keeps the id as
+// it is: attention gives such a row NaN); a token, position or slot out of range reads nothing and
+// gives a NaN row (a slot through its length -1).
+template <typename T, int NC>
+__global__ __launch_bounds__(256) void step_begin_kernel(StepArgs a, AddLnArgs ln) {
+  const int row_wgs = (a.B * a.sq + 3) / 4;
+  if ((int)blockIdx.x >= row_wgs) {
+    const int i = ((int)blockIdx.x - row_wgs) * 256 + threadIdx.x;
+    const int b = i % a.B, l = i / a.B;
+    if (l > a.n_layers) return;
+    const int64_t slot = a.slots ? a.slots[b] : b;
+    if (l == a.n_layers) {
+      if (a.slots) a.slots32[b] = (int32_t)slot;
+    } else {
+      const int64_t s = slot < 0 ? slot + a.n_slots : slot;
+      a.seqlens[(int64_t)l * a.B + b] = s >= 0 && s < a.n_slots ? a.lens[(int64_t)l * a.n_slots + s] : -1;
+    }
+    return;
+  }
+  const int lane = threadIdx.x & 63;
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= a.B * a.sq) return;
+  const int b = row / a.sq, t = row % a.sq;
+  const int64_t tok = a.tokens[b * a.ts[0] + t * a.ts[1]];
+  int64_t pos = a.positions[b * a.ps[0] + t * a.ps[1]];
+  pos = pos < 0 ? pos + a.n_ctx : pos;
+  char* xrow = static_cast<char*>(a.x) + (int64_t)row * ln.n * 2;
+  char* yrow = static_cast<char*>(ln.y) + (int64_t)row * ln.n * 2;
+  auto store_x = [&](int c, u32x4 w) { *reinterpret_cast<u32x4*>(xrow + c * 16) = w; };
+  auto store_y = [&](int c, u32x4 w) { *reinterpret_cast<u32x4*>(yrow + c * 16) = w; };
+  if (tok < 0 || tok >= a.n_vocab || pos < 0 || pos >= a.n_ctx) {
+    const u32x4 nan = {0x7fff7fffu, 0x7fff7fffu, 0x7fff7fffu, 0x7fff7fffu};
+    for (int c = lane; c < ln.n / 8; c += 64) {
+      store_x(c, nan);
+      store_y(c, nan);
+    }
+    return;
+  }
+  ln.x = static_cast<char*>(ln.x) + tok * ln.x_stride * 2;
+  ln.delta = static_cast<const char*>(ln.delta) + pos * ln.d_stride * 2;
+  LnRow<T, NC, 0> r;
+  r.load(ln, 0, lane);
+  r.finish(ln, lane, store_x, store_y);
+}
+
+// lens[l, slot of b] = the length gathered at the start + sq: repeated slots store the same value,
+// as torch's indexed add does.
+__global__ __launch_bounds__(256) void step_end_kernel(StepArgs a) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int b = i % a.B, l = i / a.B;
+  if (l >= a.n_layers) return;
+  int64_t s = a.slots ? a.slots[b] : b;
+  s = s < 0 ? s + a.n_slots : s;
+  if (s >= 0 && s < a.n_slots) a.lens[(int64_t)l * a.n_slots + s] = a.seqlens[(int64_t)l * a.B + b] + a.sq;
 }
 
 // ---- masked greedy sampling --------------------------------------------------------------
@@ -168,6 +232,29 @@ hipError_t launch_add_layernorm(int dtype, const AddLnArgs& a, hipStream_t strea
 #undef WDRZ_LN
 #undef WDRZ_LNP
 #undef WDRZ_LN3
+  return hipGetLastError();
+}
+
+hipError_t launch_step_begin(int dtype, const StepArgs& a, const AddLnArgs& ln, hipStream_t stream) {
+  const int64_t meta = (int64_t)(a.n_layers + 1) * a.B;
+  const dim3 grid((unsigned)((a.B * a.sq + 3) / 4 + (meta + 255) / 256));
+#define WDRZ_SB(NC)                                                                                       \
+  case NC:                                                                                                \
+    if (dtype == 2) hipLaunchKernelGGL((step_begin_kernel<Bf16, NC>), grid, dim3(256), 0, stream, a, ln); \
+    else hipLaunchKernelGGL((step_begin_kernel<F16, NC>), grid, dim3(256), 0, stream, a, ln);             \
+    break;
+  switch ((ln.n + 511) / 512) {
+    WDRZ_SB(1) WDRZ_SB(2) WDRZ_SB(3) WDRZ_SB(4)
+    default:
+      return hipErrorInvalidValue;
+  }
+#undef WDRZ_SB
+  return hipGetLastError();
+}
+
+hipError_t launch_step_end(const StepArgs& a, hipStream_t stream) {
+  const int64_t n = (int64_t)a.n_layers * a.B;
+  hipLaunchKernelGGL(step_end_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 

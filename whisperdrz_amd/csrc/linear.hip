@@ -314,14 +314,13 @@ void launch_rows(const LinearArgs& a, hipStream_t stream) {
 template <typename T, int ACT>
 void launch_ln_rows(const LinearArgs& a, const AddLnArgs& ln, void* x_out, int64_t xo_stride, hipStream_t stream) {
   const dim3 grid((unsigned)((a.N + 15) / 16)), block(64 * kRowWaves);
-  if (!ln.dpart) hipLaunchKernelGGL((ln_linear_kernel<T, ACT, 0>), grid, block, 0, stream, a, ln, x_out, xo_stride);
-  else if (ln.n_part == 2) hipLaunchKernelGGL((ln_linear_kernel<T, ACT, 2>), grid, block, 0, stream, a, ln, x_out, xo_stride);
+  if (ln.n_part == 2) hipLaunchKernelGGL((ln_linear_kernel<T, ACT, 2>), grid, block, 0, stream, a, ln, x_out, xo_stride);
   else hipLaunchKernelGGL((ln_linear_kernel<T, ACT, 4>), grid, block, 0, stream, a, ln, x_out, xo_stride);
 }
 
 hipError_t launch_ln_linear(int dtype, const LinearArgs& a, const AddLnArgs& ln, void* x_out, int64_t xo_stride,
                             hipStream_t stream) {
-  if (a.M < 1 || a.M > kLnRowMax || a.K > kLnMaxK || a.K != ln.n) return hipErrorInvalidValue;
+  if (a.M < 1 || a.M > kLnRowMax || a.K > kLnMaxK || a.K != ln.n || (ln.n_part != 2 && ln.n_part != 4)) return hipErrorInvalidValue;
   if (dtype == 2) {
     if (a.act) launch_ln_rows<Bf16, 1>(a, ln, x_out, xo_stride, stream);
     else launch_ln_rows<Bf16, 0>(a, ln, x_out, xo_stride, stream);

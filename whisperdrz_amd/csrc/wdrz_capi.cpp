@@ -500,21 +500,19 @@ int wdrz_ln_linear(int dtype, const void* x, int64_t x_stride, const float* part
   if (K % 128 != 0 || N % 8 != 0)
     return fail(WDRZ_EUNSUPPORTED, "K=%lld must be a multiple of 128 and N=%lld of 8", (long long)K, (long long)N);
   if (N > (1 << 24)) return fail(WDRZ_EUNSUPPORTED, "sizes too large");
-  if (partials && n_split != 2 && n_split != 4) return fail(WDRZ_EUNSUPPORTED, "n_split %d is not 2 or 4", n_split);
+  if (n_split != 2 && n_split != 4) return fail(WDRZ_EUNSUPPORTED, "n_split %d is not 2 or 4", n_split);
   if (!(eps >= 0.f)) return fail(WDRZ_EINVAL, "eps must be >= 0");
   if (M == 0) return WDRZ_OK;
   int rc;
   if ((rc = check_ptr("x", x)) || (rc = check_ptr("ln_weight", ln_weight)) || (rc = check_ptr("ln_bias", ln_bias)) ||
-      (rc = check_ptr("w", w)) || (rc = check_ptr("y", y)))
+      (rc = check_ptr("w", w)) || (rc = check_ptr("y", y)) || (rc = check_ptr("partials", partials)) ||
+      (rc = check_ptr("delta_bias", delta_bias)) || (rc = check_ptr("x_out", x_out)))
     return rc;
-  if (partials && ((rc = check_ptr("partials", partials)) || (rc = check_ptr("delta_bias", delta_bias)) ||
-                   (rc = check_ptr("x_out", x_out))))
-    return rc;
-  if (partials && x_out == x) return fail(WDRZ_EINVAL, "x_out must not be x");
+  if (x_out == x) return fail(WDRZ_EINVAL, "x_out must not be x");
   if (bias && (reinterpret_cast<uintptr_t>(bias) & 1)) return fail(WDRZ_EINVAL, "bias is not 2-byte aligned");
-  if (x_stride < K || w_stride < K || y_stride < N || (partials && x_out_stride < K))
+  if (x_stride < K || w_stride < K || y_stride < N || x_out_stride < K)
     return fail(WDRZ_EINVAL, "row strides shorter than the rows");
-  if ((x_stride * 2) % 16 || (w_stride * 2) % 16 || (y_stride * 2) % 16 || (partials && (x_out_stride * 2) % 16))
+  if ((x_stride * 2) % 16 || (w_stride * 2) % 16 || (y_stride * 2) % 16 || (x_out_stride * 2) % 16)
     return fail(WDRZ_EINVAL, "row strides are not 16-byte aligned");
   wdrz::LinearArgs a{};
   a.w = w;
@@ -538,6 +536,87 @@ int wdrz_ln_linear(int dtype, const void* x, int64_t x_stride, const float* part
   ln.n_part = n_split;
   ln.dbias = delta_bias;
   hipError_t err = wdrz::launch_ln_linear(dtype, a, ln, x_out, x_out_stride, reinterpret_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(WDRZ_ELAUNCH, "kernel launch failed: %s", hipGetErrorString(err));
+  return WDRZ_OK;
+}
+
+int wdrz_step_begin(int dtype, const int64_t* tokens, const int64_t* tok_strides, const int64_t* positions,
+                    const int64_t* pos_strides, const void* emb, int64_t emb_stride, int64_t n_vocab,
+                    const void* pos_emb, int64_t pos_emb_stride, int64_t n_ctx, const void* ln_weight,
+                    const void* ln_bias, float eps, void* x, void* y, const int64_t* slots, int32_t* slots32,
+                    const int32_t* lens, int32_t* seqlens, int64_t B, int64_t sq, int64_t n, int64_t n_layers,
+                    int64_t n_slots, void* stream) {
+  g_last_error.clear();
+  if (dtype != WDRZ_BF16 && dtype != WDRZ_F16)
+    return fail(dtype == WDRZ_F32 ? WDRZ_EUNSUPPORTED : WDRZ_EINVAL, "dtype %d: only WDRZ_BF16 / WDRZ_F16", dtype);
+  if (B < 0 || sq <= 0 || n <= 0 || n % 8 != 0 || n_layers < 0 || n_slots < 0 || n_vocab < 0 || n_ctx < 0)
+    return fail(WDRZ_EINVAL, "bad sizes B=%lld sq=%lld n=%lld (n must be a positive multiple of 8)", (long long)B,
+                (long long)sq, (long long)n);
+  if (n > 2048) return fail(WDRZ_EUNSUPPORTED, "n=%lld exceeds the supported 2048", (long long)n);
+  if (B > (1 << 20) || sq > (1 << 20) || B * sq > (1 << 28) || n_layers > 65535 || (n_layers + 1) * B > (1 << 30) ||
+      n_slots > (1 << 24))
+    return fail(WDRZ_EUNSUPPORTED, "sizes too large");
+  if (!(eps >= 0.f)) return fail(WDRZ_EINVAL, "eps must be >= 0");
+  if (B == 0) return WDRZ_OK;
+  if (!tokens || !positions || !tok_strides || !pos_strides) return fail(WDRZ_EINVAL, "tokens / positions is NULL");
+  int rc;
+  if ((rc = check_ptr("emb", emb)) || (rc = check_ptr("pos_emb", pos_emb)) || (rc = check_ptr("ln_weight", ln_weight)) ||
+      (rc = check_ptr("ln_bias", ln_bias)) || (rc = check_ptr("x", x)) || (rc = check_ptr("y", y)))
+    return rc;
+  if ((emb_stride * 2) % 16 || (pos_emb_stride * 2) % 16) return fail(WDRZ_EINVAL, "row strides are not 16-byte aligned");
+  if (slots && !slots32) return fail(WDRZ_EINVAL, "slots32 is NULL");
+  if (n_layers > 0 && (!lens || !seqlens)) return fail(WDRZ_EINVAL, "lens / seqlens is NULL");
+  wdrz::StepArgs a{};
+  a.tokens = tokens;
+  a.positions = positions;
+  for (int i = 0; i < 2; ++i) {
+    a.ts[i] = tok_strides[i];
+    a.ps[i] = pos_strides[i];
+  }
+  a.n_vocab = n_vocab;
+  a.n_ctx = n_ctx;
+  a.x = x;
+  a.slots = slots;
+  a.slots32 = slots32;
+  a.lens = const_cast<int32_t*>(lens);
+  a.seqlens = seqlens;
+  a.B = (int)B;
+  a.sq = (int)sq;
+  a.n_layers = (int)n_layers;
+  a.n_slots = (int)n_slots;
+  wdrz::AddLnArgs ln{};
+  ln.x = const_cast<void*>(emb);
+  ln.x_stride = emb_stride;
+  ln.delta = pos_emb;
+  ln.d_stride = pos_emb_stride;
+  ln.weight = ln_weight;
+  ln.bias = ln_bias;
+  ln.y = y;
+  ln.rows = B * sq;
+  ln.n = (int)n;
+  ln.eps = eps;
+  hipError_t err = wdrz::launch_step_begin(dtype, a, ln, reinterpret_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(WDRZ_ELAUNCH, "kernel launch failed: %s", hipGetErrorString(err));
+  return WDRZ_OK;
+}
+
+int wdrz_step_end(int32_t* lens, const int32_t* seqlens, const int64_t* slots, int64_t B, int64_t sq,
+                  int64_t n_layers, int64_t n_slots, void* stream) {
+  g_last_error.clear();
+  if (B < 0 || sq < 0 || n_layers < 0 || n_slots < 0) return fail(WDRZ_EINVAL, "bad sizes");
+  if (B > (1 << 20) || sq > (1 << 20) || n_layers > 65535 || n_layers * B > (1 << 30) || n_slots > (1 << 24))
+    return fail(WDRZ_EUNSUPPORTED, "sizes too large");
+  if (B == 0 || n_layers == 0) return WDRZ_OK;
+  if (!lens || !seqlens) return fail(WDRZ_EINVAL, "lens / seqlens is NULL");
+  wdrz::StepArgs a{};
+  a.slots = slots;
+  a.lens = lens;
+  a.seqlens = const_cast<int32_t*>(seqlens);
+  a.B = (int)B;
+  a.sq = (int)sq;
+  a.n_layers = (int)n_layers;
+  a.n_slots = (int)n_slots;
+  hipError_t err = wdrz::launch_step_end(a, reinterpret_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(WDRZ_ELAUNCH, "kernel launch failed: %s", hipGetErrorString(err));
   return WDRZ_OK;
 }

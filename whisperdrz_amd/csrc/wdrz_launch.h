@@ -116,6 +116,23 @@ struct AddLnArgs {
 };
 hipError_t launch_add_layernorm(int dtype, const AddLnArgs& a, hipStream_t stream);
 
+// A cached step's prologue and epilogue (decode_ops.hip). launch_step_begin's ln: x = the token
+// embedding table, delta = the positional table, y = the normalised rows (contiguous).
+struct StepArgs {
+  const int64_t* tokens;     // [B, sq], strides ts
+  const int64_t* positions;  // [B, sq], strides ps
+  int64_t ts[2], ps[2];
+  int64_t n_vocab, n_ctx;
+  void* x;                // [B * sq, n] residual rows
+  const int64_t* slots;   // [B] or nullptr (slot b)
+  int32_t* slots32;       // [B]
+  int32_t* lens;          // [n_layers, n_slots]
+  int32_t* seqlens;       // [n_layers, B]
+  int B, sq, n_layers, n_slots;
+};
+hipError_t launch_step_begin(int dtype, const StepArgs& a, const AddLnArgs& ln, hipStream_t stream);
+hipError_t launch_step_end(const StepArgs& a, hipStream_t stream);
+
 // Masked greedy sampling over logits rows (strides in elements / bytes for the masks).
 // Rows of projected K/V into the slot caches (kv_fill.hip): cache[slot[b], start + t, h, :] =
 // src[b, t, h, :] for K and V; 16-bit elements, head_dim 64, strides in elements.
@@ -170,8 +187,8 @@ struct LinearArgs {
 };
 hipError_t launch_linear(int dtype, const LinearArgs& a, hipStream_t stream);
 
-// Y = act(LayerNorm(x [+ delta]) W^T + b) for M <= 4 rows of K <= 1536: ln gives x, the partials and
-// the LayerNorm's parameters; the new residual goes to x_out (with partials only).
+// Y = act(LayerNorm(x + delta) W^T + b) for M <= 4 rows of K <= 1536: ln gives x, the delta's
+// partials and the LayerNorm's parameters; the new residual goes to x_out.
 hipError_t launch_ln_linear(int dtype, const LinearArgs& a, const AddLnArgs& ln, void* x_out, int64_t xo_stride,
                             hipStream_t stream);
 

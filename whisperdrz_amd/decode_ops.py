@@ -187,44 +187,92 @@ LN_LINEAR_ROWS = 4  # rows ln_linear takes (every workgroup repeats their LayerN
 LN_LINEAR_MAX_K = 1536
 
 
-def ln_linear(x: torch.Tensor, ln: nn.LayerNorm, weight: torch.Tensor, bias: Optional[torch.Tensor],
-              gelu: bool = False, partials: Optional[torch.Tensor] = None,
-              lin: Optional[nn.Linear] = None) -> tuple[torch.Tensor, torch.Tensor]:
+def ln_linear(x: torch.Tensor, partials: torch.Tensor, lin: nn.Linear, ln: nn.LayerNorm, weight: torch.Tensor,
+              bias: Optional[torch.Tensor], gelu: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
     """``linear(add_layernorm_partials_(x, partials, lin, ln), weight, bias, gelu)`` in one launch,
-    for up to LN_LINEAR_ROWS rows of at most LN_LINEAR_MAX_K; without ``partials``
-    ``linear(layer_norm(x, ln), weight, bias, gelu)``. ``x`` is left as it is: returns the new
-    residual (``x`` itself without ``partials``) and the Linear's output."""
+    for up to LN_LINEAR_ROWS rows of at most LN_LINEAR_MAX_K. ``x`` is left as it is: returns the
+    new residual and the Linear's output."""
     _check_cuda("x", x, x.device)
     if x.dtype not in _LN16:
         raise TypeError(f"x: dtype {x.dtype} is not supported (bfloat16, float16)")
     xr = _rows(x, "x")
     M, K = (int(v) for v in xr.shape)
+    if lin.bias is None:
+        raise ValueError("the Linear must have a bias")
     w, b = weight.detach(), bias.detach() if bias is not None else None
-    lw, lb = ln.weight.detach(), ln.bias.detach()
-    if w.dtype != x.dtype or lw.dtype != x.dtype or (b is not None and b.dtype != x.dtype):
+    lw, lb, db = ln.weight.detach(), ln.bias.detach(), lin.bias.detach()
+    if any(p is not None and p.dtype != x.dtype for p in (w, b, lw, lb, db)):
         raise TypeError("the LayerNorm and Linear parameters must have the activations' dtype")
-    if w.stride(-1) != 1 or w.shape[1] != K or tuple(lw.shape) != (K,):
+    if w.stride(-1) != 1 or w.shape[1] != K or tuple(lw.shape) != (K,) or tuple(db.shape) != (K,):
         raise ValueError("weight must be [N, K] with contiguous rows and K = x.shape[-1] = the LayerNorm's width")
+    if partials.dtype != torch.float32 or tuple(partials.shape[1:]) != (M, K) or not partials.is_contiguous():
+        raise ValueError("partials must be contiguous fp32 [n_split, rows, n] matching x")
     if b is not None and not b.is_contiguous():
         b = b.contiguous()
-    db, x_new = None, x
-    if partials is not None:
-        if partials.dtype != torch.float32 or tuple(partials.shape[1:]) != (M, K) or not partials.is_contiguous():
-            raise ValueError("partials must be contiguous fp32 [n_split, rows, n] matching x")
-        if lin is None or lin.bias is None:
-            raise ValueError("partials need the Linear they come from, with a bias")
-        db = lin.bias.detach()
-        if db.dtype != x.dtype:
-            raise TypeError("the LayerNorm and Linear parameters must have the activations' dtype")
-        x_new = torch.empty(x.shape, dtype=x.dtype, device=x.device)
     N = int(w.shape[0])
+    x_new = torch.empty(x.shape, dtype=x.dtype, device=x.device)
     y = torch.empty(M, N, dtype=x.dtype, device=x.device)
     rc = _lib.load().wdrz_ln_linear(
-        _LN16[x.dtype], xr.data_ptr(), xr.stride(0), partials.data_ptr() if partials is not None else None,
-        int(partials.shape[0]) if partials is not None else 0, db.data_ptr() if db is not None else None,
+        _LN16[x.dtype], xr.data_ptr(), xr.stride(0), partials.data_ptr(), int(partials.shape[0]), db.data_ptr(),
         x_new.data_ptr(), K, lw.data_ptr(), lb.data_ptr(), float(ln.eps), w.data_ptr(), w.stride(0),
         b.data_ptr() if b is not None else None, y.data_ptr(), N, M, N, K, 1 if gelu else 0, _stream_handle(),
     )
     if rc != _lib.WDRZ_OK:
         _raise(rc, "ln_linear")
     return x_new, y.view(*x.shape[:-1], N)
+
+
+def step_begin(tokens: torch.Tensor, positions: torch.Tensor, emb: torch.Tensor, pos_emb: torch.Tensor,
+               ln: nn.LayerNorm, slots: Optional[torch.Tensor], lens: torch.Tensor):
+    """A cached step's prologue in one launch: ``x = emb[tokens] + pos_emb[positions]``, ``ln(x)``,
+    the int32 slot map (None without ``slots``) and ``lens[:, slots]`` (``lens[:, :B]`` without).
+
+    ``tokens`` / ``positions`` int64 ``[B, sq]`` (any strides), 16-bit tables ``[n_vocab, n]`` /
+    ``[n_ctx, n]``, ``slots`` int64 ``[B]``, ``lens`` int32 ``[n_layers, n_slots]`` contiguous."""
+    for name, t in (("emb", emb), ("pos_emb", pos_emb), ("tokens", tokens), ("positions", positions), ("lens", lens)):
+        _check_cuda(name, t, emb.device)
+    if emb.dtype not in _LN16:
+        raise TypeError(f"emb: dtype {emb.dtype} is not supported (bfloat16, float16)")
+    B, sq = (int(v) for v in tokens.shape)
+    n = int(emb.shape[1])
+    e, p, lw, lb = emb.detach(), pos_emb.detach(), ln.weight.detach(), ln.bias.detach()
+    if any(t.dtype != e.dtype for t in (p, lw, lb)):
+        raise TypeError("the tables and the LayerNorm must share a dtype")
+    if tuple(positions.shape) != (B, sq) or p.shape[1] != n or tuple(lw.shape) != (n,) or e.stride(-1) != 1 \
+            or p.stride(-1) != 1 or not lens.is_contiguous():
+        raise ValueError("shapes or strides of the step's inputs do not match")
+    if tokens.dtype != torch.int64 or positions.dtype != torch.int64 or lens.dtype != torch.int32:
+        raise TypeError("tokens and positions must be int64, lens int32")
+    slots32 = None
+    if slots is not None:
+        _check_cuda("slots", slots, e.device)
+        if slots.dtype != torch.int64 or tuple(slots.shape) != (B,):
+            raise ValueError(f"slots must be int64 [{B}]")
+        slots = slots.contiguous()
+        slots32 = torch.empty(B, dtype=torch.int32, device=e.device)
+    elif B > lens.shape[1]:
+        raise ValueError(f"{B} rows exceed the {lens.shape[1]} slots")
+    x = torch.empty(B, sq, n, dtype=e.dtype, device=e.device)
+    h = torch.empty_like(x)
+    seqlens = torch.empty(lens.shape[0], B, dtype=torch.int32, device=e.device)
+    i64x2 = _lib.ctypes.c_int64 * 2
+    rc = _lib.load().wdrz_step_begin(
+        _LN16[e.dtype], tokens.data_ptr(), i64x2(*tokens.stride()), positions.data_ptr(), i64x2(*positions.stride()),
+        e.data_ptr(), e.stride(0), e.shape[0], p.data_ptr(), p.stride(0), p.shape[0], lw.data_ptr(), lb.data_ptr(),
+        float(ln.eps), x.data_ptr(), h.data_ptr(), slots.data_ptr() if slots is not None else None,
+        slots32.data_ptr() if slots is not None else None, lens.data_ptr(), seqlens.data_ptr(), B, sq, n,
+        lens.shape[0], lens.shape[1], _stream_handle(),
+    )
+    if rc != _lib.WDRZ_OK:
+        _raise(rc, "step_begin")
+    return x, h, slots32, seqlens
+
+
+def step_end_(lens: torch.Tensor, seqlens: torch.Tensor, slots: Optional[torch.Tensor], sq: int) -> None:
+    """``lens[:, slots] += sq`` (``lens[:, :B]`` without ``slots``) from the lengths ``seqlens`` that
+    ``step_begin`` gathered."""
+    slots = slots.contiguous() if slots is not None else None
+    rc = _lib.load().wdrz_step_end(lens.data_ptr(), seqlens.data_ptr(), slots.data_ptr() if slots is not None else None,
+                                   seqlens.shape[1], sq, lens.shape[0], lens.shape[1], _stream_handle())
+    if rc != _lib.WDRZ_OK:
+        _raise(rc, "step_end_")

@@ -13,8 +13,8 @@ cached attention, so the HIP kernels can be exercised exactly as WhisperDRZ driv
   ``seq_lens`` bump after all layers, final LN and tied-embedding logits (model.py:570-617,
   824-869).
 * ``TextDecoderStack._fused_blocks`` — the same blocks with each residual add fused into the
-  next LayerNorm (``decode_ops.add_layernorm_``), the step's metadata (int32 slot map, every
-  layer's gathered lengths) computed once per step, the self-attention query / key / value
+  next LayerNorm (``decode_ops.add_layernorm_``), the embeddings, the first LayerNorm and the step's
+  metadata (int32 slot map, every layer's gathered lengths) in one launch (``step_begin``), the self-attention query / key / value
   projections as one GEMM (``decode_ops.linear``), fc1 with its GELU as one kernel
   (``linear_gelu``), and the attention output projections and fc2 as split-K partials summed by
   the residual add (``linear_partials`` + ``add_layernorm_partials_``); the default for 16-bit
@@ -38,7 +38,7 @@ from torch import Tensor
 
 from .attention import flash_attn_with_kvcache, scaled_dot_product_attention
 from .decode_ops import (LN_LINEAR_MAX_K, LN_LINEAR_ROWS, add_layernorm_, add_layernorm_partials_, layer_norm, linear,
-                         linear_gelu, linear_partials, ln_linear)
+                         linear_gelu, linear_partials, ln_linear, step_begin, step_end_)
 from .kv_cache import FlashKVCache, KVSlotPool
 
 # Batch buckets of the captured decode step (reference transcriber.py:18).
@@ -227,15 +227,29 @@ class TextDecoderStack(nn.Module):
         B, seq_len = tokens.shape
         if positions.dim() == 1:
             positions = positions.unsqueeze(1).expand(B, seq_len)
+        lens = lengths_matrix(self_kv)
+        if lens is not None and self._fused_prologue(tokens, positions, slot_indices, lens):
+            x, h, batch_idx, seqlens = step_begin(tokens, positions, self.token_embedding.weight,
+                                                  self.positional_embedding, self.blocks[0].attn_ln, slot_indices, lens)
+            h = self._fused_blocks(x, h, self_kv, cross_kv, batch_idx, list(seqlens.unbind(0)))
+            # the attention never bumps lengths; the caller does, after all layers
+            step_end_(lens, seqlens, slot_indices, seq_len)
+            return h @ self.token_embedding.weight.to(h.dtype).T
         x = self.token_embedding(tokens) + self.positional_embedding[positions]
         if self.fused_small_ops and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16):
-            h = self._fused_blocks(x.contiguous(), self_kv, cross_kv, slot_indices)
+            x = x.contiguous()
+            # the step's metadata once, not per layer: the int32 slot map and every layer's gathered
+            # self lengths
+            batch_idx = None if slot_indices is None else slot_indices.to(torch.int32)
+            if lens is not None:  # one gather from the [n_layers, n_slots] lengths
+                layer_lens = list((lens[:, slot_indices] if slot_indices is not None else lens[:, :B]).contiguous())
+            else:
+                layer_lens = [s.seq_lens if slot_indices is None else s.seq_lens[slot_indices] for s in self_kv]
+            h = self._fused_blocks(x, layer_norm(x, self.blocks[0].attn_ln), self_kv, cross_kv, batch_idx, layer_lens)
         else:
             for block, s_kv, c_kv in zip(self.blocks, self_kv, cross_kv, strict=True):
                 x = block.forward_flash(x, s_kv, c_kv, slot_indices=slot_indices)
             h = self.ln(x)
-        # the attention never bumps lengths; the caller does, after all layers
-        lens = lengths_matrix(self_kv)
         if lens is not None:  # every layer's row at once, same indexing as per layer
             if slot_indices is not None:
                 lens[:, slot_indices] += seq_len
@@ -249,22 +263,30 @@ class TextDecoderStack(nn.Module):
                     s_kv.seq_lens[:B] += seq_len
         return h @ self.token_embedding.weight.to(h.dtype).T
 
-    def _fused_blocks(self, x: Tensor, self_kv: list[FlashKVCache], cross_kv: list[FlashKVCache],
-                      slot_indices: Optional[Tensor]) -> Tensor:
+    def _fused_prologue(self, tokens: Tensor, positions: Tensor, slot_indices: Optional[Tensor], lens: Tensor) -> bool:
+        """Whether ``step_begin`` / ``step_end_`` take this step: 16-bit, 16-byte aligned tables of up
+        to 2048 values on the GPU, int64 indices there, a plain embedding without hooks, at least one
+        row, rows within the slots."""
+        emb, pos, dev = self.token_embedding, self.positional_embedding, lens.device
+        w, ln = emb.weight, self.blocks[0].attn_ln
+        idx = [tokens, positions] + ([slot_indices] if slot_indices is not None else [])
+        return (self.fused_small_ops and w.is_cuda and w.dtype in (torch.bfloat16, torch.float16)
+                and all(t.device == dev for t in (w, pos, ln.weight, *idx)) and all(t.dtype == torch.int64 for t in idx)
+                and w.dtype == pos.dtype == ln.weight.dtype == ln.bias.dtype and w.shape[1] % 8 == 0
+                and w.shape[1] <= 2048 and w.is_contiguous() and pos.is_contiguous()
+                and w.data_ptr() % 16 == 0 and pos.data_ptr() % 16 == 0 and tokens.numel() > 0
+                and type(emb) is nn.Embedding and emb.max_norm is None
+                and not emb._forward_hooks and not emb._forward_pre_hooks
+                and tuple(positions.shape) == tuple(tokens.shape)
+                and (tokens.shape[0] <= lens.shape[1] if slot_indices is None
+                     else tuple(slot_indices.shape) == (tokens.shape[0],)))
+
+    def _fused_blocks(self, x: Tensor, h: Tensor, self_kv: list[FlashKVCache], cross_kv: list[FlashKVCache],
+                      batch_idx: Optional[Tensor], layer_lens: list[Tensor]) -> Tensor:
         """The blocks of ``forward_flash`` with each residual add fused into the next LayerNorm
-        (model.py:420-433): x is the residual stream, updated in place; returns ln(x)."""
+        (model.py:420-433): x is the residual stream, updated in place, h its first LayerNorm,
+        ``batch_idx`` the int32 slot map and ``layer_lens`` each layer's self lengths; returns ln(x)."""
         blocks = list(self.blocks)
-        # the step's metadata once, not per layer: the int32 slot map and every layer's gathered
-        # self lengths (one gather from the [n_layers, n_slots] lengths when the layers' lengths
-        # are its rows)
-        B = x.shape[0]
-        batch_idx = None if slot_indices is None else slot_indices.to(torch.int32)
-        lens = lengths_matrix(self_kv)
-        if lens is not None:
-            seqlens = (lens[:, slot_indices] if slot_indices is not None else lens[:, :B]).contiguous()
-            layer_lens = [seqlens[i] for i in range(len(blocks))]
-        else:
-            layer_lens = [s.seq_lens if slot_indices is None else s.seq_lens[slot_indices] for s in self_kv]
         # a small step: every add + LayerNorm inside the projection that follows it
         n = self.n_state
         if (x.numel() // n if n else 0) <= LN_LINEAR_ROWS and n % 256 == 0 and n <= LN_LINEAR_MAX_K and all(
@@ -272,16 +294,18 @@ class TextDecoderStack(nn.Module):
             part = lin = None
             for i, (block, s_kv, c_kv) in enumerate(zip(blocks, self_kv, cross_kv, strict=True)):
                 attn, cross, fc1, fc2 = block.attn, block.cross_attn, block.mlp[0], block.mlp[2]
-                x, qkv = ln_linear(x, block.attn_ln, *attn.qkv_weight(), partials=part, lin=lin)
+                if part is None:
+                    qkv = linear(h, *attn.qkv_weight())
+                else:
+                    x, qkv = ln_linear(x, part, lin, block.attn_ln, *attn.qkv_weight())
                 o = attn.attend_step(qkv, s_kv, False, layer_lens[i], batch_idx)
-                x, q = ln_linear(x, block.cross_attn_ln, cross.query.weight, cross.query.bias,
-                                 partials=linear_partials(o, attn.out, 2), lin=attn.out)
+                x, q = ln_linear(x, linear_partials(o, attn.out, 2), attn.out, block.cross_attn_ln,
+                                 cross.query.weight, cross.query.bias)
                 o = cross.attend_step(q, c_kv, True, None, batch_idx)
-                x, h = ln_linear(x, block.mlp_ln, fc1.weight, fc1.bias, gelu=True,
-                                 partials=linear_partials(o, cross.out, 2), lin=cross.out)
+                x, h = ln_linear(x, linear_partials(o, cross.out, 2), cross.out, block.mlp_ln, fc1.weight, fc1.bias,
+                                 gelu=True)
                 part, lin = linear_partials(h, fc2, 4), fc2
             return add_layernorm_partials_(x, part, lin, self.ln)
-        h = layer_norm(x, blocks[0].attn_ln)
         for i, (block, s_kv, c_kv) in enumerate(zip(blocks, self_kv, cross_kv, strict=True)):
             o = block.attn.forward_flash_step(h, s_kv, False, layer_lens[i], batch_idx, project_out=False)
             h = _out_add_layernorm(x, o, block.attn.out, block.cross_attn_ln)
@@ -372,8 +396,7 @@ class BucketedDecodeGraphs:
                                               slot_indices=slot_indices)
         self.hits[bucket] += 1
         st = self.static[bucket]
-        st["tokens"][:B].copy_(tokens)
-        st["positions"][:B].copy_(positions)
-        st["slots"][:B].copy_(slot_indices)
+        # one launch where the inputs are int64 on this device, else a copy each
+        torch._foreach_copy_([st["tokens"][:B], st["positions"][:B], st["slots"][:B]], [tokens, positions, slot_indices])
         self.graphs[bucket].replay()
         return st["logits"][:B]
