@@ -404,3 +404,39 @@ def test_default_scale_is_head_dim_power(cuda):
     d = scaled_dot_product_attention(qd, kd, vd, scale=0.125)
     torch.cuda.synchronize()
     assert torch.equal(a, b) and torch.equal(c, d)
+
+
+# (B, sq, H, Lmax): both sides of the 16-bit plan's lines: long rows split below 160 workgroups
+# (20 x 7 = 140 / 20 x 8 = 160), short ones never (1023 / 1024), eight wavefronts up to 256
+# workgroups (252 / 260), 16-row blocks up to 512 (500 / 520) or 16 queries, splits of 16-row blocks
+PLAN_SHAPES = [(7, 1, 20, 1500), (8, 1, 20, 1500), (1, 1, 1, 1023), (1, 1, 1, 1024), (2, 3, 2, 6200),
+               (63, 2, 4, 130), (65, 2, 4, 130), (1, 16, 4, 1024), (1, 17, 4, 1500), (1, 39, 2, 1500), (5, 9, 50, 70),
+               (5, 33, 35, 64), (5, 17, 50, 64), (5, 17, 52, 64), (13, 16, 40, 64), (2, 64, 64, 130), (3, 64, 64, 130)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("self_attn", [True, False])
+@pytest.mark.parametrize("B,sq,H,Lmax", PLAN_SHAPES)
+def test_plan_lines(cuda, dtype, self_attn, B, sq, H, Lmax):
+    """Every route of the 16-bit plan against the float64 oracle (the file's tolerance), caches bit
+    for bit, the workspace all zero afterwards and never asked to be larger than the size query."""
+    from whisperdrz_amd import flash_attn_with_kvcache, kvcache_workspace_size
+
+    if self_attn and sq > Lmax:
+        pytest.skip("the append would not fit")
+    kc, vc = make_cache(B + 1, Lmax, H, 64, dtype, "cpu", "head_major", 3)
+    q, k, v = (randn((B, sq, H, 64), s, dtype) for s in (5, 6, 7))
+    cs = np.random.default_rng(B + sq).integers(0, Lmax - sq + 1, B).astype(np.int32) if self_attn else None
+    if self_attn:
+        cs[0] = Lmax - sq
+    idx = np.random.default_rng(9).permutation(B + 1)[:B].astype(np.int32)
+    new = (to_np(k), to_np(v)) if self_attn else (None, None)
+    ref, kref, vref = kvcache_ref(to_np(q), to_np(kc), to_np(vc), *new, cs, idx, 0.125)
+    kd, vd = kc.to(cuda), vc.to(cuda)
+    ws = torch.zeros(max(256, kvcache_workspace_size(B, sq, H, 64, Lmax)), dtype=torch.uint8, device=cuda)
+    kw = dict(k=k.to(cuda), v=v.to(cuda), cache_seqlens=torch.from_numpy(cs).to(cuda)) if self_attn else {}
+    out = flash_attn_with_kvcache(q.to(cuda), kd, vd, cache_batch_idx=torch.from_numpy(idx).to(cuda),
+                                  softmax_scale=0.125, workspace=ws, **kw)
+    assert_close(out, ref, dtype, f"B={B} sq={sq} H={H} Lmax={Lmax} self={self_attn}")
+    assert np.array_equal(to_np(kd), kref) and np.array_equal(to_np(vd), vref)
+    assert not ws.any()

@@ -14,7 +14,7 @@
 //
 // Launch shape: one 4-wavefront workgroup per (batch row, query block of up to 8, head, key
 // split); its wavefront partials merge through LDS. Rows split their keys only when there are
-// too few rows to fill the chip; a row with several splits has each split publish an (m, l, o)
+// too few rows to keep the chip busy; a row with several splits has each split publish an (m, l, o)
 // partial to the caller's workspace, and the split that arrives last (a per-row atomic
 // counter) merges them, writes the output and resets the counter, all in the same launch.
 //
@@ -22,11 +22,12 @@
 // from the cache, so the in-place write (done by the split whose key range holds the row)
 // cannot race with any read in the same launch.
 //
-// Which kernel serves a call (launch_typed): 16-bit calls of 2-8 query rows run on
-// kv_mq_kernel (MFMA over the rows, below), 9-39 rows in its 16-row blocks when those alone fill
-// the chip, and 40 or more rows (a prompt's self or cross attention) on kv_prefill_kernel in
-// attn_dense.hip (256-query MFMA blocks); single rows, the remaining multi-row shapes and fp32
-// caches run on kv_attn_kernel.
+// Which kernel serves a call (kv_plan16): 16-bit calls of 2-8 query rows run on kv_mq_kernel (MFMA
+// over the rows, below), more rows in its 16-row blocks, or, when those fill the chip more than
+// twice, on kv_prefill_kernel in attn_dense.hip (256-query MFMA blocks); single rows and fp32 caches
+// run on kv_attn_kernel.
+#include <algorithm>
+
 #include "kv_dup.h"
 #include "wdrz_common.h"
 #include "wdrz_launch.h"
@@ -179,8 +180,25 @@ __device__ __forceinline__ void kv_finish(const KvArgs& a, int b, int t0, int nq
   __syncthreads();
   if (!sm_last) return;
   // The merging workgroup reads the partials with agent-scope atomic loads (coherent, issued
-  // only after the counter told it every partial had landed): first every (m, l) pair in
-  // parallel into LDS, then one o value per (split, query, dim).
+  // only after the counter told it every partial had landed): kMergeBatch splits' o values per
+  // (query, dim) into registers and every (m, l) pair into LDS, all in one trip to memory. (One
+  // load per split in turn, each waited for: 5 queries over 1500 rows, 12 splits, 18.0 us a launch
+  // against 10.9; one query 11.4 against 9.0.)
+  constexpr int kMergeBatch = 16;
+  constexpr int kItems = (SQ * kHeadDim + kThreads - 1) / kThreads;  // (query, dim) pairs per thread
+  float ov[kItems][kMergeBatch];
+  auto load_o = [&](int it, int sp0) __attribute__((always_inline)) {
+    const int idx = tid + it * kThreads, t = idx / kHeadDim, d = idx % kHeadDim;
+#pragma unroll
+    for (int u = 0; u < kMergeBatch; ++u) {
+      ov[it][u] = 0.f;
+      if (sp0 + u < n_split_b && t < nq)
+        ov[it][u] = __hip_atomic_load(part + ((sp0 + u) * sq_stride + t) * kPart + d, __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT);
+    }
+  };
+#pragma unroll
+  for (int it = 0; it < kItems; ++it) load_o(it, 0);
   __shared__ float sm_pm[kMaxMergeSplits * SQ], sm_pl[kMaxMergeSplits * SQ];
   for (int idx = tid; idx < n_split_b * nq; idx += kThreads) {
     const int sp = idx / nq, t = idx % nq;
@@ -191,17 +209,24 @@ __device__ __forceinline__ void kv_finish(const KvArgs& a, int b, int t0, int nq
     pp[kHeadDim + 1] = 0.f;
   }
   __syncthreads();
-  for (int idx = tid; idx < nq * kHeadDim; idx += kThreads) {
-    const int t = idx / kHeadDim, d = idx % kHeadDim;
+#pragma unroll
+  for (int it = 0; it < kItems; ++it) {
+    const int idx = tid + it * kThreads, t = idx / kHeadDim, d = idx % kHeadDim;
+    if (t >= nq) continue;
     float mm = kNegBig;
     for (int sp = 0; sp < n_split_b; ++sp) mm = fmaxf(mm, sm_pm[sp * SQ + t]);
     float L = 0.f, O = 0.f;
-    for (int sp = 0; sp < n_split_b; ++sp) {
-      const float f = fast_exp2(sm_pm[sp * SQ + t] - mm);
-      L = __builtin_fmaf(sm_pl[sp * SQ + t], f, L);
-      float* po = part + (sp * sq_stride + t) * kPart + d;
-      O = __builtin_fmaf(__hip_atomic_load(po, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), f, O);
-      *po = 0.f;
+    for (int sp0 = 0; sp0 < n_split_b; sp0 += kMergeBatch) {
+      if (sp0) load_o(it, sp0);
+#pragma unroll
+      for (int u = 0; u < kMergeBatch; ++u) {
+        if (sp0 + u < n_split_b) {
+          const float f = fast_exp2(sm_pm[(sp0 + u) * SQ + t] - mm);
+          L = __builtin_fmaf(sm_pl[(sp0 + u) * SQ + t], f, L);
+          O = __builtin_fmaf(ov[it][u], f, O);
+          part[((sp0 + u) * sq_stride + t) * kPart + d] = 0.f;
+        }
+      }
     }
     store_out(t, d, O / L);
   }
@@ -502,7 +527,7 @@ __global__ __launch_bounds__(kWavesPerWg * 64) void kv_attn_kernel(KvArgs a) {
 
 // ============================================================================================
 // Multi-query rows on the matrix core (16-bit types: 2 <= sq <= 8 in one block, the draft
-// verify; longer prefills in blocks of 16 rows when those blocks fill the chip, see the C layer).
+// verify; longer ones in blocks of 16 rows, see kv_plan16).
 // With several queries per row the VALU form above spends most of its time on the
 // per-query dot products, reductions and exps of every key; here a wavefront takes 32 keys
 // per step and computes
@@ -515,7 +540,7 @@ __global__ __launch_bounds__(kWavesPerWg * 64) void kv_attn_kernel(KvArgs a) {
 // 4*(l/16)..+3 of each 16-key block, i.e. keys {4g..4g+3, 16+4g..16+4g+3} for g = l/16, and the
 // V^T operand is read in that same key order. Query slots past the block's rows are computed and
 // discarded.
-// The four wavefronts of a workgroup take interleaved 32-key chunks of the row (or split);
+// The wavefronts of a workgroup take interleaved 32-key chunks of the row (or split);
 // their partials merge through LDS as in the VALU kernel.
 // ============================================================================================
 constexpr int kMqChunk = 32;                   // keys per wavefront step
@@ -557,14 +582,13 @@ __device__ __forceinline__ float group4_max(float x) {
   return fmaxf(__uint_as_float(r16[0]), __uint_as_float(r16[1]));
 }
 
-// SQ: query rows per workgroup, 8 (one block of sq <= 8 rows) or 16 (blocks of 16 rows of a
-// longer prefill; every MFMA query slot used).
-template <typename T, bool HAS_NEW, int SQ>
+// SQ: query rows per workgroup, 8 (one block of sq <= 8 rows) or 16 (blocks of 16 rows; every MFMA
+// query slot used). kWaves: 4, or 8 for launches of few workgroups (kv_plan16).
+template <typename T, bool HAS_NEW, int SQ, int kWaves>
 // At most 128 VGPRs (four wavefronts per SIMD): measured 5% faster for config 5 than the
 // unconstrained 148 (three per SIMD, the row's 1280 workgroups then need 1.7 rounds).
-__global__ __launch_bounds__(kWavesPerWg * 64, 4) void kv_mq_kernel(KvArgs a) {
+__global__ __launch_bounds__(kWaves * 64, 4) void kv_mq_kernel(KvArgs a) {
   typedef typename Mfma16<T>::op_t op_t;
-  constexpr int kWaves = kWavesPerWg;
   static_assert(SQ <= 16, "16 query slots per MFMA tile");
   __shared__ float sm_acc[kWaves][SQ][kHeadDim];
   __shared__ float sm_m[kWaves][SQ];
@@ -730,38 +754,45 @@ __global__ __launch_bounds__(kWavesPerWg * 64, 4) void kv_mq_kernel(KvArgs a) {
   kv_finish<T, SQ, kWaves>(a, b, t0, nq, a.n_qblocks > 1 ? SQ : nq, h, split, n_split_b, bad, sm_acc, sm_m, sm_l);
 }
 
+template <typename T, int SQ>
+void launch_row(const KvArgs& a, dim3 grid, hipStream_t stream) {
+  const dim3 block(kWavesPerWg * 64);
+  if (a.kn) hipLaunchKernelGGL((kv_attn_kernel<T, SQ, true>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((kv_attn_kernel<T, SQ, false>), grid, block, 0, stream, a);
+}
+template <typename T, int SQ, int W>
+void launch_mq(const KvArgs& a, dim3 grid, hipStream_t stream) {
+  if (a.kn) hipLaunchKernelGGL((kv_mq_kernel<T, true, SQ, W>), grid, dim3(W * 64), 0, stream, a);
+  else hipLaunchKernelGGL((kv_mq_kernel<T, false, SQ, W>), grid, dim3(W * 64), 0, stream, a);
+}
+
 template <typename T>
 hipError_t launch_typed(const KvArgs& a, hipStream_t stream) {
   const int64_t n_units = (int64_t)a.B * a.n_qblocks * a.H;
   if (n_units > 0x7fffffff) return hipErrorInvalidValue;
   dim3 grid((unsigned)n_units, 1, a.n_splits);
-  const bool has_new = a.kn != nullptr;
   const int sq_blk = a.n_qblocks > 1 ? kMaxSQ : a.sq;
   if constexpr (ElemBytes<T>::value == 2) {
-    // many queries (a prompt's self and cross attention): 256-query MFMA blocks (attn_dense.hip),
-    // each key row read ~sq/256 times instead of once per 16-query block
-    if (a.sq >= kPrefillMinSq) return launch_kv_prefill(__is_same(T, Bf16) ? 2 : 1, a, stream);
-    if (a.mq_rows == 16) {  // prefill in 16-row blocks on the matrix cores
-      if (has_new)
-        hipLaunchKernelGGL((kv_mq_kernel<T, true, 16>), grid, dim3(kWavesPerWg * 64), 0, stream, a);
-      else
-        hipLaunchKernelGGL((kv_mq_kernel<T, false, 16>), grid, dim3(kWavesPerWg * 64), 0, stream, a);
-      return hipGetLastError();
+    switch (a.route) {
+      case kKvPrefill:  // 256-query MFMA blocks (attn_dense.hip)
+        return launch_kv_prefill(__is_same(T, Bf16) ? 2 : 1, a, stream);
+      case kKvMq16:
+        if (a.waves == 8) launch_mq<T, 16, 8>(a, grid, stream);
+        else launch_mq<T, 16, kWavesPerWg>(a, grid, stream);
+        return hipGetLastError();
+      case kKvMq8:
+        if (a.waves == 8) launch_mq<T, kMaxSQ, 8>(a, grid, stream);
+        else launch_mq<T, kMaxSQ, kWavesPerWg>(a, grid, stream);
+        return hipGetLastError();
+      default:
+        if (a.sq != 1) return hipErrorInvalidValue;
+        launch_row<T, 1>(a, grid, stream);
+        return hipGetLastError();
     }
-    if (a.n_qblocks == 1 && sq_blk >= 2) {
-      if (has_new)
-        hipLaunchKernelGGL((kv_mq_kernel<T, true, kMaxSQ>), grid, dim3(kWavesPerWg * 64), 0, stream, a);
-      else
-        hipLaunchKernelGGL((kv_mq_kernel<T, false, kMaxSQ>), grid, dim3(kWavesPerWg * 64), 0, stream, a);
-      return hipGetLastError();
-    }
-  }
-#define WDRZ_KV_CASE(SQV)                                                                       \
-  case SQV:                                                                                     \
-    if (has_new)                                                                                \
-      hipLaunchKernelGGL((kv_attn_kernel<T, SQV, true>), grid, dim3(kWavesPerWg * 64), 0, stream, a); \
-    else                                                                                         \
-      hipLaunchKernelGGL((kv_attn_kernel<T, SQV, false>), grid, dim3(kWavesPerWg * 64), 0, stream, a); \
+  } else {
+#define WDRZ_KV_CASE(SQV)              \
+  case SQV:                            \
+    launch_row<T, SQV>(a, grid, stream); \
     break;
   switch (sq_blk) {
     WDRZ_KV_CASE(1)
@@ -776,17 +807,15 @@ hipError_t launch_typed(const KvArgs& a, hipStream_t stream) {
       return hipErrorInvalidValue;
   }
 #undef WDRZ_KV_CASE
-  return hipGetLastError();
+    return hipGetLastError();
+  }
 }
 
 }  // namespace
 
-void kv_split_plan(int64_t units, int64_t Lk, int* n_splits, int* split_len) {
-  // One workgroup per row walks all its keys when there are enough rows to fill the chip
-  // (splitting costs a partial round trip per split and, measured, never pays off then).
-  // Fewer rows split their keys so that >= 1024 workgroups (four per CU) are in flight.
-  const int64_t max_splits = (Lk + kMinSplitKeys - 1) / kMinSplitKeys;
-  int64_t want = (1024 + units - 1) / (units > 0 ? units : 1);
+// Splits of Lk keys so that about `want` workgroups share a row, each with at least min_keys.
+static void kv_split_keys(int64_t want, int64_t Lk, int64_t min_keys, int* n_splits, int* split_len) {
+  const int64_t max_splits = (Lk + min_keys - 1) / min_keys;
   if (want < 1) want = 1;
   if (want > max_splits) want = max_splits;
   if (want > kMaxMergeSplits) want = kMaxMergeSplits;
@@ -795,6 +824,62 @@ void kv_split_plan(int64_t units, int64_t Lk, int* n_splits, int* split_len) {
   *split_len = (int)len;
   *n_splits = (int)((Lk + len - 1) / len);
   if (*n_splits < 1) *n_splits = 1;
+}
+
+void kv_split_plan(int64_t units, int64_t Lk, int* n_splits, int* split_len) {
+  // fp32 rows (and what the workspace query allows for): up to eight queries per key on the VALU,
+  // so a row is compute-bound and its keys are split until >= 1024 workgroups (four per CU) are in
+  // flight. 5 fp32 queries over 1500 rows, 1 / 4 / 16 streams: unsplit 73 / 74 / 84 us, split for 160
+  // workgroups 17 / 43 / 84, for 1024 17 / 21 / 58.
+  kv_split_keys((1024 + units - 1) / (units > 0 ? units : 1), Lk, kMinSplitKeys, n_splits, split_len);
+}
+
+// 16-bit rows are bound by streaming their keys: one 4-wavefront workgroup walks 1500 of them in
+// ~7 us, and merging splits costs ~3 us (publish, count, read back: three trips to the coherence
+// point), so splits pay only for long rows that leave most CUs without a workgroup. Measured
+// (20 heads, per launch; splits for >= 1024 workgroups, as before -> this): self over <= 400 of 448
+// rows, one query 1 / 8 / 16 / 48 streams 7.6 / 7.9 / 10.7 / 16.8 -> 5.6 / 6.6 / 8.7 / 13.3 us; cross over 1500, 5
+// queries 10.9 / 19.5 / 30.0 / 72.3 -> 8.9 / 16.4 / 29.4 / 63.0. At 6 streams (120 workgroups)
+// unsplit 13.4 us, two splits 13.0; at 8 (160) unsplit 14.9, three splits 15.6.
+constexpr int64_t kSplitUnits = 160;      // workgroups below which long rows are split
+constexpr int64_t kSplitMinLk = 1024;     // rows shorter than this are never split
+constexpr int64_t kSplitMinKeys = 192;
+// Eight wavefronts a workgroup instead of four while the launch has no more workgroups than CUs:
+// 5 queries, self, 1 / 12 streams 6.7 / 8.3 -> 5.9 / 7.7 us; at 24 and 48 streams 10.4 and 15.4 ->
+// 10.2 and 17.6 (a second round of workgroups no longer fits beside the first).
+constexpr int64_t kWideWgs = 256;
+// Blocks of 16 queries re-read the row's keys once per block, 256-query blocks stage them once but
+// leave a small launch few workgroups. Cross over 1500 rows, 16-query blocks / 256-query blocks:
+// 224 queries x 2 streams (560 workgroups) 34.8 / 40.0 us, 112 x 4 (560) 37.1 / 34.4, 64 x 6 (480)
+// 29.2 / 34.2, 64 x 8 (640) 41.1 / 34.6.
+// Below kPrefillMinSq queries the second and third block of a row are the question: cross, 17 / 33
+// queries x 32 streams 82 / 111 us in blocks of 16, 67 / 69 in 256-query blocks; 16 queries (one
+// block) 45 / 69. Self rows are short (their 256-query kernel also appends): 39 queries x 32 streams
+// 29.8 / 30.
+constexpr int64_t kMq16Wgs = 512;
+constexpr int kCrossMqMaxSq = 16;
+
+void kv_plan16(KvArgs* a) {
+  const int64_t B = a->B, H = a->H;
+  const int64_t blocks16 = B * ((a->sq + 15) / 16) * H;
+  a->n_qblocks = 1;
+  a->n_splits = 1;
+  a->split_len = a->Lk;
+  if (a->sq > 8) {
+    a->n_qblocks = (a->sq + 15) / 16;
+    const bool many = a->sq >= kPrefillMinSq || (a->kn == nullptr && a->sq > kCrossMqMaxSq);
+    a->route = blocks16 > kMq16Wgs && many ? kKvPrefill : kKvMq16;
+  } else {
+    a->route = a->sq > 1 ? kKvMq8 : kKvRow;
+  }
+  const int64_t units = B * a->n_qblocks * H;
+  // kPrefillMinSq or more queries: the workspace query promises that none is needed
+  if (a->route != kKvPrefill && a->sq < kPrefillMinSq && units < kSplitUnits && a->Lk >= kSplitMinLk) {
+    // blocks of 16 rows: at most half as many, so that they fit the workspace of 8-row blocks
+    kv_split_keys(std::min<int64_t>((kSplitUnits + units - 1) / units, kMaxMergeSplits / (a->sq > 8 ? 2 : 1)), a->Lk,
+                  kSplitMinKeys, &a->n_splits, &a->split_len);
+  }
+  a->waves = units * a->n_splits <= kWideWgs ? 8 : kWavesPerWg;
 }
 
 size_t kv_workspace_bytes(int64_t units, int64_t sq_blk, int n_splits) {

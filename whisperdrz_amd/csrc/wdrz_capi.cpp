@@ -230,8 +230,8 @@ int wdrz_attn_fwd(int dtype, const void* q, const void* k, const void* v, void* 
 size_t wdrz_attn_kvcache_workspace_size(int64_t B, int64_t sq, int64_t H, int64_t D, int64_t Lmax) {
   (void)D;
   if (B <= 0 || sq <= 0 || H <= 0 || Lmax <= 0) return 0;
-  // kPrefillMinSq or more query rows never split their keys (16-bit types run them on the
-  // 256-query prefill kernel, fp32 on one workgroup per 8-row block): no workspace
+  // kPrefillMinSq or more query rows never split their keys: no workspace. Fewer: what fp32 needs,
+  // which covers the 16-bit plan (fewer splits).
   if (sq >= wdrz::kPrefillMinSq) return 0;
   const int64_t n_qblocks = (sq + 7) / 8;
   const int64_t units = B * n_qblocks * H;
@@ -294,12 +294,6 @@ int wdrz_attn_kvcache(int dtype, const void* q, void* k_cache, void* v_cache, co
   a.H = (int)H;
   a.Lk = (int)Lmax;
   a.n_slots = (int)n_slots;
-  // Prefill (sq > 8) in 16-bit types runs on the multi-query MFMA kernel in 16-row blocks when
-  // those blocks fill the chip on their own (so the launch never splits its keys and needs no
-  // workspace); otherwise in blocks of 8 rows, as the workspace size query assumes.
-  const bool mq16 = eb == 2 && sq > 8 && B * ((sq + 15) / 16) * H >= 1024;
-  a.n_qblocks = (int)(mq16 ? (sq + 15) / 16 : (sq + 7) / 8);
-  a.mq_rows = mq16 ? 16 : 0;
   const int64_t* S[4] = {q_strides, kc_strides, vc_strides, o_strides};
   int64_t* Dst[4] = {a.qs, a.kcs, a.vcs, a.os};
   for (int i = 0; i < 4; ++i)
@@ -310,15 +304,25 @@ int wdrz_attn_kvcache(int dtype, const void* q, void* k_cache, void* v_cache, co
       a.vns[j] = vn_strides[j] * eb;
     }
   a.c = softmax_scale * 1.4426950408889634f;
-  const int64_t units = B * a.n_qblocks * H;
-  if (units > 0x7fffffff) return fail(WDRZ_EUNSUPPORTED, "B * ceil(sq / rows per block) * H exceeds 2^31 - 1");
-  if (sq >= wdrz::kPrefillMinSq) {  // never split (see wdrz_attn_kvcache_workspace_size)
-    a.n_splits = 1;
-    a.split_len = (int)Lmax;
-  } else {
-    wdrz::kv_split_plan(units, Lmax, &a.n_splits, &a.split_len);
+  int64_t units;
+  if (eb == 2) {
+    wdrz::kv_plan16(&a);
+    units = B * a.n_qblocks * H;
+  } else {  // blocks of 8 rows
+    a.n_qblocks = (int)((sq + 7) / 8);
+    units = B * a.n_qblocks * H;
   }
-  const size_t need = wdrz::kv_workspace_bytes(units, sq < 8 ? sq : 8, a.n_splits);
+  if (units > 0x7fffffff) return fail(WDRZ_EUNSUPPORTED, "B * ceil(sq / rows per block) * H exceeds 2^31 - 1");
+  if (eb != 2) {
+    if (sq >= wdrz::kPrefillMinSq) {  // never split (see wdrz_attn_kvcache_workspace_size)
+      a.n_splits = 1;
+      a.split_len = (int)Lmax;
+    } else {
+      wdrz::kv_split_plan(units, Lmax, &a.n_splits, &a.split_len);
+    }
+  }
+  const int block = eb == 2 && sq > 8 ? 16 : 8;
+  const size_t need = wdrz::kv_workspace_bytes(units, sq < block ? sq : block, a.n_splits);
   if (need > 0) {
     if (!workspace || workspace_bytes < need)
       return fail(WDRZ_EWORKSPACE, "workspace of %zu bytes required (got %zu)", need, workspace ? workspace_bytes : 0);

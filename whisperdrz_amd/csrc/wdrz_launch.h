@@ -23,12 +23,20 @@ struct KvArgs {
   float* ws_part;  // split partials (split mode with n_splits > 1)
   int* ws_count;   // per-row arrival counters, zero between calls
   int B, sq, H, Lk, n_slots, n_qblocks, n_splits, split_len;
-  int mq_rows;  // 16: query blocks of 16 rows on the multi-query MFMA kernel; 0: blocks of 8 (or one block)
+  int route;  // 16-bit: KvRoute (kv_plan16)
+  int waves;  // 16-bit: wavefronts per workgroup of the multi-query kernel
   int64_t qs[3], kcs[3], vcs[3], kns[3], vns[3], os[3];
   float c;  // softmax scale * log2(e)
 };
 
-// Split count and keys per split for `units` = B*n_qblocks*H rows over Lk keys.
+// Kernel of a 16-bit call: one query row per workgroup, 2-8 or blocks of 16 on the multi-query MFMA
+// kernel, or 256-query blocks.
+enum KvRoute { kKvRow, kKvMq8, kKvMq16, kKvPrefill };
+constexpr int kPrefillMinSq = 40;  // queries from which no call splits its keys (no workspace)
+// Sets route, n_qblocks, n_splits, split_len and waves of a 16-bit call from its sizes. Its
+// workspace is never larger than kv_split_plan's for blocks of 8 rows.
+void kv_plan16(KvArgs* a);
+// Split count and keys per split for `units` = B*n_qblocks*H rows over Lk keys (fp32).
 // Depends only on sizes, so the workspace size can be queried without data.
 void kv_split_plan(int64_t units, int64_t Lk, int* n_splits, int* split_len);
 // Workspace when n_splits > 1: per-row int32 counters (zero between calls), then partials.
@@ -38,10 +46,9 @@ void kv_workspace_layout(void* ws, int64_t units, KvArgs* a);
 // Launch the attention kernel: one workgroup per (row, key split); with n_splits > 1 the
 // partials merge in-launch through the workspace. dtype: 0 f32, 1 f16, 2 bf16.
 hipError_t launch_kv_attn(int dtype, const KvArgs& a, hipStream_t stream);
-// Many-query cached attention (16-bit, sq >= kPrefillMinSq): 256-query MFMA blocks. Self (new
+// Many-query cached attention (16-bit, route kKvPrefill): 256-query MFMA blocks. Self (new
 // rows given): causal, keys below cache_seqlens from the slot and the rest from k_new / v_new, the
 // new rows appended. Cross (no new rows): all Lk cache rows, nothing appended.
-constexpr int kPrefillMinSq = 40;
 hipError_t launch_kv_prefill(int dtype, const KvArgs& a, hipStream_t stream);
 
 // Dense MFMA attention (bf16 / fp16). Strides in ELEMENTS in [B, H, L, D] order.
