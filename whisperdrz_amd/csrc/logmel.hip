@@ -22,10 +22,12 @@
 // Why an FFT: the direct transform on the fp32 matrix cores (a [32 x 400] x [400 x 512] product
 // per 32 frames, the form before this one) took 240 us for 16 windows of 30 s and 50 us for one,
 // after an init launch that rebuilt its tables (3.3 us); the 55 MB this must move take 11 us. Now
-// 63 us for 16 windows and 14.5 us for one (a whole call 237 -> 76 and 53.6 -> 17 us), and nearer
-// to 64-bit results (3.7e-7 against 4.9e-7). What bounds it is the sum of VALU and LDS issue per
-// wavefront (the phases of a workgroup's wavefronts coincide): without the transforms' arithmetic
-// 60 us, without the filterbank's loop 51 us, without building the filter weights 60 us.
+// 60 us for 16 windows and 14 us for one (a whole call 237 -> 72 and 53.6 -> 16.5 us), and nearer
+// to 64-bit results (3.6e-7 against 5.3e-7). What bounds it: half of a wavefront's cycles are VALU
+// issue (~1700 instructions per 6 frames, a third of them the filterbank and log10), half waits
+// for samples, LDS and the other wavefronts of its phase; no part's removal takes more than a sixth
+// (transforms' arithmetic 3 us, filterbank loop 12, filter weights 3, stores 4 of the call's 76 us
+// when it was measured).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -68,6 +70,9 @@ constexpr int kWeights = ((2 * kBins + 6 * kMaxMels) / 4 + 4) * 4;
 constexpr int kMaxParts = 128;  // workgroups a window (= maxima in the workspace)
 static_assert(kSeg + kHopPad * (kSeg / kHop) + 1 <= kWaves * kWaveFloats, "sample buffer");
 static_assert(32 + 4 * kWaveFrames * kPGroups <= kWaveFloats, "power tile");
+
+// Three workgroups a CU need at most 42 of the 128 units of 1280 bytes that LDS is given out in.
+static_assert(4 * (kWaves * kWaveFloats + kWeights + kMaxMels) <= 42 * 1280, "three workgroups a CU");
 
 // ---- tables, computed at compile time in double -------------------------------------------------
 constexpr double kPi = 3.14159265358979323846;
@@ -187,6 +192,14 @@ __device__ __forceinline__ double mel_edge(int j, int n_mels) {
   return m < 15.0 ? f_sp * m : 1000.0 * exp(logstep * (m - 15.0));
 }
 
+// log10 of a normal number: log2 (one instruction, no denormals to scale) times log10(2) in two parts.
+__device__ __forceinline__ float log10_normal(float x) {
+  constexpr float hi = 0.30102999f, lo = (float)(0.30102999566398119521 - (double)hi);
+  const float y = __builtin_amdgcn_logf(x);
+  const float r = y * hi;
+  return r + __builtin_fmaf(y, lo, __builtin_fmaf(y, hi, -r));
+}
+
 // LDS ops of one wavefront run in order: between its own writes and reads only the compiler has to
 // be kept from moving them.
 __device__ __forceinline__ void wave_fence() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront"); }
@@ -197,9 +210,10 @@ __global__ __launch_bounds__(kThreads) void logmel_spec_kernel(LogMelArgs a) {
 
   __shared__ __align__(16) float buf[kWaves * kWaveFloats];  // samples, then transforms and powers
   __shared__ __align__(16) float wts[kWeights];
-  __shared__ uint8_t start[kMaxMels + 2];  // first bin at or above each edge
-  __shared__ float wmax[kWaves];
-  double* edges = reinterpret_cast<double*>(buf);  // until the first samples are stored
+  __shared__ uint32_t filt[kMaxMels];      // first power group, groups << 8, first weight << 16
+  // until the first samples are stored: the edges, and the first bin at or above each
+  double* edges = reinterpret_cast<double*>(buf);
+  uint8_t* start = reinterpret_cast<uint8_t*>(edges + kMaxMels + 2);
   auto wt_base = [&](int m) { return (start[m] + start[m + 1] + 6 * m) / 4 * 4; };
 
   const float* x = a.audio + (int64_t)b * a.audio_stride;
@@ -250,6 +264,10 @@ __global__ __launch_bounds__(kThreads) void logmel_spec_kernel(LogMelArgs a) {
           wts[wt_base(lo) + k - (start[lo] & ~3)] = (float)((down > 0.0 ? down : 0.0) * 2.0 / (edges[lo + 2] - e0));
         if (lo > 0)
           wts[wt_base(lo - 1) + k - (start[lo - 1] & ~3)] = (float)((up > 0.0 ? up : 0.0) * 2.0 / (e1 - edges[lo - 1]));
+      }
+      for (int m = tid; m < a.n_mels; m += kThreads) {
+        const int g0 = start[m] >> 2, g1 = (start[m + 2] + 3) >> 2;
+        filt[m] = (uint32_t)g0 | (uint32_t)(g1 - g0) << 8 | (uint32_t)wt_base(m) << 16;
       }
       __syncthreads();  // the samples take the edges' place
     }
@@ -341,20 +359,25 @@ __global__ __launch_bounds__(kThreads) void logmel_spec_kernel(LogMelArgs a) {
     {
       const int fr = min(lane & 31, kFrames - 1), f = f0 + fr;
       const float* P = buf + power_pos(fr / kWaveFrames, fr % kWaveFrames, 0);
-      for (int p = wave; 2 * p < a.n_mels; p += kWaves) {
-        const int mel = 2 * p + (lane >> 5), melc = min(mel, a.n_mels - 1);
-        const int g0 = start[melc] >> 2, g1 = (start[melc + 2] + 3) >> 2;
-        const float* w = wts + wt_base(melc);
+      const bool mine = (lane & 31) < kFrames && f < a.n_frames;  // frames past the last: no maximum
+      int mel = 2 * wave + (lane >> 5);
+      float* out = a.out + (int64_t)b * a.os[0] + (int64_t)mel * a.os[1] + f;
+      const int64_t step = 2 * kWaves * a.os[1];
+      for (; mel < a.n_mels; mel += 2 * kWaves, out += step) {
+        const uint32_t d = filt[mel];
+        const float* p = P + 4 * kWaveFrames * (d & 0xff);
+        const float* w = wts + (d >> 16);
+        const float* end = w + 4 * ((d >> 8) & 0xff);
         float acc = 0.f;
-        for (int g = g0; g < g1; ++g) {  // weights of the bins outside the filter are zero
-          const f32x4 pv = *reinterpret_cast<const f32x4*>(P + 4 * kWaveFrames * g);
-          const f32x4 wv = *reinterpret_cast<const f32x4*>(w + 4 * (g - g0));
+        for (; w != end; w += 4, p += 4 * kWaveFrames) {  // weights of the bins outside the filter are zero
+          const f32x4 pv = *reinterpret_cast<const f32x4*>(p);
+          const f32x4 wv = *reinterpret_cast<const f32x4*>(w);
           acc += (pv[0] * wv[0] + pv[1] * wv[1]) + (pv[2] * wv[2] + pv[3] * wv[3]);
         }
-        const float lv = log10f(fmaxf(acc, 1e-10f));
-        if (mel < a.n_mels && f < a.n_frames && (lane & 31) < kFrames) {
+        const float lv = log10_normal(fmaxf(acc, 1e-10f));
+        if (mine) {
           vmax = fmaxf(vmax, lv);
-          if (f < a.out_frames) a.out[(int64_t)b * a.os[0] + (int64_t)mel * a.os[1] + f] = lv;
+          if (f < a.out_frames) *out = lv;
         }
       }
     }
@@ -364,11 +387,11 @@ __global__ __launch_bounds__(kThreads) void logmel_spec_kernel(LogMelArgs a) {
   const int tid = threadIdx.x;
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, o));
-  if ((tid & 63) == 0) wmax[tid >> 6] = vmax;
+  if ((tid & 63) == 0) buf[tid >> 6] = vmax;
   __syncthreads();
   if (tid == 0) {
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w) vmax = fmaxf(vmax, wmax[w]);
+    for (int w = 1; w < kWaves; ++w) vmax = fmaxf(vmax, buf[w]);
     a.part_max[(int64_t)b * kMaxParts + blockIdx.x] = vmax;
   }
 }
