@@ -300,3 +300,51 @@ def test_pipe_kernel_large_scores(cuda, case, Lq, causal):
         assert torch.isfinite(out[b]).all()
         err = (out[b].double() - ref).abs().max().item()
         assert err <= 3e-2, f"b={b}: max|diff|={err:.3e}"
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("L", [40, 200])
+def test_fp32_split_range_and_nonfinite(cuda, causal, L):
+    """fp32 operands far from 1 (the three-way split is exact at any scale), and infinities and NaN,
+    which do not survive the split: the workgroup's queries then run on the fp32 matrix cores. Against
+    64 bits within the file's fp32 tolerance (1e-5 of the largest value)."""
+    from whisperdrz_amd import scaled_dot_product_attention
+
+    B, H = 1, 2
+    q, k, v = (randn((B, H, L, 64), s, torch.float32) for s in (21, 22, 23))
+
+    def ref(q, k, v):
+        s = (q.double() @ k.double().transpose(-1, -2)) * 0.125
+        if causal:
+            s = s.masked_fill(torch.ones(L, L, dtype=torch.bool).triu(1), float("-inf"))
+        return torch.softmax(s, -1) @ v.double()
+
+    def run(q, k, v):
+        return scaled_dot_product_attention(q.to(cuda), k.to(cuda), v.to(cuda), is_causal=causal, scale=0.125).cpu()
+
+    for qs, ks, vs in ((1e-15, 1e15, 1e30), (3e18, 1e-18, 1e-30)):
+        want = ref(q * qs, k * ks, v * vs)
+        err = (run(q * qs, k * ks, v * vs).double() - want).abs().max() / want.abs().max()
+        assert err <= 1e-5, (qs, ks, vs, float(err))
+    # one query row of infinities: NaN there, every other row as it was
+    q2 = q.clone()
+    q2[0, 0, 3] = float("inf")
+    got, want = run(q2, k, v), ref(q, k, v)
+    assert got[0, 0, 3].isnan().all()
+    keep = torch.ones(B, H, L, dtype=torch.bool)
+    keep[0, 0, 3] = False
+    assert (got.double() - want)[keep].abs().max() <= 1e-5 * want.abs().max()
+    # an infinite value: infinite where the key is seen, and only in that column
+    v2 = v.clone()
+    v2[0, 1, 5, 7] = float("inf")
+    got = run(q, k, v2)
+    seen = torch.arange(L) >= 5 if causal else torch.ones(L, dtype=torch.bool)
+    assert (got[0, 1, seen, 7] == float("inf")).all()
+    other = torch.arange(64) != 7
+    assert (got[0, 1][:, other].double() - want[0, 1][:, other]).abs().max() <= 1e-5 * want.abs().max()
+    # a NaN key: every query that sees it
+    k2 = k.clone()
+    k2[0, 0, L - 1, 0] = float("nan")
+    got = run(q, k2, v)
+    rows = slice(L - 1, L) if causal else slice(0, L)
+    assert got[0, 0, rows].isnan().all() and torch.isfinite(got[0, 1]).all()
