@@ -13,9 +13,9 @@
 //                        reflect padding; each wavefront runs its frames' real 400-point
 //                        transforms as complex 200-point ones (even samples + i odd samples) in
 //                        registers and LDS, the powers go to LDS, and the filterbank is applied
-//                        as the two weights each bin has; log10 is stored, and the workgroup's
+//                        as the two weights each bin has; (log10 + 4) / 4 is stored, and the workgroup's
 //                        maximum of its window goes to the workspace.
-//   logmel_finish_kernel (max(x, max - 8) + 4) / 4, and -1.5 past the last frame.
+//   logmel_finish_kernel raises what lies below max - 8, and writes -1.5 past the last frame.
 // fp32 throughout, like the reference; window, twiddles and filterbank are computed in double and
 // rounded once.
 //
@@ -377,7 +377,7 @@ __global__ __launch_bounds__(kThreads) void logmel_spec_kernel(LogMelArgs a) {
         const float lv = log10_normal(fmaxf(acc, 1e-10f));
         if (mine) {
           vmax = fmaxf(vmax, lv);
-          if (f < a.out_frames) *out = lv;
+          if (f < a.out_frames) *out = (lv + 4.0f) / 4.0f;
         }
       }
     }
@@ -396,8 +396,11 @@ __global__ __launch_bounds__(kThreads) void logmel_spec_kernel(LogMelArgs a) {
   }
 }
 
-// One row (window, mel) piece of 256 VEC frames per workgroup. VEC 4: 16-byte accesses, for rows
-// that start 16-byte aligned and hold whole groups of four.
+// One row (window, mel) piece of 256 VEC frames per workgroup. The rows hold (x + 4) / 4 already;
+// rounding keeps the order, so max(x, max - 8) scaled is the larger of the two scaled values, and
+// only frames below that floor (and the padding) are written. VEC 4: 16-byte accesses, for rows that
+// start 16-byte aligned and hold whole groups of four. Reading and writing every frame took 10.4 us
+// of 16 windows' call, this 8.6.
 template <int VEC>
 __global__ __launch_bounds__(256) void logmel_finish_kernel(LogMelArgs a) {
   const int b = blockIdx.z, m = blockIdx.y;
@@ -412,11 +415,15 @@ __global__ __launch_bounds__(256) void logmel_finish_kernel(LogMelArgs a) {
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, o));
   if (f >= a.out_frames) return;
-  const float floor_v = vmax - 8.0f;
+  const float floor_v = (vmax - 8.0f + 4.0f) / 4.0f;
+  bool write = false;
 #pragma unroll
-  for (int i = 0; i < VEC; ++i)
-    v[i] = f + i < a.n_frames ? (fmaxf(v[i], floor_v) + 4.0f) / 4.0f : -1.5f;  // audio.py:133-137
-  __builtin_memcpy(p, v, sizeof(v));
+  for (int i = 0; i < VEC; ++i) {
+    const float old = v[i];
+    v[i] = f + i < a.n_frames ? fmaxf(old, floor_v) : -1.5f;  // audio.py:133-137
+    write = write || f + i >= a.n_frames || old < floor_v;
+  }
+  if (write) __builtin_memcpy(p, v, sizeof(v));
 }
 
 }  // namespace
