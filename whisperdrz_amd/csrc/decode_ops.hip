@@ -29,7 +29,7 @@ namespace {
 template <typename T, int NC, int NP>
 __global__ __launch_bounds__(256) void add_layernorm_kernel(AddLnArgs a) {
   const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (row >= a.rows) return;
   char* xrow = static_cast<char*>(a.x) + row * a.x_stride * 2;
   char* yrow = static_cast<char*>(a.y) + row * a.y_stride * 2;
@@ -200,16 +200,21 @@ __global__ __launch_bounds__(kArgmaxThreads) void masked_argmax_kernel(ArgmaxArg
 
 }  // namespace
 
+// One row per workgroup up to here: a workgroup's rows are fetched by one CU, and four of them (18 KB
+// each with four partials) take longer than one. 52 rows of 1280 behind 2 / 4 partials 3.59 / 3.96 ->
+// 3.17 / 3.44 us, 1024 rows 5.64 / 7.01 -> 5.22 / 6.90, 2048 rows 7.8 / 10.8 either way.
+constexpr int64_t kLnSpreadRows = 1024;
 hipError_t launch_add_layernorm(int dtype, const AddLnArgs& a, hipStream_t stream) {
   if (a.rows == 0) return hipSuccess;
-  const dim3 grid((unsigned)((a.rows + 3) / 4));
+  const unsigned per_wg = a.rows <= kLnSpreadRows ? 1 : 4;
+  const dim3 grid((unsigned)((a.rows + per_wg - 1) / per_wg)), block(64 * per_wg);
   const int nc = (a.n + 511) / 512;
   const int np = a.dpart ? a.n_part : 0;
   // the partials form keeps 2 NP fp32 quads per chunk in registers: n <= 1536 (NC <= 3)
   if ((np != 0 && np != 2 && np != 4) || (np != 0 && nc > 3)) return hipErrorInvalidValue;
 #define WDRZ_LN3(NC, NP)                                                                                 \
-  if (dtype == 2) hipLaunchKernelGGL((add_layernorm_kernel<Bf16, NC, NP>), grid, dim3(256), 0, stream, a); \
-  else hipLaunchKernelGGL((add_layernorm_kernel<F16, NC, NP>), grid, dim3(256), 0, stream, a);
+  if (dtype == 2) hipLaunchKernelGGL((add_layernorm_kernel<Bf16, NC, NP>), grid, block, 0, stream, a); \
+  else hipLaunchKernelGGL((add_layernorm_kernel<F16, NC, NP>), grid, block, 0, stream, a);
 #define WDRZ_LNP(NC)     \
   case NC:               \
     if (np == 0) {       \
