@@ -11,8 +11,8 @@
 // accumulated in fp32; what is left out (x1 y2, x2 y1, x2 y2) is below 2^-25 of |x y|, less than one
 // fp32 rounding. 48 v_mfma_f32_32x32x16_bf16 of 32 cycles then do the work of 64
 // v_mfma_f32_32x32x2_f32 of 64 cycles per 32 x 32 step, and, unlike beside those, the softmax's VALU
-// instructions issue meanwhile. Measured, one encoder layer (B=1 H=20 L=1500): 110.6 -> 71.7
-// us, B=16 1641 -> 1112; causal 448 x 448, B=16: 176 -> 112; error against 64 bits 5.3e-7 -> 4.5e-7. Bound now: the MFMAs (24 for S^T, 24 for O^T, in
+// instructions issue meanwhile. Measured, one encoder layer (B=1 H=20 L=1500): 110.6 -> 70.4
+// us, B=16 1641 -> 1081; causal 448 x 448, B=16: 176 -> 109; error against 64 bits 5.3e-7 -> 4.5e-7. Bound now: the MFMAs (24 for S^T, 24 for O^T, in
 // two wavefronts per SIMD) and the split of K, V and P on the VALU (11 instructions a pair).
 // Infinities and NaN do not survive the split (inf - inf): they give NaN output, and a workgroup
 // that computed one repeats its queries on the fp32 matrix cores (f32_tile), whose result stands.
@@ -436,12 +436,21 @@ __device__ __forceinline__ bool split_tile(const DenseArgs& a, SplitStage* stage
   f32x16 s_cur, s_nxt;
   if (live(0)) scores(0, s_cur);
   auto unit = [&](int u, f32x16& cur, f32x16& nxt) __attribute__((always_inline)) {
+    // The two wavefronts of a SIMD split and store their share of stage u + 2 at opposite ends of the
+    // stage, so that one's VALU work runs beside the other's MFMAs (with the priority below, 74.3 ->
+    // 70.4 us a layer). The buffer last held stage u - 1, whose reads came before the last barrier.
+    if (kh == 1 && u + 2 < n_units) {
+      lstore((u + 2) % 3);
+      if (u + 3 < n_units) gload(u + 3);
+    }
     if (live(u)) {
+      __builtin_amdgcn_s_setprio(1);
       if (u + 1 < n_units && live(u + 1)) scores((u + 1) % 3, nxt);
+      __builtin_amdgcn_s_setprio(0);
       f32_softmax<CAUSAL>(a, p, 2 * u + kh, cur, m_run, l_run, acc_o);
       pv(u % 3, cur);
     }
-    if (u + 2 < n_units) {
+    if (kh == 0 && u + 2 < n_units) {
       lstore((u + 2) % 3);
       if (u + 3 < n_units) gload(u + 3);
     }
