@@ -299,6 +299,20 @@ def test_attention_prep_fused_heads_and_edges(cuda, heads, B, T, A, lens, caps, 
     _check_fused(got, ref, what)
 
 
+@pytest.mark.parametrize("B,n_heads_sel,T", [(13, 20, 70), (9, 30, 33), (1, 1, 448), (2, 20, 129)])
+def test_attention_prep_fused_chunks(cuda, B, n_heads_sel, T):
+    """Chunkings of the text rows by launch size: one chunk of all rows (13 x 20 and 9 x 30 heads),
+    single-block chunks (1 x 1), chunks of several blocks with a part block and rows past the lengths."""
+    from whisperdrz_amd import dtw_attention_prep
+
+    A, n_layers, n_heads = 96, 2, 20
+    q_out, k_out = _captures(B, T, A, n_layers, n_heads, torch.bfloat16, seed=B + n_heads_sel + T)
+    head_mask = _mask(n_layers, n_heads, [(i // n_heads, i % n_heads) for i in range(n_heads_sel)])
+    lens, caps = [T - (b * 5) % T for b in range(B)], [A - b for b in range(B)]
+    got = dtw_attention_prep([q.to(cuda) for q in q_out], [k.to(cuda) for k in k_out], head_mask, lens, caps)
+    _check_fused(got, dtw_prep_ref(_qk_ref(q_out, k_out, head_mask, n_heads), lens, caps, 7), f"B={B} T={T}")
+
+
 def test_attention_prep_fused_many_heads_and_layouts(cuda):
     # 32 heads (the most the entry takes), one projection a column slice of a wider tensor
     from whisperdrz_amd import dtw_attention_prep
