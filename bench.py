@@ -10,7 +10,7 @@ algorithmic HBM bytes (only valid K/V rows are counted), each with 32 distinct p
 captured into one hipGraph and replayed, and under ``cpu_baseline`` the reference's CPU torch
 path (torch SDPA, fp32) timed on this host's cores on a bounded sample. Under ``dtw_prep`` it
 carries the DTW alignment inputs (compute_attention and _dtw_prep_batch) in GB/s of algorithmic
-HBM bytes, and under ``log_mel`` the GPU log-mel front end in TFLOP/s of fp32 matrix work, each
+HBM bytes, and under ``log_mel`` the GPU log-mel front end in GB/s of its samples and mel, each
 with its own roofline and CPU baseline.
 
 Under ``cross_fill`` it times the encoder output's projection into every layer's cross cache (the
@@ -38,7 +38,6 @@ if ROOT not in sys.path:
 METRIC = "enc-attn TFLOP/s + decode-attn HBM GB/s at large-v3 shape, % of MI355X roofline"
 # MI355X published peaks (dense, no sparsity).
 PEAK_BF16_TFLOPS = 2500.0
-PEAK_FP32_TFLOPS = 157.3
 PEAK_HBM_GBS = 8000.0
 
 H, D = 20, 64
@@ -153,8 +152,9 @@ def bench_encoder(dev, steps: int, warmup: int) -> dict:
 
 def bench_config1(dev, steps: int, warmup: int) -> dict:
     """Config 1 (the reference's CPU-runnable case) on the GPU: one encoder layer, B=1 H=20
-    L=1500 D=64 in fp32, non-causal, scale 1/8, on the fp32 matrix cores (dense_f32_kernel), so
-    its roofline is the fp32 matrix peak; 8 seeded input sets in rotation."""
+    L=1500 D=64 in fp32, non-causal, scale 1/8 (dense_f32_kernel: every fp32 product is six bf16
+    matrix products, so its roofline is a sixth of the bf16 matrix peak); 8 seeded input sets in
+    rotation."""
     from whisperdrz_amd import scaled_dot_product_attention
 
     B, L, n_sets = 1, 1500, 8
@@ -175,7 +175,7 @@ def bench_config1(dev, steps: int, warmup: int) -> dict:
     us = timed_events(run, steps, stream) * 1e3 / n_sets
     tflops = flop / (us * 1e-6) / 1e12
     log(f"[bench] config1 fp32 dense (B=1 H=20 L=1500): {us:.1f} us per layer, {tflops:.2f} TFLOP/s "
-        f"({100 * tflops / PEAK_FP32_TFLOPS:.1f}% of the fp32 matrix peak)")
+        f"({100 * 6 * tflops / PEAK_BF16_TFLOPS:.1f}% of a sixth of the bf16 matrix peak)")
     del sets
     torch.cuda.empty_cache()
     return {
@@ -183,10 +183,10 @@ def bench_config1(dev, steps: int, warmup: int) -> dict:
                     "(the shape of cpu_baseline), 8 seeded input sets in rotation",
         "us_per_layer": round(us, 2),
         "tflops": round(tflops, 3),
-        "roofline": {"bound": "mfma", "achieved": round(tflops, 3), "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
-                     "frac": round(tflops / PEAK_FP32_TFLOPS, 4), "traffic": measured_traffic("dense_f32_kernel<false>"),
+        "roofline": {"bound": "mfma", "achieved": round(tflops, 3), "peak": round(PEAK_BF16_TFLOPS / 6, 1),
+                     "unit": "TFLOP/s", "frac": round(6 * tflops / PEAK_BF16_TFLOPS, 4), "traffic": measured_traffic("dense_f32_kernel<false>"),
                      "traffic_source": "profiles/pmc_traffic.json (rocprofv3 FETCH_SIZE/WRITE_SIZE passes)",
-                     "kernel": "dense_f32_kernel<false> (v_mfma_f32_32x32x2_f32)"},
+                     "kernel": "dense_f32_kernel<false> (six v_mfma_f32_32x32x16_bf16 products per fp32 product)"},
     }
 
 
@@ -782,10 +782,10 @@ def bench_cross_fill(dev, steps: int, warmup: int) -> dict:
 MEL_B, MEL_N, MEL_MELS = 16, 480000, 128
 
 
-def mel_flop(n_frames: int) -> float:
-    """Algorithmic matrix-core work per window: the windowed DFT of the 201 kept bins (real and
-    imaginary parts, 400 samples) and the mel projection (201 bins -> 128 mels), 2 flops per MAC."""
-    return n_frames * (2.0 * 400 * 2 * 201 + 2.0 * 201 * MEL_MELS)
+def mel_bytes() -> int:
+    """Bytes a batch cannot do without: the samples read once, the mel written once (fp32). The work
+    beside them is small (a 400-point real FFT per frame), so the front end's roofline is HBM."""
+    return 4 * MEL_B * (MEL_N + MEL_MELS * 3000)
 
 
 def bench_logmel(dev, steps: int, warmup: int) -> dict:
@@ -798,10 +798,9 @@ def bench_logmel(dev, steps: int, warmup: int) -> dict:
         for x in audio:
             log_mel_spectrogram(x, MEL_MELS, 3000)
     ms = timed_events(lambda: [log_mel_spectrogram(x, MEL_MELS, 3000) for x in audio], steps, stream) / len(audio)
-    flop = MEL_B * mel_flop(MEL_N // 160)
-    tflops = flop / (ms * 1e-3) / 1e12
+    gbs = mel_bytes() / (ms * 1e-3) / 1e9
     log(f"[bench] log-mel: {ms * 1e3:.1f} us per {MEL_B} x 30 s windows ({MEL_B / ms * 1e3:.0f} windows/s), "
-        f"{tflops:.1f} TFLOP/s fp32 ({100 * tflops / PEAK_FP32_TFLOPS:.1f}% of the fp32 matrix peak)")
+        f"{gbs:.0f} GB/s ({100 * gbs / PEAK_HBM_GBS:.1f}% of HBM)")
     del audio
     return {
         "workload": f"LogMelSpectrogram: {MEL_B} windows of 30 s (480000 samples, fp32, on the GPU) -> "
@@ -809,13 +808,14 @@ def bench_logmel(dev, steps: int, warmup: int) -> dict:
         "us_per_batch": round(ms * 1e3, 2),
         "windows_per_s": round(MEL_B / ms * 1e3, 1),
         "roofline": {
-            "bound": "mfma",
-            "achieved": round(tflops, 2),
-            "peak": PEAK_FP32_TFLOPS,
-            "unit": "TFLOP/s",
-            "frac": round(tflops / PEAK_FP32_TFLOPS, 4),
-            "flop_per_batch": flop,
-            "kernel": "logmel_spec_kernel (fp32 MFMA)",
+            "bound": "hbm",
+            "achieved": round(gbs, 1),
+            "peak": PEAK_HBM_GBS,
+            "unit": "GB/s",
+            "frac": round(gbs / PEAK_HBM_GBS, 4),
+            "traffic": None,
+            "bytes_per_batch": mel_bytes(),
+            "kernel": "logmel_spec_kernel, logmel_finish_kernel",
         },
     }
 
@@ -1059,7 +1059,7 @@ _ALG_BYTES = {
     "dtw_qk_kernel<wdrz::Bf16>": 430080000 + 2 * 16 * 10 * (448 + 1500) * 64,
     "kv_fill_kernel": 2 * 2 * 16 * 1500 * 1280 * 2,
     "median_filter_kernel<3>": 2 * 16 * 10 * 448 * 1500 * 4,
-    "dtw_qk_rowcol_kernel<wdrz::Bf16>": 2 * 16 * 10 * (448 + 1500) * 64 + 16 * 10 * 448 * 8 + 16 * 10 * 4 * 1500 * 8,
+    "dtw_qk_rowcol_kernel<wdrz::Bf16>": 2 * 16 * 10 * (448 + 1500) * 64 + 16 * 10 * 448 * 8 + 16 * 10 * 3 * 1500 * 8,
     "dtw_qk_band_kernel<wdrz::Bf16, 3>": 2 * 16 * 10 * (448 + 1500) * 64 + 16 * 10 * (448 + 1500) * 8
     + 16 * 448 * 1500 * 4,
     "dense_f32_kernel<false>": 4 * 1500 * 20 * 64 * 4,
@@ -1199,7 +1199,7 @@ def pmc_sample(dev) -> None:
         log_mel_spectrogram(audio, MEL_MELS, 3000)
         torch.cuda.synchronize()
     del audio
-    # config 1 (fp32 matrix cores), one bf16 window (the key-split kernel), the decode step's
+    # config 1 (fp32), one bf16 window (the key-split kernel), the decode step's
     # fused fc1 + GELU on three distinct (cold) weights
     from whisperdrz_amd import linear_gelu
 

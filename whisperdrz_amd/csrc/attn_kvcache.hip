@@ -842,8 +842,10 @@ void kv_split_plan(int64_t units, int64_t Lk, int* n_splits, int* split_len) {
 // queries 10.9 / 19.5 / 30.0 / 72.3 -> 8.9 / 16.4 / 29.4 / 63.0. At 6 streams (120 workgroups)
 // unsplit 13.4 us, two splits 13.0; at 8 (160) unsplit 14.9, three splits 15.6.
 constexpr int64_t kSplitUnits = 160;      // workgroups below which long rows are split
-constexpr int64_t kSplitMinLk = 1024;     // rows shorter than this are never split
-constexpr int64_t kSplitMinKeys = 192;
+// 448-row caches lose by any split (one stream 5.6 -> 7.6 us), 1500-row ones win up to 7 streams; a
+// row of 1024 keys streams for about as long as a merge takes.
+constexpr int64_t kSplitMinLk = 1024;
+constexpr int64_t kSplitMinKeys = 192;    // one stream, cross: 12 splits of 128 keys 9.0 us, 8 of 192 8.4
 // Eight wavefronts a workgroup instead of four while the launch has no more workgroups than CUs:
 // 5 queries, self, 1 / 12 streams 6.7 / 8.3 -> 5.9 / 7.7 us; at 24 and 48 streams 10.4 and 15.4 ->
 // 10.2 and 17.6 (a second round of workgroups no longer fits beside the first).
