@@ -162,3 +162,33 @@ def test_width_not_multiple_of_128(cuda):
             pos = ph.self_kv[0].seq_lens[slots].long()
             _close(hip.forward_flash(tok, ph.self_kv, ph.cross_kv, pos, slot_indices=slots),
                    ref.forward_flash(tok, pr.self_kv, pr.cross_kv, pos, slot_indices=slots), dtype, "step logits")
+
+
+def test_graph_inputs_from_host_and_other_types(cuda):
+    """The captured step's inputs come in one grouped copy: host tensors, int32 indices and strided
+    views give the same logits and lengths as int64 tensors on the GPU, bit for bit."""
+    from whisperdrz_amd.decoder import BucketedDecodeGraphs
+
+    hip, _ = _make(cuda, torch.bfloat16)
+    B = 3
+    pool = _pool(cuda, torch.bfloat16, 4)
+    g = torch.Generator(device=cuda).manual_seed(4)
+    pool.arena.view(torch.bfloat16).normal_(generator=g)
+    tokens = torch.randint(0, N_VOCAB, (B, 1), generator=g, device=cuda)
+    lens = torch.tensor([5, 9, 1], device=cuda)
+    slots = torch.arange(B, device=cuda)
+    outs = []
+    with torch.no_grad():
+        graphs = BucketedDecodeGraphs(hip, pool, N_VOCAB, buckets=[4])
+        graphs.capture(4)
+        wide = torch.zeros(B, 5, dtype=torch.long, device=cuda)
+        wide[:, 2:3] = tokens
+        for args in ((tokens, lens, slots), (tokens.cpu(), lens.cpu(), slots.cpu()),
+                     (tokens.int(), lens.int(), slots.int()), (wide[:, 2:3], lens, slots)):
+            pool.self_seq_lens[:, :B] = lens.int()
+            pool.self_seq_lens[:, B] = 1
+            logits = graphs.forward(*args).clone()
+            outs.append((logits, pool.self_seq_lens.clone()))
+    for logits, after in outs[1:]:
+        assert torch.equal(logits, outs[0][0]) and torch.equal(after, outs[0][1])
+    assert torch.equal(outs[0][1][:, :B], (lens.int() + 1).expand(N_LAYER, B))
