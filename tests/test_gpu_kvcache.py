@@ -440,3 +440,30 @@ def test_plan_lines(cuda, dtype, self_attn, B, sq, H, Lmax):
     assert_close(out, ref, dtype, f"B={B} sq={sq} H={H} Lmax={Lmax} self={self_attn}")
     assert np.array_equal(to_np(kd), kref) and np.array_equal(to_np(vd), vref)
     assert not ws.any()
+
+
+# (B, sq, H, Lmax) of the 16-bit kernels whose only 16-bit rounding is the output's
+EXACT_P_SHAPES = [(1, 1, 20, 448), (4, 1, 20, 1500), (8, 1, 20, 1500), (16, 1, 20, 1500)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("self_attn", [True, False])
+@pytest.mark.parametrize("B,sq,H,Lmax", EXACT_P_SHAPES)
+def test_probabilities_are_not_rounded(cuda, dtype, self_attn, B, sq, H, Lmax):
+    """Element by element within the output's own rounding (half an ulp: 2^-8 / 2^-11 of the value)
+    and what fp32 scores, exponents and sums (and, for several queries, a probability held as two
+    16-bit values: 2^-17 / 2^-23 of it) leave: below 2^-16 / 2^-18 of the largest |v|, since the
+    result is a mean of v. Probabilities rounded to 16 bits miss it several times over."""
+    from whisperdrz_amd import flash_attn_with_kvcache
+
+    u, rest = (2.0 ** -8, 2.0 ** -16) if dtype == torch.bfloat16 else (2.0 ** -11, 2.0 ** -18)
+    kc, vc = make_cache(B, Lmax, H, 64, dtype, "cpu", "head_major", 3)
+    q, k, v = (randn((B, sq, H, 64), s, dtype) for s in (5, 6, 7))
+    cs = np.full(B, Lmax - sq, np.int32) if self_attn else None
+    new = (to_np(k), to_np(v)) if self_attn else (None, None)
+    ref, _, _ = kvcache_ref(to_np(q), to_np(kc), to_np(vc), *new, cs, None, 0.125)
+    kw = dict(k=k.to(cuda), v=v.to(cuda), cache_seqlens=torch.from_numpy(cs).to(cuda)) if self_attn else {}
+    out = to_np(flash_attn_with_kvcache(q.to(cuda), kc.to(cuda), vc.to(cuda), softmax_scale=0.125, **kw))
+    over = np.abs(out - ref) - u * np.abs(ref)
+    bound = rest * float(np.abs(to_np(vc)).max())
+    assert over.max() <= bound, f"B={B} sq={sq} self={self_attn}: {over.max():.2e} past the rounding > {bound:.2e}"

@@ -10,7 +10,7 @@
 // bound and uses no MFMA. A head row of K or V is 64 elements = one 16-byte load per lane
 // across LPK lanes (8 lanes in 16-bit types, 16 in fp32). Lane groups of LPK lanes each own
 // a strided subset of the keys, keep kUnroll keys in flight per batch and run an online
-// softmax in the log2 domain; in 16-bit types q.k and P.V run on v_dot2 (P.V over key pairs).
+// softmax in the log2 domain; in 16-bit types q.k runs on v_dot2, P.V in fp32 throughout.
 //
 // Launch shape: one 4-wavefront workgroup per (batch row, query block of up to 8, head, key
 // split); its wavefront partials merge through LDS. Rows split their keys only when there are
@@ -38,7 +38,7 @@ namespace {
 
 constexpr int kMaxSQ = 8;  // query rows per workgroup
 constexpr int kWavesPerWg = 4;   // wavefronts per workgroup
-constexpr int kUnroll = 4;       // keys per lane group per batch (even: P V runs on key pairs)
+constexpr int kUnroll = 4;       // keys per lane group per batch
 constexpr int kMinSplitKeys = 128;
 constexpr int kMaxMergeSplits = 32;  // upper bound on splits per row (host plan guarantees it)
 constexpr float kTau = 8.0f;  // lazy-rescale threshold (log2 units)
@@ -431,41 +431,20 @@ __global__ __launch_bounds__(kWavesPerWg * 64) void kv_attn_kernel(KvArgs a) {
         for (int e = 0; e < EPL; ++e) acc[t][e] *= alpha;
       }
     }
-    // ---- P V ----
-    if constexpr (EB == 2) {
-      // Keys in pairs: v_perm gathers dim e of both keys into one dword, v_dot2 multiplies it
-      // with the packed pair of probabilities.
+    // ---- P V in fp32: probabilities rounded to 16 bits cost a third of the result's error (fp16,
+    // one query over 1500 rows, 4 / 16 streams: 2.8e-4 / 2.9e-4 from 64 bits, this 2.1e-4, which is
+    // the output's own rounding) and save nothing in fp16 (v_fma_mix); bf16 pays 16 more
+    // instructions a key pair: 4 / 8 / 52 streams 11.3 / 13.7 / 68.7 -> 11.6 / 14.1 / 69.0 us ----
 #pragma unroll
-      for (int u = 0; u < kUnroll; u += 2) {
-        u32x4 vlo, vhi;
+    for (int u = 0; u < kUnroll; ++u) {
+      Slice<T> vs;
+      vs.from_raw(vr[u]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          vlo[i] = __builtin_amdgcn_perm(vr[u + 1][i], vr[u][i], 0x05040100u);
-          vhi[i] = __builtin_amdgcn_perm(vr[u + 1][i], vr[u][i], 0x07060302u);
-        }
+      for (int t = 0; t < SQ; ++t) {
+        const float p = fast_exp2(sc[t][u] - m[t]);
+        l[t] += p;
 #pragma unroll
-        for (int t = 0; t < SQ; ++t) {
-          const uint32_t pp = Dot2<T>::pack(fast_exp2(sc[t][u] - m[t]), fast_exp2(sc[t][u + 1] - m[t]));
-          l[t] = Dot2<T>::run(pp, Dot2<T>::kOnes, l[t]);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            acc[t][2 * i] = Dot2<T>::run(pp, vlo[i], acc[t][2 * i]);
-            acc[t][2 * i + 1] = Dot2<T>::run(pp, vhi[i], acc[t][2 * i + 1]);
-          }
-        }
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        Slice<T> vs;
-        vs.from_raw(vr[u]);
-#pragma unroll
-        for (int t = 0; t < SQ; ++t) {
-          const float p = fast_exp2(sc[t][u] - m[t]);
-          l[t] += p;
-#pragma unroll
-          for (int e = 0; e < EPL; ++e) acc[t][e] = __builtin_fmaf(p, vs.v[e], acc[t][e]);
-        }
+        for (int e = 0; e < EPL; ++e) acc[t][e] = __builtin_fmaf(p, vs.v[e], acc[t][e]);
       }
     }
   };
