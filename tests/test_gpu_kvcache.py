@@ -443,7 +443,8 @@ def test_plan_lines(cuda, dtype, self_attn, B, sq, H, Lmax):
 
 
 # (B, sq, H, Lmax) of the 16-bit kernels whose only 16-bit rounding is the output's
-EXACT_P_SHAPES = [(1, 1, 20, 448), (4, 1, 20, 1500), (8, 1, 20, 1500), (16, 1, 20, 1500)]
+EXACT_P_SHAPES = [(1, 1, 20, 448), (4, 1, 20, 1500), (8, 1, 20, 1500), (16, 1, 20, 1500), (1, 2, 20, 1500),
+                  (16, 5, 20, 1500), (4, 12, 20, 1500), (2, 39, 20, 448)]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -467,3 +468,28 @@ def test_probabilities_are_not_rounded(cuda, dtype, self_attn, B, sq, H, Lmax):
     over = np.abs(out - ref) - u * np.abs(ref)
     bound = rest * float(np.abs(to_np(vc)).max())
     assert over.max() <= bound, f"B={B} sq={sq} self={self_attn}: {over.max():.2e} past the rounding > {bound:.2e}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("self_attn", [True, False])
+@pytest.mark.parametrize("B,sq,H,Lmax", [(2, 1, 3, 300), (2, 5, 3, 300), (1, 12, 2, 1500), (16, 2, 20, 200)])
+def test_infinite_values(cuda, dtype, self_attn, B, sq, H, Lmax):
+    """An infinite value is infinite in the outputs that see it, in its column alone, and changes
+    nothing elsewhere by more than an ulp of the largest output (another order of the sums)."""
+    from whisperdrz_amd import flash_attn_with_kvcache
+
+    kc, vc = make_cache(B, Lmax, H, 64, dtype, "cpu", "head_major", 3)
+    q, k, v = (randn((B, sq, H, 64), s, dtype) for s in (5, 6, 7))
+    q, kc = 0.1 * q, 0.1 * kc  # near-uniform probabilities: none rounds to zero
+    cs = torch.full((B,), Lmax - sq, dtype=torch.int32, device=cuda)
+    kw = dict(k=k.to(cuda), v=v.to(cuda), cache_seqlens=cs) if self_attn else {}
+    run = lambda values: to_np(flash_attn_with_kvcache(q.to(cuda), kc.clone().to(cuda), values.clone().to(cuda), **kw))
+    plain = run(vc)
+    bad = vc.clone()
+    bad[0, 7, 1, 9], bad[0, 150, 0, 3] = float("inf"), float("-inf")
+    out = run(bad)
+    hit = np.zeros(out.shape, bool)
+    hit[0, :, 1, 9] = hit[0, :, 0, 3] = True
+    assert (out[0, :, 1, 9] == np.inf).all() and (out[0, :, 0, 3] == -np.inf).all()
+    ulp = (2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10) * np.abs(plain).max()
+    assert np.abs(out - plain)[~hit].max() <= ulp

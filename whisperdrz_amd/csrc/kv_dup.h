@@ -62,7 +62,7 @@ __device__ __forceinline__ int kv_dup_winner(const KvArgs& a, int slot, int p, i
   int w = -1;
   for (int i = 0; i < a.B; ++i) {
     const int ci = a.seqlens[i];
-    if (kv_dup_appends(a, a.bidx[i], ci, slot) && p >= ci && p < ci + a.sq) {
+    if (kv_dup_appends(a, a.bidx ? a.bidx[i] : i, ci, slot) && p >= ci && p < ci + a.sq) {
       w = i;
       cs_w = ci;
     }
@@ -99,7 +99,8 @@ __device__ __forceinline__ float kv_elem(const char* row, int d) {
 // wavefronts); in each batch of 64 keys a lane computes one key's score, then the lanes take the
 // 64 head dimensions for P.V. emit(t, d, o, m, l) receives, in lane d, the unnormalised output
 // and the running max (log2 units) and sum, as the fast paths keep them for their merge. q_lds: 64
-// floats of LDS per wavefront. Slow (latency-bound): used only for the overlapping appends above.
+// floats of LDS per wavefront. Slow (latency-bound): used only for the overlapping appends above and
+// where a fast path's arithmetic meets an infinite value.
 template <typename T, int kWaves, typename Emit>
 __device__ __forceinline__ void kv_generic_rows(const KvArgs& a, int b, int h, int slot, int cs, int t0, int nq,
                                                 int k_begin, int k_end, bool self_attn, float (*q_lds)[kHeadDim],
