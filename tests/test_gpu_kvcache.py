@@ -408,7 +408,7 @@ def test_default_scale_is_head_dim_power(cuda):
 
 # (B, sq, H, Lmax): both sides of the 16-bit plan's lines: long rows split below 160 workgroups
 # (20 x 7 = 140 / 20 x 8 = 160), short ones never (1023 / 1024), eight wavefronts up to 256
-# workgroups (252 / 260), 16-row blocks up to 512 (500 / 520) or 16 queries, splits of 16-row blocks
+# workgroups (252 / 260), 16-row blocks up to 512 (500 / 520) or 39 queries, splits of 16-row blocks
 PLAN_SHAPES = [(7, 1, 20, 1500), (8, 1, 20, 1500), (1, 1, 1, 1023), (1, 1, 1, 1024), (2, 3, 2, 6200),
                (63, 2, 4, 130), (65, 2, 4, 130), (1, 16, 4, 1024), (1, 17, 4, 1500), (1, 39, 2, 1500), (5, 9, 50, 70),
                (5, 33, 35, 64), (5, 17, 50, 64), (5, 17, 52, 64), (13, 16, 40, 64), (2, 64, 64, 130), (3, 64, 64, 130)]
@@ -444,7 +444,7 @@ def test_plan_lines(cuda, dtype, self_attn, B, sq, H, Lmax):
 
 # (B, sq, H, Lmax) of the 16-bit kernels whose only 16-bit rounding is the output's
 EXACT_P_SHAPES = [(1, 1, 20, 448), (4, 1, 20, 1500), (8, 1, 20, 1500), (16, 1, 20, 1500), (1, 2, 20, 1500),
-                  (16, 5, 20, 1500), (4, 12, 20, 1500), (2, 39, 20, 448)]
+                  (16, 5, 20, 1500), (4, 12, 20, 1500), (2, 39, 20, 448), (16, 17, 20, 500), (9, 39, 20, 500)]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

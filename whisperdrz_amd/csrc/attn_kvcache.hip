@@ -23,9 +23,9 @@
 // cannot race with any read in the same launch.
 //
 // Which kernel serves a call (kv_plan16): 16-bit calls of 2-8 query rows run on kv_mq_kernel (MFMA
-// over the rows, below), more rows in its 16-row blocks, or, when those fill the chip more than
-// twice, on kv_prefill_kernel in attn_dense.hip (256-query MFMA blocks); single rows and fp32 caches
-// run on kv_attn_kernel.
+// over the rows, below), more rows in its 16-row blocks, or, from 40 rows on and when those fill the
+// chip more than twice, on kv_prefill_kernel in attn_dense.hip (256-query MFMA blocks); single rows and
+// fp32 caches run on kv_attn_kernel.
 #include <algorithm>
 
 #include "kv_dup.h"
@@ -871,12 +871,11 @@ constexpr int64_t kWideWgs = 256;
 // leave a small launch few workgroups. Cross over 1500 rows, 16-query blocks / 256-query blocks:
 // 224 queries x 2 streams (560 workgroups) 34.8 / 40.0 us, 112 x 4 (560) 37.1 / 34.4, 64 x 6 (480)
 // 29.2 / 34.2, 64 x 8 (640) 41.1 / 34.6.
-// Below kPrefillMinSq queries the second and third block of a row are the question: cross, 17 / 33
-// queries x 32 streams 82 / 111 us in blocks of 16, 67 / 69 in 256-query blocks; 16 queries (one
-// block) 45 / 69. Self rows are short (their 256-query kernel also appends): 39 queries x 32 streams
-// 29.8 / 30.
+// Below kPrefillMinSq queries every call stays on the blocks of 16: the 256-query kernels round the
+// scaled queries and the probabilities to 16 bits (cross, 17-39 fp16 queries: 3.6e-4 from 64 bits
+// against 2.1e-4 here), although they are faster there (cross, 17 / 33 queries x 32 streams 82 / 111 us
+// in blocks of 16, 67 / 69 in 256-query blocks).
 constexpr int64_t kMq16Wgs = 512;
-constexpr int kCrossMqMaxSq = 16;
 
 void kv_plan16(KvArgs* a) {
   const int64_t B = a->B, H = a->H;
@@ -886,8 +885,7 @@ void kv_plan16(KvArgs* a) {
   a->split_len = a->Lk;
   if (a->sq > 8) {
     a->n_qblocks = (a->sq + 15) / 16;
-    const bool many = a->sq >= kPrefillMinSq || (a->kn == nullptr && a->sq > kCrossMqMaxSq);
-    a->route = blocks16 > kMq16Wgs && many ? kKvPrefill : kKvMq16;
+    a->route = blocks16 > kMq16Wgs && a->sq >= kPrefillMinSq ? kKvPrefill : kKvMq16;
   } else {
     a->route = a->sq > 1 ? kKvMq8 : kKvRow;
   }
