@@ -406,12 +406,15 @@ def test_default_scale_is_head_dim_power(cuda):
     assert torch.equal(a, b) and torch.equal(c, d)
 
 
-# (B, sq, H, Lmax): both sides of the 16-bit plan's lines: long rows split below 160 workgroups
-# (20 x 7 = 140 / 20 x 8 = 160), short ones never (1023 / 1024), eight wavefronts up to 256
-# workgroups (252 / 260), 16-row blocks up to 512 (500 / 520) or 39 queries, splits of 16-row blocks
+# (B, sq, H, Lmax): both sides of the 16-bit plan's lines: long rows split up to 128 of them (32 x 4 /
+# 43 x 3) and from 257 to 341 (64 x 4 / 257, 31 x 11 / 38 x 9; not in 16-row blocks), short ones never
+# (767 / 768), eight wavefronts up to 256 workgroups (252 / 260), 16-row blocks up to 512 (500 / 520) or
+# 39 queries, splits of 16-row blocks
 PLAN_SHAPES = [(7, 1, 20, 1500), (8, 1, 20, 1500), (1, 1, 1, 1023), (1, 1, 1, 1024), (2, 3, 2, 6200),
                (63, 2, 4, 130), (65, 2, 4, 130), (1, 16, 4, 1024), (1, 17, 4, 1500), (1, 39, 2, 1500), (5, 9, 50, 70),
-               (5, 33, 35, 64), (5, 17, 50, 64), (5, 17, 52, 64), (13, 16, 40, 64), (2, 64, 64, 130), (3, 64, 64, 130)]
+               (5, 33, 35, 64), (5, 17, 50, 64), (5, 17, 52, 64), (13, 16, 40, 64), (2, 64, 64, 130), (3, 64, 64, 130),
+               (1, 2, 1, 767), (1, 2, 1, 768), (32, 1, 4, 800), (43, 1, 3, 800), (64, 1, 4, 1030), (257, 1, 1, 1030),
+               (31, 1, 11, 1030), (38, 1, 9, 1030), (16, 5, 20, 1030), (16, 12, 20, 800)]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

@@ -853,16 +853,30 @@ void kv_split_plan(int64_t units, int64_t Lk, int* n_splits, int* split_len) {
 
 // 16-bit rows are bound by streaming their keys: one 4-wavefront workgroup walks 1500 of them in
 // ~7 us, and merging splits costs ~3 us (publish, count, read back: three trips to the coherence
-// point), so splits pay only for long rows that leave most CUs without a workgroup. Measured
-// (20 heads, per launch; splits for >= 1024 workgroups, as before -> this): self over <= 400 of 448
-// rows, one query 1 / 8 / 16 / 48 streams 7.6 / 7.9 / 10.7 / 16.8 -> 5.6 / 6.6 / 8.7 / 13.3 us; cross over 1500, 5
-// queries 10.9 / 19.5 / 30.0 / 72.3 -> 8.9 / 16.4 / 29.4 / 63.0. At 6 streams (120 workgroups)
-// unsplit 13.4 us, two splits 13.0; at 8 (160) unsplit 14.9, three splits 15.6.
-constexpr int64_t kSplitUnits = 160;      // workgroups below which long rows are split
-// 448-row caches lose by any split (one stream 5.6 -> 7.6 us), 1500-row ones win up to 7 streams; a
-// row of 1024 keys streams for about as long as a merge takes.
-constexpr int64_t kSplitMinLk = 1024;
+// point), so splits pay only for long rows, and only where whole rows leave the chip unevenly loaded.
+// Per launch, bf16, cold caches in a graph, us:
+//   * up to half as many rows as CUs: two splits and more, still one workgroup a CU. Cross over 1500,
+//     one query, unsplit / split: 1 stream of 20 heads 11.9 / 8.3, 5 streams (100 rows) 13.0 / 11.9, 6
+//     (120) 13.3 / 12.7; 5 queries x 1 / 6 13.7 / 15.3 -> 8.6 / 13.2.
+//   * from there to one row a CU: unsplit. 7 streams (140 rows) 13.7 / 16.2 (two splits are more than
+//     256 workgroups), 8 14.3 / 15.3 (seven splits); 5 queries x 7 15.4 / 19.1.
+//   * up to a third more rows than CUs: a few CUs with two rows hold up the rest; up to four splits
+//     even that out. 13 streams (260 rows) 24.0 / 22.3, 16 26.5 / 25.1, 17 27.6 / 26.1; 18 (360)
+//     28.2 / 28.4; 5 queries x 13 / 16 / 17 26.9 / 28.5 / 29.0 -> 25.7 / 28.0 / 28.5. With splits of
+//     fewer than 512 keys the 5 queries lose (16 streams: 29.4).
+// Beyond, unsplit (20 streams 27.2 / 29.3). Rows of 4000 to 32000 keys follow the same lines within 10%,
+// except a few streams of 5 queries, which would take more splits (4 streams x 6000 keys 30.7 / 26.5, 8
+// x 16000 131 / 118).
+constexpr int64_t kCus = 256;
+constexpr int64_t kSplitWgs = 160;        // workgroups that splits of up to half the CUs' rows aim at
+constexpr int64_t kEvenRows = kCus * 4 / 3;
+constexpr int64_t kEvenWgs = 1024;
+// Self rows of 448 lose by any split (one stream with 200 / 400 keys 5.1 / 6.6 -> 6.6 / 7.2 us; the
+// one-stream step 238.3 -> 241.2 and 245.0 -> 243.1). Longer rows, one stream: 600 keys 6.8 / 6.9, 800
+// 8.1 / 7.4, 1000 9.1 / 7.5; four: 800 8.6 / 8.8, 1000 9.6 / 9.4.
+constexpr int64_t kSplitMinLk = 768;
 constexpr int64_t kSplitMinKeys = 192;    // one stream, cross: 12 splits of 128 keys 9.0 us, 8 of 192 8.4
+constexpr int64_t kEvenMinKeys = 512;
 // Eight wavefronts a workgroup instead of four while the launch has no more workgroups than CUs:
 // 5 queries, self, 1 / 12 streams 6.7 / 8.3 -> 5.9 / 7.7 us; at 24 and 48 streams 10.4 and 15.4 ->
 // 10.2 and 17.6 (a second round of workgroups no longer fits beside the first).
@@ -891,10 +905,14 @@ void kv_plan16(KvArgs* a) {
   }
   const int64_t units = B * a->n_qblocks * H;
   // kPrefillMinSq or more queries: the workspace query promises that none is needed
-  if (a->route != kKvPrefill && a->sq < kPrefillMinSq && units < kSplitUnits && a->Lk >= kSplitMinLk) {
-    // blocks of 16 rows: at most half as many, so that they fit the workspace of 8-row blocks
-    kv_split_keys(std::min<int64_t>((kSplitUnits + units - 1) / units, kMaxMergeSplits / (a->sq > 8 ? 2 : 1)), a->Lk,
-                  kSplitMinKeys, &a->n_splits, &a->split_len);
+  if (a->route != kKvPrefill && a->sq < kPrefillMinSq && a->Lk >= kSplitMinLk) {
+    // blocks of 16 rows: at most half as many, and none to even the load, so that they fit the
+    // workspace of 8-row blocks
+    if (units <= kCus / 2)
+      kv_split_keys(std::min<int64_t>((kSplitWgs + units - 1) / units, kMaxMergeSplits / (a->sq > 8 ? 2 : 1)), a->Lk,
+                    kSplitMinKeys, &a->n_splits, &a->split_len);
+    else if (a->sq <= 8 && units > kCus && units <= kEvenRows)
+      kv_split_keys((kEvenWgs + units - 1) / units, a->Lk, kEvenMinKeys, &a->n_splits, &a->split_len);
   }
   a->waves = units * a->n_splits <= kWideWgs ? 8 : kWavesPerWg;
 }
