@@ -192,3 +192,30 @@ def test_graph_inputs_from_host_and_other_types(cuda):
     for logits, after in outs[1:]:
         assert torch.equal(logits, outs[0][0]) and torch.equal(after, outs[0][1])
     assert torch.equal(outs[0][1][:, :B], (lens.int() + 1).expand(N_LAYER, B))
+
+
+def _steps_match(hip, ref, ph, pr, dtype, B, g, cuda, what):
+    """A few cached steps of B rows on both stacks from the caches' present state."""
+    slots = torch.arange(B, device=cuda)
+    with torch.no_grad():
+        for _ in range(2):
+            tok = torch.randint(0, N_VOCAB, (B, 1), generator=g, device=cuda)
+            pos = ph.self_kv[0].seq_lens[slots].long()
+            _close(hip.forward_flash(tok, ph.self_kv, ph.cross_kv, pos, slot_indices=slots),
+                   ref.forward_flash(tok, pr.self_kv, pr.cross_kv, pos, slot_indices=slots), dtype, what)
+            assert all(torch.equal(a.seq_lens, b.seq_lens) for a, b in zip(ph.self_kv, pr.self_kv))
+
+
+@pytest.mark.parametrize("hidden", [640, 1024])
+@pytest.mark.parametrize("B", [1, 4, 5])
+def test_other_mlp_widths(cuda, hidden, B):
+    """An MLP width that the split-K kernel does not take (640 is no multiple of 512) keeps torch's
+    MLP, in steps of up to four rows as in larger ones."""
+    dtype = torch.bfloat16
+    hip, ref = _make(cuda, dtype)
+    for a, b in zip(hip.blocks, ref.blocks):
+        a.mlp = torch.nn.Sequential(torch.nn.Linear(N_STATE, hidden), torch.nn.GELU(),
+                                    torch.nn.Linear(hidden, N_STATE)).to(cuda, dtype)
+        b.mlp = copy.deepcopy(a.mlp)
+    g = torch.Generator(device=cuda).manual_seed(hidden + B)
+    _steps_match(hip, ref, _pool(cuda, dtype, B), _pool(cuda, dtype, B), dtype, B, g, cuda, f"hidden {hidden}")

@@ -290,7 +290,8 @@ class TextDecoderStack(nn.Module):
         # a small step: every add + LayerNorm inside the projection that follows it
         n = self.n_state
         if (x.numel() // n if n else 0) <= LN_LINEAR_ROWS and n % 256 == 0 and n <= LN_LINEAR_MAX_K and all(
-                m.bias is not None for b in blocks for m in (b.attn.out, b.cross_attn.out, b.mlp[2])):
+                m.bias is not None for b in blocks for m in (b.attn.out, b.cross_attn.out, b.mlp[2])) and all(
+                b.mlp[2].in_features % 512 == 0 for b in blocks):
             part = lin = None
             for i, (block, s_kv, c_kv) in enumerate(zip(blocks, self_kv, cross_kv, strict=True)):
                 attn, cross, fc1, fc2 = block.attn, block.cross_attn, block.mlp[0], block.mlp[2]
