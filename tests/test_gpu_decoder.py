@@ -219,3 +219,17 @@ def test_other_mlp_widths(cuda, hidden, B):
         b.mlp = copy.deepcopy(a.mlp)
     g = torch.Generator(device=cuda).manual_seed(hidden + B)
     _steps_match(hip, ref, _pool(cuda, dtype, B), _pool(cuda, dtype, B), dtype, B, g, cuda, f"hidden {hidden}")
+
+
+def test_int64_lengths(cuda):
+    """Layer lengths kept as rows of an int64 matrix (the kernels take int32): the step converts them,
+    as it does separate int64 lengths."""
+    dtype, B = torch.bfloat16, 3
+    hip, ref = _make(cuda, dtype)
+    pools = [_pool(cuda, dtype, B) for _ in range(2)]
+    for p in pools:
+        lens = torch.tensor([[2, 0, 5]] * N_LAYER, device=cuda)
+        for l, kv in enumerate(p.self_kv):
+            kv.seq_lens = lens[l]
+    g = torch.Generator(device=cuda).manual_seed(3)
+    _steps_match(hip, ref, *pools, dtype, B, g, cuda, "int64 lengths")

@@ -265,13 +265,14 @@ class TextDecoderStack(nn.Module):
 
     def _fused_prologue(self, tokens: Tensor, positions: Tensor, slot_indices: Optional[Tensor], lens: Tensor) -> bool:
         """Whether ``step_begin`` / ``step_end_`` take this step: 16-bit, 16-byte aligned tables of up
-        to 2048 values on the GPU, int64 indices there, a plain embedding without hooks, at least one
-        row, rows within the slots."""
+        to 2048 values on the GPU, int64 indices and int32 lengths there, a plain embedding without
+        hooks, at least one row, rows within the slots."""
         emb, pos, dev = self.token_embedding, self.positional_embedding, lens.device
         w, ln = emb.weight, self.blocks[0].attn_ln
         idx = [tokens, positions] + ([slot_indices] if slot_indices is not None else [])
         return (self.fused_small_ops and w.is_cuda and w.dtype in (torch.bfloat16, torch.float16)
                 and all(t.device == dev for t in (w, pos, ln.weight, *idx)) and all(t.dtype == torch.int64 for t in idx)
+                and lens.dtype == torch.int32
                 and w.dtype == pos.dtype == ln.weight.dtype == ln.bias.dtype and w.shape[1] % 8 == 0
                 and w.shape[1] <= 2048 and w.is_contiguous() and pos.is_contiguous()
                 and w.data_ptr() % 16 == 0 and pos.data_ptr() % 16 == 0 and tokens.numel() > 0
