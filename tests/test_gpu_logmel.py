@@ -97,3 +97,16 @@ def test_rejects(cuda):
         log_mel_spectrogram(torch.zeros(1000, device=cuda), n_mels=129)
     with pytest.raises(NotImplementedError):
         LogMelSpectrogram(128, n_fft=512)
+
+
+def test_overflowing_power_is_infinite(cuda):
+    """Samples whose power overflows fp32 make the mel, its maximum and with it the whole window
+    infinite, never NaN: a 1 kHz tone of 1e18 (three bins of power above 3.4e38, all inside the one
+    filter) beside the same tone at 1, which stays as it is alone."""
+    from whisperdrz_amd import log_mel_spectrogram
+
+    t = torch.arange(16000, dtype=torch.float64) / 16000
+    tone = torch.sin(2 * np.pi * 1000 * t)
+    got = log_mel_spectrogram(torch.stack([1e18 * tone, tone]).float().to(cuda), 1)
+    assert (got[0] == float("inf")).all()
+    _check(got[1], log_mel_ref(tone.float().numpy(), 1), "the finite window")

@@ -192,12 +192,14 @@ __device__ __forceinline__ double mel_edge(int j, int n_mels) {
   return m < 15.0 ? f_sp * m : 1000.0 * exp(logstep * (m - 15.0));
 }
 
-// log10 of a normal number: log2 (one instruction, no denormals to scale) times log10(2) in two parts.
+// log10 of a normal number or infinity: log2 (one instruction, no denormals to scale) times log10(2) in
+// two parts (inf - inf between them, so infinity is returned as it is).
 __device__ __forceinline__ float log10_normal(float x) {
   constexpr float hi = 0.30102999f, lo = (float)(0.30102999566398119521 - (double)hi);
   const float y = __builtin_amdgcn_logf(x);
   const float r = y * hi;
-  return r + __builtin_fmaf(y, lo, __builtin_fmaf(y, hi, -r));
+  const float v = r + __builtin_fmaf(y, lo, __builtin_fmaf(y, hi, -r));
+  return y < INFINITY ? v : y;
 }
 
 // LDS ops of one wavefront run in order: between its own writes and reads only the compiler has to
