@@ -196,3 +196,25 @@ def test_step_begin_end(cuda, dtype, B, sq, n, with_slots):
     assert torch.equal(x2.view(B * sq, n)[1:], x.view(B * sq, n)[1:])
     if with_slots:
         assert (seqlens2[:, 0] == -1).all()
+
+
+def test_step_ends_operands(cuda):
+    """Operands elsewhere, of other types or of sizes that do not fit are refused on the host."""
+    from whisperdrz_amd.decode_ops import step_begin, step_end_
+
+    i32, i64, dt = torch.int32, torch.int64, torch.bfloat16
+    lens, seqlens = torch.zeros(2, 4, dtype=i32, device=cuda), torch.zeros(2, 3, dtype=i32, device=cuda)
+    slots = torch.zeros(3, dtype=i64, device=cuda)
+    for bad in ((lens, seqlens.cpu(), slots), (lens, seqlens, slots.cpu()), (lens.cpu(), seqlens, slots)):
+        with pytest.raises(RuntimeError, match="is on"):
+            step_end_(*bad, 1)
+    with pytest.raises(TypeError):
+        step_end_(lens.long(), seqlens, slots, 1)
+    for bad in ((lens[:1], seqlens, slots), (lens, seqlens[:, ::2], None), (lens, seqlens, slots[:2]),
+                (lens, seqlens, slots.int()), (lens[:, :2].contiguous(), seqlens, None)):
+        with pytest.raises(ValueError):
+            step_end_(*bad, 1)
+    tok = torch.zeros(3, 1, dtype=i64, device=cuda)
+    emb = torch.zeros(5, 16, dtype=dt, device=cuda)
+    with pytest.raises(RuntimeError, match="is on cpu"):
+        step_begin(tok, tok, emb, emb, torch.nn.LayerNorm(16).to(dt), slots, lens)

@@ -196,3 +196,17 @@ def test_ln_linear_errors(cuda):
         ln_linear(x, torch.zeros(3, 2, 128, device=cuda), fc, ln, w, None)
     with pytest.raises(TypeError):
         ln_linear(x.float(), part[:, :2].contiguous(), fc, ln, w, None)
+
+
+@pytest.mark.parametrize("which", ["partials", "weight", "bias", "ln", "lin"])
+def test_ln_linear_operands_elsewhere(cuda, which):
+    """An operand on another device than x is refused on the host, before anything is launched."""
+    from whisperdrz_amd import ln_linear
+
+    dt = torch.bfloat16
+    a = {"partials": torch.zeros(2, 2, 128), "weight": torch.zeros(32, 128, dtype=dt), "bias": torch.zeros(32, dtype=dt),
+         "ln": torch.nn.LayerNorm(128).to(dt), "lin": torch.nn.Linear(8, 128).to(dt)}
+    a = {k: v if k == which else v.to(cuda) for k, v in a.items()}
+    x = torch.zeros(2, 128, dtype=dt, device=cuda)
+    with pytest.raises(RuntimeError, match="is on cpu"):
+        ln_linear(x, a["partials"], a["lin"], a["ln"], a["weight"], a["bias"])

@@ -201,6 +201,10 @@ def ln_linear(x: torch.Tensor, partials: torch.Tensor, lin: nn.Linear, ln: nn.La
         raise ValueError("the Linear must have a bias")
     w, b = weight.detach(), bias.detach() if bias is not None else None
     lw, lb, db = ln.weight.detach(), ln.bias.detach(), lin.bias.detach()
+    for name, t in (("partials", partials), ("weight", w), ("bias", b), ("ln.weight", lw), ("ln.bias", lb),
+                    ("lin.bias", db)):
+        if t is not None:
+            _check_cuda(name, t, x.device)
     if any(p is not None and p.dtype != x.dtype for p in (w, b, lw, lb, db)):
         raise TypeError("the LayerNorm and Linear parameters must have the activations' dtype")
     if w.stride(-1) != 1 or w.shape[1] != K or tuple(lw.shape) != (K,) or tuple(db.shape) != (K,):
@@ -229,7 +233,8 @@ def step_begin(tokens: torch.Tensor, positions: torch.Tensor, emb: torch.Tensor,
 
     ``tokens`` / ``positions`` int64 ``[B, sq]`` (any strides), 16-bit tables ``[n_vocab, n]`` /
     ``[n_ctx, n]``, ``slots`` int64 ``[B]``, ``lens`` int32 ``[n_layers, n_slots]`` contiguous."""
-    for name, t in (("emb", emb), ("pos_emb", pos_emb), ("tokens", tokens), ("positions", positions), ("lens", lens)):
+    for name, t in (("emb", emb), ("pos_emb", pos_emb), ("tokens", tokens), ("positions", positions), ("lens", lens),
+                    ("ln.weight", ln.weight), ("ln.bias", ln.bias)):
         _check_cuda(name, t, emb.device)
     if emb.dtype not in _LN16:
         raise TypeError(f"emb: dtype {emb.dtype} is not supported (bfloat16, float16)")
@@ -271,7 +276,20 @@ def step_begin(tokens: torch.Tensor, positions: torch.Tensor, emb: torch.Tensor,
 def step_end_(lens: torch.Tensor, seqlens: torch.Tensor, slots: Optional[torch.Tensor], sq: int) -> None:
     """``lens[:, slots] += sq`` (``lens[:, :B]`` without ``slots``) from the lengths ``seqlens`` that
     ``step_begin`` gathered."""
-    slots = slots.contiguous() if slots is not None else None
+    _check_cuda("lens", lens, lens.device)
+    _check_cuda("seqlens", seqlens, lens.device)
+    if lens.dtype != torch.int32 or seqlens.dtype != torch.int32:
+        raise TypeError("lens and seqlens must be int32")
+    if lens.dim() != 2 or seqlens.dim() != 2 or seqlens.shape[0] != lens.shape[0] or not lens.is_contiguous() \
+            or not seqlens.is_contiguous():
+        raise ValueError("lens and seqlens must be contiguous [n_layers, n_slots] and [n_layers, B]")
+    if slots is not None:
+        _check_cuda("slots", slots, lens.device)
+        if slots.dtype != torch.int64 or tuple(slots.shape) != (seqlens.shape[1],):
+            raise ValueError(f"slots must be int64 [{seqlens.shape[1]}]")
+        slots = slots.contiguous()
+    elif seqlens.shape[1] > lens.shape[1]:
+        raise ValueError(f"{seqlens.shape[1]} rows exceed the {lens.shape[1]} slots")
     rc = _lib.load().wdrz_step_end(lens.data_ptr(), seqlens.data_ptr(), slots.data_ptr() if slots is not None else None,
                                    seqlens.shape[1], sq, lens.shape[0], lens.shape[1], _stream_handle())
     if rc != _lib.WDRZ_OK:
