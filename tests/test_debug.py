@@ -84,3 +84,18 @@ def test_debug_library_exports_every_symbol():
     lib = ctypes.CDLL(str(_lib.DEBUG_LIB_PATH))
     _lib._declare(lib)  # raises AttributeError for a missing export
     assert lib.wdrz_abi_version() == _lib.ABI_VERSION
+
+
+def test_step_metadata():
+    import numpy as np
+
+    from whisperdrz_amd.debug import check_step_metadata
+
+    ok = dict(tokens=np.array([[0], [9]]), positions=np.array([[-4], [3]]), slots=np.array([-2, 1]), n_vocab=10,
+              n_ctx=4, n_slots=2)
+    check_step_metadata(**ok)
+    check_step_metadata(**{**ok, "slots": None})
+    for name, bad in (("tokens", [[-1], [0]]), ("tokens", [[0], [10]]), ("positions", [[4], [0]]),
+                      ("positions", [[-5], [0]]), ("slots", [2, 0]), ("slots", [-3, 0])):
+        with pytest.raises(IndexError, match=name[:-1]):
+            check_step_metadata(**{**ok, name: np.array(bad)})

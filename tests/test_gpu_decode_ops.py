@@ -218,3 +218,23 @@ def test_step_ends_operands(cuda):
     emb = torch.zeros(5, 16, dtype=dt, device=cuda)
     with pytest.raises(RuntimeError, match="is on cpu"):
         step_begin(tok, tok, emb, emb, torch.nn.LayerNorm(16).to(dt), slots, lens)
+
+
+@pytest.mark.parametrize("which", ["token", "position", "slot"])
+def test_step_begin_debug_mode_refuses_ids(cuda, monkeypatch, which):
+    """WDRZ_DEBUG=1: an id out of range is refused on the host instead of giving a NaN row."""
+    from whisperdrz_amd import _lib
+    from whisperdrz_amd.decode_ops import step_begin
+
+    monkeypatch.setenv("WDRZ_DEBUG", "1")
+    assert _lib.debug_mode()
+    ids = {"token": [[1], [2]], "position": [[0], [3]], "slot": [0, 1]}
+    emb = torch.zeros(5, 16, dtype=torch.bfloat16, device=cuda)
+    ln = torch.nn.LayerNorm(16).to(cuda, torch.bfloat16)
+    lens = torch.zeros(2, 4, dtype=torch.int32, device=cuda)
+    call = lambda i: step_begin(*(torch.tensor(i[k], device=cuda) for k in ("token", "position")), emb, emb, ln,
+                                torch.tensor(i["slot"], device=cuda), lens)
+    call(ids)
+    ids[which][1] = 9 if which == "slot" else [9]
+    with pytest.raises(IndexError, match=which):
+        call(ids)

@@ -2,7 +2,8 @@
 
 ``WDRZ_DEBUG=1`` makes :func:`whisperdrz_amd.flash_attn_with_kvcache` copy the slot ids and
 pre-append lengths of every call to the host and check them with :func:`check_kvcache_metadata`
-before launching (it also selects ``libwdrz_attn_debug.so``, whose C layer repeats the checks).
+before launching (it also selects ``libwdrz_attn_debug.so``, whose C layer repeats the checks), and
+a fused step's prologue check its ids with :func:`check_step_metadata`.
 The release path never reads device memory from the host, so it stays capture-safe; these checks
 do, so they are for debugging runs only.
 
@@ -18,7 +19,7 @@ from typing import Optional
 
 import numpy as np
 
-__all__ = ["check_kvcache_metadata", "force_torch", "probe"]
+__all__ = ["check_kvcache_metadata", "check_step_metadata", "force_torch", "probe"]
 
 
 def force_torch() -> bool:
@@ -59,3 +60,21 @@ def check_kvcache_metadata(cache_seqlens: Optional[np.ndarray], cache_batch_idx:
     if bad.size:
         i = int(bad[0])
         raise ValueError(f"row {i} appends [{int(cs[i])}, {int(cs[i]) + sq}) outside the cache [0, {max_seq})")
+
+
+def check_step_metadata(tokens: np.ndarray, positions: np.ndarray, slots: Optional[np.ndarray], n_vocab: int,
+                        n_ctx: int, n_slots: int) -> None:
+    """Check the ids of one cached step's prologue (host arrays).
+
+    Raises ``IndexError``, as torch's indexing does on the CPU, for a token outside ``[0, n_vocab)``,
+    a position outside ``[-n_ctx, n_ctx)`` or a slot outside ``[-n_slots, n_slots)``. Without the
+    checks the kernel reads nothing for such an id and the row's logits are NaN.
+    """
+    for name, ids, lo, hi in (("token", tokens, 0, n_vocab), ("position", positions, -n_ctx, n_ctx),
+                              ("slot", slots, -n_slots, n_slots)):
+        if ids is None:
+            continue
+        flat = np.asarray(ids, dtype=np.int64).reshape(-1)
+        bad = flat[(flat < lo) | (flat >= hi)]
+        if bad.size:
+            raise IndexError(f"{name} {int(bad[0])} outside [{lo}, {hi})")

@@ -232,7 +232,9 @@ def step_begin(tokens: torch.Tensor, positions: torch.Tensor, emb: torch.Tensor,
     the int32 slot map (None without ``slots``) and ``lens[:, slots]`` (``lens[:, :B]`` without).
 
     ``tokens`` / ``positions`` int64 ``[B, sq]`` (any strides), 16-bit tables ``[n_vocab, n]`` /
-    ``[n_ctx, n]``, ``slots`` int64 ``[B]``, ``lens`` int32 ``[n_layers, n_slots]`` contiguous."""
+    ``[n_ctx, n]``, ``slots`` int64 ``[B]``, ``lens`` int32 ``[n_layers, n_slots]`` contiguous. An id out
+    of range reads nothing and gives a NaN row (a slot: length -1, NaN from the attention); WDRZ_DEBUG=1
+    refuses it."""
     for name, t in (("emb", emb), ("pos_emb", pos_emb), ("tokens", tokens), ("positions", positions), ("lens", lens),
                     ("ln.weight", ln.weight), ("ln.bias", ln.bias)):
         _check_cuda(name, t, emb.device)
@@ -257,6 +259,11 @@ def step_begin(tokens: torch.Tensor, positions: torch.Tensor, emb: torch.Tensor,
         slots32 = torch.empty(B, dtype=torch.int32, device=e.device)
     elif B > lens.shape[1]:
         raise ValueError(f"{B} rows exceed the {lens.shape[1]} slots")
+    if _lib.debug_mode():  # host copies of the ids: debugging runs only, not graph capture
+        from .debug import check_step_metadata
+
+        check_step_metadata(tokens.cpu().numpy(), positions.cpu().numpy(),
+                            slots.cpu().numpy() if slots is not None else None, e.shape[0], p.shape[0], lens.shape[1])
     x = torch.empty(B, sq, n, dtype=e.dtype, device=e.device)
     h = torch.empty_like(x)
     seqlens = torch.empty(lens.shape[0], B, dtype=torch.int32, device=e.device)
