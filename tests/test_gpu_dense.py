@@ -305,7 +305,7 @@ def test_pipe_kernel_large_scores(cuda, case, Lq, causal):
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("L", [40, 200])
 def test_fp32_split_range_and_nonfinite(cuda, causal, L):
-    """fp32 operands far from 1 (the three-way split is exact at any scale), and infinities and NaN,
+    """fp32 operands far from 1 (the three-way split is exact from 2^-110 on), and infinities and NaN,
     which do not survive the split: the workgroup's queries then run on the fp32 matrix cores. Against
     64 bits within the file's fp32 tolerance (1e-5 of the largest value)."""
     from whisperdrz_amd import scaled_dot_product_attention
@@ -348,3 +348,27 @@ def test_fp32_split_range_and_nonfinite(cuda, causal, L):
     got = run(q, k2, v)
     rows = slice(L - 1, L) if causal else slice(0, L)
     assert got[0, 0, rows].isnan().all() and torch.isfinite(got[0, 1]).all()
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("L", [40, 200])
+@pytest.mark.parametrize("qs,ks,vs", [(1, 1, 1e-34), (1, 1, 3e-37), (1e-36, 1e36, 1), (1e36, 1e-36, 1), (1, 1, 0)])
+def test_fp32_tiny_operands(cuda, causal, L, qs, ks, vs):
+    """Normal fp32 operands below 2^-110, of which the three-way split loses the last bits: their
+    workgroups run on the fp32 matrix cores. Against 64 bits within the file's fp32 tolerance, over
+    the whole output and in one tiny column beside ordinary ones."""
+    from whisperdrz_amd import scaled_dot_product_attention
+
+    q, k, v = (randn((1, 2, L, 64), s, torch.float32) for s in (31, 32, 33))
+    q, k = q * qs, k * ks
+    for cols in (slice(0, 64), slice(5, 6)):
+        vc = v.clone()
+        vc[..., cols] *= vs
+        got = scaled_dot_product_attention(q.to(cuda), k.to(cuda), vc.to(cuda), is_causal=causal, scale=0.125)
+        s = (q.double() @ k.double().transpose(-1, -2)) * 0.125
+        if causal:
+            s = s.masked_fill(torch.ones(L, L, dtype=torch.bool).triu(1), float("-inf"))
+        want = torch.softmax(s, -1) @ vc.double()
+        for c in (slice(0, 64), slice(5, 6)):
+            err, top = (got.cpu().double() - want)[..., c].abs().max(), want[..., c].abs().max()
+            assert err <= 1e-5 * top, (cols, c, float(err), float(top))

@@ -5,17 +5,22 @@
 // L=1500 D=64, and the uncached decoder with a top-left causal mask). O = softmax(scale Q K^T) V
 // per (b, h), online softmax in the log2 domain, fp32 results.
 //
-// Products on the bf16 matrix cores, exactly split (split_tile): every fp32 operand is the sum of
-// three bf16 values, x = x0 + x1 + x2 (8 + 8 + 8 bits of the 24-bit significand, each rounded to
-// nearest, so the sum is exact), and x y is taken as x0 y0 + x0 y1 + x1 y0 + x1 y1 + x0 y2 + x2 y0,
-// accumulated in fp32; what is left out (x1 y2, x2 y1, x2 y2) is below 2^-25 of |x y|, less than one
-// fp32 rounding. 48 v_mfma_f32_32x32x16_bf16 of 32 cycles then do the work of 64
+// Products on the bf16 matrix cores, exactly split (split_tile): an fp32 operand of magnitude 2^-110
+// or more is the sum of three bf16 values, x = x0 + x1 + x2 (8 + 8 + 8 bits of the 24-bit significand,
+// each rounded to nearest), and x y is taken as x0 y0 + x0 y1 + x1 y0 + x1 y1 + x0 y2 + x2 y0,
+// accumulated in fp32; what is left out (x1 y2, x2 y1, x2 y2) is up to about 2^-24 of |x y|, one fp32
+// unit roundoff. 48 v_mfma_f32_32x32x16_bf16 of 32 cycles then do the work of 64
 // v_mfma_f32_32x32x2_f32 of 64 cycles per 32 x 32 step, and, unlike beside those, the softmax's VALU
-// instructions issue meanwhile. Measured, one encoder layer (B=1 H=20 L=1500): 110.6 -> 70.4
-// us, B=16 1641 -> 1081; causal 448 x 448, B=16: 176 -> 109; error against 64 bits 5.3e-7 -> 4.5e-7. Bound now: the MFMAs (24 for S^T, 24 for O^T, in
-// two wavefronts per SIMD) and the split of K, V and P on the VALU (11 instructions a pair).
-// Infinities and NaN do not survive the split (inf - inf): they give NaN output, and a workgroup
-// that computed one repeats its queries on the fp32 matrix cores (f32_tile), whose result stands.
+// instructions issue meanwhile. Measured, one encoder layer (B=1 H=20 L=1500): 110.6 -> 70.4 us, B=16
+// 1641 -> 1081; causal 448 x 448, B=16: 176 -> 109; error against 64 bits 5.3e-7 -> 4.5e-7. Bound now:
+// the MFMAs (24 for S^T, 24 for O^T, in two wavefronts per SIMD) and the split of K, V and P on the
+// VALU (11 instructions a pair).
+// Where the split falls short, the workgroup repeats its queries on the fp32 matrix cores (f32_tile),
+// whose result stands. Infinities and NaN do not survive it (inf - inf): they give NaN output. Below
+// 2^-110 the third part is below the smallest bf16 value and up to 2^-134 is lost: in V that shows
+// as an output below kTinyOut (zero among them, which values below 2^-134 alone give), in a query or
+// key only beside a huge partner, which queries of magnitude 2^-90 to 2^90 (or zero) rule out. (What
+// remains is a probability below 2^-110 times a value 2^110 above the others.)
 //
 // f32_tile: both products on v_mfma_f32_32x32x2_f32 (32x32 output, K = 2 per instruction, lane halves
 // h = lane / 32 supplying the two K slots):
@@ -126,8 +131,11 @@ __device__ __forceinline__ void f32_softmax(const DenseArgs& a, const F32Tile& p
   l_run += psum;
 }
 
+// Outputs below this (or NaN) and scaled queries beyond these are not left to the split operands.
+constexpr float kTinyOut = 0x1p-100f, kTinyQ = 0x1p-90f, kHugeQ = 0x1p90f;
+
 // Merges the two key halves of each query group through LDS (smem, free by now), normalises and
-// stores; true in a lane that stored a NaN.
+// stores; true in a lane that stored a NaN or a value below kTinyOut.
 __device__ __forceinline__ bool f32_merge_store(const DenseArgs& a, const F32Tile& p, float* smem, float m_run,
                                                 float l_run, const f32x16 (&acc_o)[2]) {
   const int lane = p.lane;
@@ -148,7 +156,7 @@ __device__ __forceinline__ bool f32_merge_store(const DenseArgs& a, const F32Til
   const float a0 = fast_exp2(m_run - m), a1 = fast_exp2(m1 - m);
   const float l_me = l_run * a0 + mg[33 * 64 + lane] * a1;
   const float inv = 1.f / (l_me + __shfl_xor(l_me, 32));
-  bool nan = false;
+  bool tiny = false;
   // lane holds dims 32 db + 8j + 4h + r (r = 0..3) of its query
   float* orow = p.O + (int64_t)p.q_me * a.os[2];
 #pragma unroll
@@ -160,11 +168,11 @@ __device__ __forceinline__ bool f32_merge_store(const DenseArgs& a, const F32Til
       for (int r = 0; r < 4; ++r) {
         const int x = 4 * j + r;
         w[r] = (acc_o[db][x] * a0 + mg[(16 * db + x) * 64 + lane] * a1) * inv;
-        nan = nan || w[r] != w[r];
+        tiny = tiny || !(fabsf(w[r]) >= kTinyOut);
       }
       store16(orow + 32 * db + 8 * j + 4 * p.hl, __builtin_bit_cast(u32x4, w));
     }
-  return nan;
+  return tiny;
 }
 
 // ---- the tile on the fp32 matrix cores -------------------------------------------------------------
@@ -306,7 +314,7 @@ __device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// Returns true in lanes that stored a NaN.
+// Returns true in lanes that saw operands or results which the split does not serve.
 template <bool CAUSAL>
 __device__ __forceinline__ bool split_tile(const DenseArgs& a, SplitStage* stage) {
   const F32Tile p = f32_place<CAUSAL>(a);
@@ -316,6 +324,8 @@ __device__ __forceinline__ bool split_tile(const DenseArgs& a, SplitStage* stage
 
   // Q, pre-scaled by c: plane i, instruction kk holds head dims 16 kk + 8h .. + 7 of this lane's query
   u32x4 qop[3][4];
+  float q_hi = 0.f;     // the largest |q| and, as bits 2 |q| - 1, the smallest that is not zero
+  uint32_t q_lo = ~0u;
   {
     const float* qp = p.Q + (int64_t)min(p.q_me, a.Lq - 1) * a.qs[2] + 8 * hl;
 #pragma unroll
@@ -323,6 +333,11 @@ __device__ __forceinline__ bool split_tile(const DenseArgs& a, SplitStage* stage
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const f32x4 v = __builtin_bit_cast(f32x4, load16(qp + 16 * kk + 4 * j));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          q_hi = fmaxf(q_hi, fabsf(v[e]));
+          q_lo = min(q_lo, (__float_as_uint(v[e]) << 1) - 1);
+        }
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           uint32_t w[3];
@@ -332,6 +347,8 @@ __device__ __forceinline__ bool split_tile(const DenseArgs& a, SplitStage* stage
         }
       }
   }
+  // (all zero: q_lo's float is NaN)
+  const bool q_range = q_hi * fabsf(a.c) > kHugeQ || __uint_as_float(q_lo >> 1) * fabsf(a.c) < kTinyQ;
 
   // Staging: thread t moves dims 4 (t % 16) .. + 3 of the keys 2 (t / 16) and + 1 of a stage, so that
   // V^T's key pairs are packed in one thread.
@@ -462,7 +479,7 @@ __device__ __forceinline__ bool split_tile(const DenseArgs& a, SplitStage* stage
     unit(u + 1, s_nxt, s_cur);
   }
   if (u < n_units) unit(u, s_cur, s_nxt);
-  return f32_merge_store(a, p, reinterpret_cast<float*>(stage), m_run, l_run, acc_o);
+  return f32_merge_store(a, p, reinterpret_cast<float*>(stage), m_run, l_run, acc_o) || q_range;
 }
 
 template <bool CAUSAL>
