@@ -1,6 +1,8 @@
 """Helpers shared by the parity tests (tolerances, seeded inputs, cache layouts)."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
 
@@ -45,3 +47,20 @@ def make_cache(n_slots, Lmax, H, D, dtype, device, layout, seed):
     ks = kc.permute(0, 2, 1, 3).contiguous().to(device)
     vs = vc.permute(0, 2, 1, 3).contiguous().to(device)
     return ks.permute(0, 2, 1, 3), vs.permute(0, 2, 1, 3)
+
+
+def splits_keys(q, kc, vc, k=None, v=None, seqlens=None, bidx=None) -> bool:
+    """Whether wdrz_attn_kvcache itself splits these keys (its size query allows for more): without a
+    workspace it refuses exactly then. A call that does not split runs, appending k / v."""
+    from whisperdrz_amd import _lib
+
+    lib = _lib.load()
+    code = {torch.bfloat16: _lib.WDRZ_BF16, torch.float16: _lib.WDRZ_F16, torch.float32: _lib.WDRZ_F32}[q.dtype]
+    (B, sq, H, D), out = q.shape, torch.empty_like(q)
+    ptr = lambda t: None if t is None else t.data_ptr()
+    st = lambda t: (ctypes.c_int64 * 4)(*(q if t is None else t).stride())
+    rc = lib.wdrz_attn_kvcache(code, ptr(q), ptr(kc), ptr(vc), ptr(k), ptr(v), ptr(seqlens), ptr(bidx), ptr(out),
+                               B, sq, H, D, kc.shape[0], kc.shape[1], st(q), st(kc), st(vc), st(k), st(v), st(out),
+                               ctypes.c_float(0.125), 1, None, 0, torch.cuda.current_stream().cuda_stream)
+    assert rc in (_lib.WDRZ_OK, _lib.WDRZ_EWORKSPACE), lib.wdrz_last_error().decode()
+    return rc == _lib.WDRZ_EWORKSPACE

@@ -78,6 +78,27 @@ def _strides(*s):
 FAKE = 0x10000  # 16-byte-aligned non-null pointer value; validation fails before any use
 
 
+def test_workspace_query_covers_the_16bit_plan(lib):
+    """The size query answers with the fp32 plan; whatever the 16-bit plan (fewer splits, blocks of 16
+    rows) asks for has to fit. A workspace of the queried size that is not aligned is refused for its
+    alignment, after its size; a call that needs none gets as far as the missing GPU."""
+    import torch
+
+    if torch.cuda.is_available():
+        pytest.skip("made-up pointers: only where nothing can be launched")
+    st, n_ws = _strides(1 << 20, 1 << 12, 64, 1), 0
+    for B, H in [(1, 1), (1, 2), (1, 20), (2, 20), (7, 20), (8, 16), (43, 3), (13, 20), (257, 1), (17, 20), (31, 11), (38, 9)]:
+        for sq in list(range(1, 18)) + [24, 25, 32, 33, 39, 40]:
+            for L in (767, 768, 769, 896, 1023, 1024, 1025, 1500, 1537, 3000, 6145, 50000):
+                size = lib.wdrz_attn_kvcache_workspace_size(B, sq, H, 64, L)
+                rc = lib.wdrz_attn_kvcache(2, FAKE, FAKE, FAKE, None, None, None, None, FAKE, B, sq, H, 64, B, L, st,
+                                           st, st, st, st, st, 0.125, 0, FAKE + 16, size, None)
+                assert rc in (1, 3), (B, H, sq, L, size, lib.wdrz_last_error())
+                n_ws += rc == 1
+                assert rc == 3 or (sq < 40 and L >= 768 and b"256-byte aligned" in lib.wdrz_last_error())
+    assert n_ws > 100
+
+
 def call_fwd(lib, **over):
     args = dict(dtype=2, q=FAKE, k=FAKE, v=FAKE, o=FAKE, B=1, H=2, Lq=8, Lk=8, D=64,
                 qs=_strides(1024, 512, 64, 1), ks=_strides(1024, 512, 64, 1), vs=_strides(1024, 512, 64, 1),

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from oracle.attention_oracle import kvcache_ref
-from tests._util import assert_close, make_cache, randn, to_np
+from tests._util import assert_close, make_cache, randn, splits_keys, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -81,14 +81,20 @@ def test_identity_batch_idx(cuda, self_attn):
           self_attn=self_attn, bidx_mode="none")
 
 
-@pytest.mark.parametrize("B,H,Lmax", [(1, 20, 448), (2, 20, 1500), (1, 1, 1500), (3, 5, 448)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,H,Lmax", [(1, 20, 448), (2, 20, 1500), (1, 1, 1500), (3, 5, 448), (5, 6, 800), (13, 20, 1030)])
 @pytest.mark.parametrize("self_attn", [True, False])
-def test_split_kv_paths(cuda, B, H, Lmax, self_attn):
-    """Small batches split the keys over several workgroups (workspace + combine pass)."""
+def test_split_kv_paths(cuda, dtype, B, H, Lmax, self_attn):
+    """Small batches split the keys over several workgroups (workspace + combine pass): fp32 at any
+    length, 16-bit rows from 768 keys on."""
     from whisperdrz_amd import kvcache_workspace_size
 
     assert kvcache_workspace_size(B, 1, H, D, Lmax) > 0
-    _case(cuda, torch.bfloat16, B=B, sq=1, H=H, n_slots=B + 2, Lmax=Lmax, layout="head_major", seed=300 + B,
+    kc, vc = make_cache(B, Lmax, H, D, dtype, cuda, "head_major", 1)
+    q, cs = randn((B, 1, H, D), 2, dtype).to(cuda), torch.zeros(B, dtype=torch.int32, device=cuda)
+    new = dict(k=q, v=q, seqlens=cs) if self_attn else {}
+    assert splits_keys(q, kc, vc, **new) == (dtype == torch.float32 or Lmax >= 768)
+    _case(cuda, dtype, B=B, sq=1, H=H, n_slots=B + 2, Lmax=Lmax, layout="head_major", seed=300 + B,
           self_attn=self_attn)
 
 
@@ -121,10 +127,11 @@ def _dup_metadata(B, sq, n_slots, Lmax, case, seed):
 def test_duplicate_slots_follow_reference_order(cuda, dtype, sq, B, case):
     """Repeated cache_batch_idx entries (bucket padding, transcriber.py:76-78, 165-167): the
     fallback appends row by row (model.py:51-54), so the last batch row covering a position wins,
-    and every row attends over the cache after all appends (model.py:55-57). B=6 takes the
-    split-KV path, 64 the one-row-per-workgroup path, 70 the metadata scan beyond one wavefront;
-    sq 1 / 5 / 12 / 48 reach kv_attn_kernel, kv_mq_kernel (bf16), the 8-row blocks and
-    kv_prefill_kernel (bf16)."""
+    and every row attends over the cache after all appends (model.py:55-57). B=70 takes
+    the metadata scan beyond one wavefront; B=6 splits its keys in fp32 (16-bit splits: the test
+    below). sq 1 / 5 / 12 / 48 reach in bf16 kv_attn_kernel, kv_mq_kernel, its 16-row blocks and, from
+    B=64 on, kv_prefill_kernel (B=6: the 16-row blocks); fp32 runs on kv_attn_kernel, in 8-row
+    blocks."""
     if dtype == torch.float32 and sq == 48 and B == 70:
         pytest.skip("fp32 keeps the VALU kernel at every sq; one fp32 case per batch shape is enough")
     print(f"dup case={case} dtype={dtype} sq={sq} B={B}", flush=True)
@@ -132,6 +139,23 @@ def test_duplicate_slots_follow_reference_order(cuda, dtype, sq, B, case):
     bidx, cs = _dup_metadata(B, sq, n_slots, Lmax, case, 1000 + sq + B)
     _case(cuda, dtype, B=B, sq=sq, H=H, n_slots=n_slots, Lmax=Lmax, layout="head_major", seed=700 + sq + B,
           cs=cs, bidx_np=bidx)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("sq", [1, 5, 12, 17])
+@pytest.mark.parametrize("case", ["identical", "overlap", "disjoint", "three"])
+def test_duplicate_slots_with_split_keys(cuda, dtype, sq, case):
+    """Repeated slot ids where the 16-bit kernels split the rows' keys: a region's positions then lie in
+    several workgroups' ranges, and the generic path's partials go through the merge."""
+    print(f"dup split case={case} dtype={dtype} sq={sq}", flush=True)
+    B, H, Lmax = 6, 3, 1500
+    bidx, cs = _dup_metadata(B, sq, B + 4, 300, case, 2000 + sq)
+    cs += (384 if sq <= 16 else 320) - sq // 2 - cs[0]  # row 0's region lies across two splits (of 192 / 320 keys)
+    kc, vc = make_cache(B + 4, Lmax, H, D, dtype, cuda, "head_major", 1)
+    q = randn((B, sq, H, D), 2, dtype).to(cuda)
+    assert splits_keys(q, kc, vc, q, q, torch.from_numpy(cs).to(cuda), torch.from_numpy(bidx).to(cuda))
+    _case(cuda, dtype, B=B, sq=sq, H=H, n_slots=B + 4, Lmax=Lmax, layout="head_major", seed=800 + sq, cs=cs,
+          bidx_np=bidx)
 
 
 def test_config3_shape_fp32_tolerance(cuda):
@@ -171,37 +195,39 @@ def test_verify_equals_sequential_steps(cuda):
         assert_close(out, to_np(seqout), dtype, "verify vs sequential")
 
 
-@pytest.mark.parametrize("sq", [1, 2, 5, 8, 9])
+@pytest.mark.parametrize("dtype,Lmax", [(torch.bfloat16, 1500), (torch.float32, 600)])
+@pytest.mark.parametrize("sq", [1, 2, 5, 8, 9, 17, 39])
 @pytest.mark.parametrize("self_attn", [True, False])
-def test_split_workspace_stays_in_bounds(cuda, sq, self_attn):
+def test_split_workspace_stays_in_bounds(cuda, dtype, Lmax, sq, self_attn):
     """Split-path calls touch exactly the workspace bytes the size query reports: a guard
     region right behind it keeps its bytes, and the workspace itself is left all-zero."""
     from whisperdrz_amd import flash_attn_with_kvcache, kvcache_workspace_size
 
-    B, H, Lmax = 2, 4, 600
+    B, H = 2, 4
     need = kvcache_workspace_size(B, sq, H, D, Lmax)
-    assert need > 0, "this shape is meant to take the split path"
     guard = 4096
     buf = torch.zeros(need + guard, dtype=torch.uint8, device=cuda)
     buf[need:] = 0xAB
     rng = np.random.default_rng(sq)
-    kc, vc = make_cache(B, Lmax, H, D, torch.bfloat16, cuda, "head_major", 70 + sq)
+    kc, vc = make_cache(B, Lmax, H, D, dtype, cuda, "head_major", 70 + sq)
     kc0, vc0 = to_np(kc), to_np(vc)
-    q = randn((B, sq, H, D), 71 + sq, torch.bfloat16).to(cuda)
+    q = randn((B, sq, H, D), 71 + sq, dtype).to(cuda)
     bidx_np = np.array([1, 0], dtype=np.int32)
     bidx = torch.from_numpy(bidx_np).to(cuda)
     print(f"workspace guard: sq={sq} self={self_attn} need={need}", flush=True)
     if self_attn:
-        k = randn((B, sq, H, D), 72 + sq, torch.bfloat16).to(cuda)
+        k = randn((B, sq, H, D), 72 + sq, dtype).to(cuda)
         cs = rng.integers(0, Lmax - sq + 1, size=B).astype(np.int32)
+        assert splits_keys(q, kc, vc, k, k, torch.from_numpy(cs).to(cuda), bidx), "meant to take the split path"
         out = flash_attn_with_kvcache(q, kc, vc, k=k, v=k, cache_seqlens=torch.from_numpy(cs).to(cuda),
                                       cache_batch_idx=bidx, softmax_scale=0.125, workspace=buf[:need])
         ref, _, _ = kvcache_ref(to_np(q), kc0, vc0, to_np(k), to_np(k), cs, bidx_np, 0.125)
     else:
+        assert splits_keys(q, kc, vc, bidx=bidx), "meant to take the split path"
         out = flash_attn_with_kvcache(q, kc, vc, cache_batch_idx=bidx, softmax_scale=0.125, workspace=buf[:need])
         ref, _, _ = kvcache_ref(to_np(q), kc0, vc0, None, None, None, bidx_np, 0.125)
     torch.cuda.synchronize()
-    assert_close(out, ref, torch.bfloat16, f"guarded workspace sq={sq}")
+    assert_close(out, ref, dtype, f"guarded workspace sq={sq}")
     assert int(torch.count_nonzero(buf[:need])) == 0, "workspace not left all-zero"
     assert bool((buf[need:] == 0xAB).all()), "bytes past the reported workspace size were written"
 
@@ -230,17 +256,19 @@ def test_bad_slot_gives_nan_not_fault(cuda, sq, self_attn):
     assert torch.equal(kc, snap_k)
 
 
-def test_prefill_bad_metadata_gives_nan_not_fault(cuda):
-    """The prefill kernel (sq >= 40): an out-of-range slot id and a row whose append would run past
-    the cache give NaN rows, no append and no memory access; the valid row is appended and finite."""
+@pytest.mark.parametrize("H", [2, 40])
+def test_prefill_bad_metadata_gives_nan_not_fault(cuda, H):
+    """70 queries on the 16-row blocks (2 heads: 30 of them) and on the prefill kernel (40 heads: 600):
+    an out-of-range slot id and a row whose append would run past the cache give NaN rows, no append
+    and no memory access; the valid row is appended and finite."""
     from whisperdrz_amd import flash_attn_with_kvcache
 
     sq, Lmax = 70, 128
-    kc, vc = make_cache(3, Lmax, 2, D, torch.bfloat16, cuda, "slot_major", 1)
+    kc, vc = make_cache(3, Lmax, H, D, torch.bfloat16, cuda, "slot_major", 1)
     snap_k, snap_v = kc.clone(), vc.clone()
-    q = randn((3, sq, 2, D), 2, torch.bfloat16).to(cuda)
-    k = randn((3, sq, 2, D), 3, torch.bfloat16).to(cuda)
-    v = randn((3, sq, 2, D), 4, torch.bfloat16).to(cuda)
+    q = randn((3, sq, H, D), 2, torch.bfloat16).to(cuda)
+    k = randn((3, sq, H, D), 3, torch.bfloat16).to(cuda)
+    v = randn((3, sq, H, D), 4, torch.bfloat16).to(cuda)
     bidx = torch.tensor([1, 3, 2], dtype=torch.int32, device=cuda)   # slot 3 is outside the pool
     seq = torch.tensor([5, 5, 60], dtype=torch.int32, device=cuda)   # 60 + 70 > 128
     out = flash_attn_with_kvcache(q, kc, vc, k=k, v=v, cache_seqlens=seq, cache_batch_idx=bidx, causal=True)
@@ -252,35 +280,39 @@ def test_prefill_bad_metadata_gives_nan_not_fault(cuda):
     assert torch.equal(kc, snap_k) and torch.equal(vc, snap_v)
 
 
-def test_workspace_reuse_across_shapes(cuda):
+@pytest.mark.parametrize("dtype,Lmax", [(torch.bfloat16, 1500), (torch.float16, 800), (torch.float32, 700)])
+def test_workspace_reuse_across_shapes(cuda, dtype, Lmax):
     """Split-path calls of different shapes share one workspace; each is correct and the
     workspace is all-zero after every call (its counters start at zero for the next one)."""
     from whisperdrz_amd import flash_attn_with_kvcache, kvcache_workspace_size
 
-    H, Lmax = 6, 700
-    shapes = [(1, 1), (3, 5), (2, 1), (1, 9), (4, 2), (1, 1)]
+    H = 6
+    # few rows and many in turn, 16-row blocks between: a call's counters lie over an earlier one's partials
+    shapes = [(1, 1), (3, 5), (2, 1), (1, 9), (4, 2), (1, 1), (1, 39), (21, 1), (2, 17), (10, 12), (1, 8)]
     need = max(kvcache_workspace_size(B, sq, H, D, Lmax) for B, sq in shapes)
     ws = torch.zeros(need, dtype=torch.uint8, device=cuda)
     for i, (B, sq) in enumerate(shapes):
         for self_attn in (True, False):
             print(f"reuse case {i}: B={B} sq={sq} self={self_attn}", flush=True)
             rng = np.random.default_rng(i)
-            kc, vc = make_cache(B + 1, Lmax, H, D, torch.bfloat16, cuda, "head_major", 40 + i)
+            kc, vc = make_cache(B + 1, Lmax, H, D, dtype, cuda, "head_major", 40 + i)
             kc0, vc0 = to_np(kc), to_np(vc)
-            q = randn((B, sq, H, D), 50 + i, torch.bfloat16).to(cuda)
+            q = randn((B, sq, H, D), 50 + i, dtype).to(cuda)
             bidx_np = rng.permutation(B + 1)[:B].astype(np.int32)
             bidx = torch.from_numpy(bidx_np).to(cuda)
             if self_attn:
-                k = randn((B, sq, H, D), 60 + i, torch.bfloat16).to(cuda)
+                k = randn((B, sq, H, D), 60 + i, dtype).to(cuda)
                 cs = rng.integers(0, Lmax - sq + 1, size=B).astype(np.int32)
+                assert splits_keys(q, kc, vc, k, k, torch.from_numpy(cs).to(cuda), bidx)
                 out = flash_attn_with_kvcache(q, kc, vc, k=k, v=k, cache_seqlens=torch.from_numpy(cs).to(cuda),
                                               cache_batch_idx=bidx, softmax_scale=0.125, workspace=ws)
                 ref, _, _ = kvcache_ref(to_np(q), kc0, vc0, to_np(k), to_np(k), cs, bidx_np, 0.125)
             else:
+                assert splits_keys(q, kc, vc, bidx=bidx)
                 out = flash_attn_with_kvcache(q, kc, vc, cache_batch_idx=bidx, softmax_scale=0.125, workspace=ws)
                 ref, _, _ = kvcache_ref(to_np(q), kc0, vc0, None, None, None, bidx_np, 0.125)
             torch.cuda.synchronize()
-            assert_close(out, ref, torch.bfloat16, f"reuse case {i}")
+            assert_close(out, ref, dtype, f"reuse case {i}")
             assert int(torch.count_nonzero(ws)) == 0, "workspace not left all-zero"
 
 

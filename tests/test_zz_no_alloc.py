@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from oracle.attention_oracle import kvcache_ref
-from tests._util import assert_close, make_cache, randn, to_np
+from tests._util import assert_close, make_cache, randn, splits_keys, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -48,8 +48,8 @@ def test_noalloc_matches_workspace_entry(cuda, self_attn):
     from whisperdrz_amd import _lib
 
     lib = _lib.load()
-    # first call larger than the second; both split their keys (workspace > 0)
-    shapes = [(3, 5, 20, 1500), (1, 1, 4, 448)]
+    # first call larger than the second; both split their keys
+    shapes = [(3, 5, 20, 1500), (1, 1, 4, 800)]
     for i, (B, sq, H, Lmax) in enumerate(shapes):
         need = lib.wdrz_attn_kvcache_workspace_size(B, sq, H, D, Lmax)
         assert 0 < need <= 4718592, need
@@ -73,6 +73,7 @@ def test_noalloc_matches_workspace_entry(cuda, self_attn):
         out_na = torch.empty((B, sq, H, D), dtype=torch.bfloat16, device=cuda)
         out_ws = torch.empty_like(out_na)
         ws = torch.zeros(need, dtype=torch.uint8, device=cuda)
+        assert splits_keys(q, kc, vc, k, v, seq, bidx)
         _call(lib, True, q, kc, vc, k, v, seq, bidx, out_na, None)
         _call(lib, False, q, kc2, vc2, k, v, seq, bidx, out_ws, ws)
         torch.cuda.synchronize()
