@@ -107,8 +107,9 @@ __device__ __forceinline__ void kv_append_store(const KvArgs& a, const AppendPie
 
 // Combines the per-wavefront partials (o[64], m, l per query, in LDS) of one workgroup and
 // writes the output rows, or, when the row's keys are split over several workgroups,
-// publishes this split's partial and lets the last split to arrive merge them all.
-template <typename T, int SQ, int kWaves>
+// publishes this split's partial and lets the last split to arrive merge them all. SPLIT false: the
+// launch splits no row.
+template <typename T, int SQ, int kWaves, bool SPLIT = true>
 __device__ __forceinline__ void kv_finish(const KvArgs& a, int b, int t0, int nq, int sq_stride, int h, int split,
                                           int n_split_b, bool bad, float (&sm_acc)[kWaves][SQ][kHeadDim],
                                           float (&sm_m)[kWaves][SQ], float (&sm_l)[kWaves][SQ]) {
@@ -141,7 +142,7 @@ __device__ __forceinline__ void kv_finish(const KvArgs& a, int b, int t0, int nq
     }
   };
 
-  if (n_split_b == 1) {
+  if (!SPLIT || n_split_b == 1) {
     for (int idx = tid; idx < nq * kHeadDim; idx += kThreads) {
       const int t = idx / kHeadDim, d = idx % kHeadDim;
       float O, M, L;
@@ -150,6 +151,7 @@ __device__ __forceinline__ void kv_finish(const KvArgs& a, int b, int t0, int nq
     }
     return;
   }
+  if constexpr (!SPLIT) return;
 
   // ---- several splits: publish this split's partial; the last split to arrive merges ----
   // Partials are laid out with the workspace's row stride sq_stride (= the launch's query block,
@@ -277,7 +279,10 @@ __device__ __forceinline__ void kv_general_row(const KvArgs& a, const AppendPiec
   kv_finish<T, SQ, kWaves>(a, b, t0, nq, sq_stride, h, split, n_split_b, false, sm_acc, sm_m, sm_l);
 }
 
-template <typename T, int SQ, bool HAS_NEW>
+// SPLIT false: the launch splits no row (self calls of 16-bit rows). Without the merge's code it is
+// shorter by 0.2-0.3 us: one stream, 10 / 100 / 200 keys 4.9 / 5.0 / 5.8 -> 4.6 / 4.7 / 5.5 us, 64 streams
+// of 400 keys 25.1 -> 24.8. Unsplit cross rows don't gain (8 / 16 streams 15.2 / 25.3 -> 15.5 / 25.1).
+template <typename T, int SQ, bool HAS_NEW, bool SPLIT>
 __global__ __launch_bounds__(kWavesPerWg * 64) void kv_attn_kernel(KvArgs a) {
   constexpr int kThreads = kWavesPerWg * 64;
   constexpr int kWaves = kWavesPerWg;
@@ -303,7 +308,7 @@ __global__ __launch_bounds__(kWavesPerWg * 64) void kv_attn_kernel(KvArgs a) {
   const int bq = (int)(blockIdx.x / (unsigned)a.H);
   const int b = bq / a.n_qblocks;
   const int t0 = (bq % a.n_qblocks) * SQ;
-  const int split = blockIdx.z;
+  const int split = SPLIT ? blockIdx.z : 0;
   const int nq = min(SQ, a.sq - t0);
 
   const int slot = a.bidx ? a.bidx[b] : b;
@@ -327,10 +332,10 @@ __global__ __launch_bounds__(kWavesPerWg * 64) void kv_attn_kernel(KvArgs a) {
   // Keys this query block needs: [0, key_lim).
   const int key_lim = HAS_NEW ? cs + t0 + nq : a.Lk;
   // Splits that hold keys of this row; the others have nothing to do.
-  const int n_split_b = bad ? 1 : max(1, (key_lim + a.split_len - 1) / a.split_len);
+  const int n_split_b = !SPLIT || bad ? 1 : max(1, (key_lim + a.split_len - 1) / a.split_len);
   if (split >= n_split_b) return;
   const int k_begin = split * a.split_len;
-  const int k_end = bad ? k_begin : min(key_lim, k_begin + a.split_len);
+  const int k_end = bad ? k_begin : SPLIT ? min(key_lim, k_begin + a.split_len) : key_lim;
   if (HAS_NEW && dup.general && !bad) {
     kv_general_row<T, SQ, kWaves>(a, app, b, h, slot, cs, t0, nq, SQ, split, n_split_b, k_begin, k_end, sm_acc,
                                   sm_m, sm_l);
@@ -511,7 +516,7 @@ __global__ __launch_bounds__(kWavesPerWg * 64) void kv_attn_kernel(KvArgs a) {
   }
   __syncthreads();
 
-  kv_finish<T, SQ, kWaves>(a, b, t0, nq, SQ, h, split, n_split_b, bad, sm_acc, sm_m, sm_l);
+  kv_finish<T, SQ, kWaves, SPLIT>(a, b, t0, nq, SQ, h, split, n_split_b, bad, sm_acc, sm_m, sm_l);
 }
 
 // ============================================================================================
@@ -774,8 +779,14 @@ __global__ __launch_bounds__(kWaves * 64, 4) void kv_mq_kernel(KvArgs a) {
 template <typename T, int SQ>
 void launch_row(const KvArgs& a, dim3 grid, hipStream_t stream) {
   const dim3 block(kWavesPerWg * 64);
-  if (a.kn) hipLaunchKernelGGL((kv_attn_kernel<T, SQ, true>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((kv_attn_kernel<T, SQ, false>), grid, block, 0, stream, a);
+  if constexpr (ElemBytes<T>::value == 2) {
+    if (a.kn && a.n_splits == 1) {
+      hipLaunchKernelGGL((kv_attn_kernel<T, SQ, true, false>), grid, block, 0, stream, a);
+      return;
+    }
+  }
+  if (a.kn) hipLaunchKernelGGL((kv_attn_kernel<T, SQ, true, true>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((kv_attn_kernel<T, SQ, false, true>), grid, block, 0, stream, a);
 }
 template <typename T, int SQ, int W>
 void launch_mq(const KvArgs& a, dim3 grid, hipStream_t stream) {
@@ -871,9 +882,10 @@ constexpr int64_t kCus = 256;
 constexpr int64_t kSplitWgs = 160;        // workgroups that splits of up to half the CUs' rows aim at
 constexpr int64_t kEvenRows = kCus * 4 / 3;
 constexpr int64_t kEvenWgs = 1024;
-// Self rows of 448 lose by any split (one stream with 200 / 400 keys 5.1 / 6.6 -> 6.6 / 7.2 us; the
-// one-stream step 238.3 -> 241.2 and 245.0 -> 243.1). Longer rows, one stream: 600 keys 6.8 / 6.9, 800
-// 8.1 / 7.4, 1000 9.1 / 7.5; four: 800 8.6 / 8.8, 1000 9.6 / 9.4.
+// Self rows of 448 lose by splits (of 128 keys: one stream with 10 / 100 / 200 / 300 / 440 keys 4.6 / 4.7 /
+// 5.5 / 6.4 / 7.2 -> 4.9 / 5.0 / 7.1 / 7.3 / 7.6 us, four with 300 6.6 -> 8.2; the one-stream step 241 -> 249).
+// Longer rows, one stream: 600 keys 6.8 / 6.9, 800 8.1 / 7.4, 1000 9.1 / 7.5; four: 800 8.6 / 8.8, 1000 9.6 /
+// 9.4.
 constexpr int64_t kSplitMinLk = 768;
 constexpr int64_t kSplitMinKeys = 192;    // one stream, cross: 12 splits of 128 keys 9.0 us, 8 of 192 8.4
 constexpr int64_t kEvenMinKeys = 512;
