@@ -135,15 +135,15 @@ def test_masked_argmax(cuda, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("V", [1, 7, 8, 9, 8191, 8193, 57344, 57353])
-def test_masked_argmax_vector_edges(cuda, dtype, V):
-    """Row lengths around the 8-token loads and one round of them (57344), rows and mask rows at
-    odd offsets (unaligned loads), the maximum at the first, last and last vectorised token; whole
-    numbers compared exactly."""
+@pytest.mark.parametrize("rows,V", [(5, V) for V in (1, 7, 8, 9, 2047, 2049, 4096, 4097, 8191, 8193, 57344, 57353)]
+                         + [(513, V) for V in (4, 14336, 14337)])
+def test_masked_argmax_vector_edges(cuda, dtype, rows, V):
+    """Row lengths around the 8-token loads, one round of them (14336 from 256 threads, 57344 from
+    1024) and the lines between the two forms, rows and mask rows at odd offsets (unaligned loads), the
+    maximum at the first, last and last vectorised token; whole numbers compared exactly."""
     from whisperdrz_amd import masked_argmax
 
     g = torch.Generator(device=cuda).manual_seed(V)
-    rows = 5
     logits = torch.randn(rows, V + 3, generator=g, device=cuda).to(dtype)[:, 1 : V + 1]
     blocked = (torch.rand(rows, V + 5, generator=g, device=cuda) < 0.2)[:, 3:]
     penalty = (torch.rand(rows, V + 2, generator=g, device=cuda) < 0.2)[:, 1:]

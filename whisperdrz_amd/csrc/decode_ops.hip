@@ -110,16 +110,15 @@ __device__ __forceinline__ bool argmax_beats(float v, int i, float b, int bi) {
 }
 
 // Bound: the row's bytes through one CU (2 or 4 B of logits plus 2 mask bytes per token) and the
-// latency of getting them. A 1024-thread workgroup takes a row, each thread 8 tokens at a time
-// with whole-word loads (logits 16 / 32 bytes, each mask 8 bytes; rows start at any element, so
+// latency of getting them. A workgroup (1024 threads, for short rows 256) takes a row, each thread 8 tokens
+// at a time with whole-word loads (logits 16 / 32 bytes, each mask 8 bytes; rows start at any element, so
 // the loads are unaligned), kArgmaxBatch of them requested before the first is used: a 51866-token
 // row is one round of requests. The 256-thread form before it loaded one token and two mask bytes
 // at a time. 52 rows x 51866 bf16 with both masks: 81 -> 12.3 us (kernel), 131 -> 11.9 us a call.
-constexpr int kArgmaxThreads = 1024;
 constexpr int kArgmaxVec = 8;    // tokens per load
-constexpr int kArgmaxBatch = 7;  // loads in flight per thread: 57344 tokens per round
+constexpr int kArgmaxBatch = 7;  // loads in flight per thread: 57344 tokens per round of 1024 threads
 
-template <typename T>
+template <typename T, int kArgmaxThreads>
 __global__ __launch_bounds__(kArgmaxThreads) void masked_argmax_kernel(ArgmaxArgs a) {
   constexpr int kWords = kArgmaxVec * ElemBytes<T>::value / 4;
   const int row = blockIdx.x;
@@ -263,12 +262,23 @@ hipError_t launch_step_end(const StepArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+template <typename T>
+static void launch_argmax_t(const ArgmaxArgs& a, hipStream_t stream) {
+  // 256 threads where 1024 mostly launch and reduce idle lanes: rows of two loads a thread, and more rows
+  // than two full workgroups a CU while one round of 256 threads' loads holds a row. Both masks, bf16, us,
+  // 1024 / 256 threads: 52 rows of 1000 5.1 / 3.9, of 4000 5.4 / 4.7; 600 rows of 1000 9.6 / 4.6, of 14000
+  // 17.4 / 14.5; 2000 rows of 8000 32.6 / 17.8.
+  const dim3 grid((unsigned)a.rows);
+  if (a.V <= 4096 || (a.rows > 512 && a.V <= 256 * kArgmaxVec * kArgmaxBatch))
+    hipLaunchKernelGGL((masked_argmax_kernel<T, 256>), grid, dim3(256), 0, stream, a);
+  else hipLaunchKernelGGL((masked_argmax_kernel<T, 1024>), grid, dim3(1024), 0, stream, a);
+}
+
 hipError_t launch_masked_argmax(int dtype, const ArgmaxArgs& a, hipStream_t stream) {
   if (a.rows == 0) return hipSuccess;
-  const dim3 grid((unsigned)a.rows);
-  if (dtype == 2) hipLaunchKernelGGL(masked_argmax_kernel<Bf16>, grid, dim3(kArgmaxThreads), 0, stream, a);
-  else if (dtype == 1) hipLaunchKernelGGL(masked_argmax_kernel<F16>, grid, dim3(kArgmaxThreads), 0, stream, a);
-  else hipLaunchKernelGGL(masked_argmax_kernel<F32>, grid, dim3(kArgmaxThreads), 0, stream, a);
+  if (dtype == 2) launch_argmax_t<Bf16>(a, stream);
+  else if (dtype == 1) launch_argmax_t<F16>(a, stream);
+  else launch_argmax_t<F32>(a, stream);
   return hipGetLastError();
 }
 
