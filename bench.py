@@ -63,6 +63,12 @@ def measured_traffic(kernel: str):
     return None if k is None else int(k["traffic_bytes"])
 
 
+def summed_traffic(kernels):
+    """`measured_traffic` of several kernels together, None where any of them was not measured."""
+    each = [measured_traffic(k) for k in kernels or ()]
+    return sum(each) if each and None not in each else None
+
+
 def timed_events(fn, iters: int, stream: torch.cuda.Stream) -> float:
     """Milliseconds per call of fn() over `iters` calls, timed with HIP events on `stream`."""
     start = torch.cuda.Event(enable_timing=True)
@@ -265,7 +271,7 @@ def bench_decode(dev, steps: int, warmup: int) -> dict:
                 "peak": PEAK_HBM_GBS,
                 "unit": "GB/s",
                 "frac": round(gbs / PEAK_HBM_GBS, 4),
-                "traffic": (sum(measured_traffic(k) or 0 for k in kernels) or None) if kernels else None,
+                "traffic": summed_traffic(kernels),
                 "traffic_source": "profiles/pmc_traffic.json (rocprofv3 FETCH_SIZE/WRITE_SIZE passes)",
                 "bytes_per_layer": bytes_per_layer,
             },
@@ -303,7 +309,7 @@ def bench_decode(dev, steps: int, warmup: int) -> dict:
     sumL3 = int(L3.sum())
     bytes3 = 2 * H * D * E * sumL3 + 2 * H * D * E * Bs + 2 * H * D * E * Bs + 8 * Bs
     res["config3_self_decode"] = run_graph("config3 self sq=1", body3, bytes3, {"sum_L": sumL3},
-                                           kernels=("kv_attn_kernel<wdrz::Bf16, 1, true>",))
+                                           kernels=("kv_attn_kernel<wdrz::Bf16, 1, true, false>",))
 
     # ---- config 4: cross-attention decode, sq=1, 1500 keys per stream ----
     q4 = [q_new(6000 + i, 1)[0] for i in range(N_LAYERS)]
@@ -319,7 +325,7 @@ def bench_decode(dev, steps: int, warmup: int) -> dict:
         "config4 cross sq=1", body4, bytes4,
         {"inputs": "per layer K = xa W_k, V = xa W_v with xa ~ N(0,1) [64, 1500, 1280] bf16 (one simulated "
                    "encoder output) and seeded W_k, W_v ~ N(0, 1/1280) [1280, 1280] per layer; queries ~ N(0,1)"},
-        kernels=("kv_attn_kernel<wdrz::Bf16, 1, false>",))
+        kernels=("kv_attn_kernel<wdrz::Bf16, 1, false, true>",))
 
     # ---- config 5: 5-token draft verify (self, causal within the draft) + cross ----
     sq = 5
@@ -344,7 +350,7 @@ def bench_decode(dev, steps: int, warmup: int) -> dict:
     res["config5_verify_self_plus_cross"] = run_graph(
         "config5 verify sq=5 (self+cross)", body5, bytes5_self + bytes5_cross,
         {"sum_L": sumL5, "bytes_self_per_layer": bytes5_self, "bytes_cross_per_layer": bytes5_cross},
-        kernels=("kv_mq_kernel<wdrz::Bf16, true, 8>", "kv_mq_kernel<wdrz::Bf16, false, 8>"),
+        kernels=("kv_mq_kernel<wdrz::Bf16, true, 8, 4>", "kv_mq_kernel<wdrz::Bf16, false, 8, 4>"),
     )
     # ---- prefill: a 224-token prompt into empty self caches (the window's first call) ----
     sqp = 224
@@ -466,7 +472,7 @@ def bench_dtw(dev, steps: int, warmup: int) -> dict:
             "peak": PEAK_HBM_GBS,
             "unit": "GB/s",
             "frac": round(gbs / PEAK_HBM_GBS, 4),
-            "traffic": (sum(measured_traffic(k) or 0 for k in DTW_KERNELS) or None),
+            "traffic": summed_traffic(DTW_KERNELS),
             "traffic_source": "profiles/pmc_traffic.json (rocprofv3 FETCH_SIZE/WRITE_SIZE passes)",
             "bytes_per_prep": nbytes,
             "kernels": list(DTW_KERNELS),
@@ -1050,10 +1056,10 @@ def cpu_baseline(budget_s: float = 12.0) -> dict:
 # read and write at least), against which the measured traffic is compared.
 _ALG_BYTES = {
     "dense_pipe_kernel<wdrz::Bf16, 3>": 4 * 16 * 1500 * 20 * 64 * 2,  # Q + K + V + O
-    "kv_attn_kernel<wdrz::Bf16, 1, true>": 68526592,
-    "kv_attn_kernel<wdrz::Bf16, 1, false>": 491847936,
-    "kv_mq_kernel<wdrz::Bf16, true, 8>": 75279872,
-    "kv_mq_kernel<wdrz::Bf16, false, 8>": 493158656,
+    "kv_attn_kernel<wdrz::Bf16, 1, true, false>": 68526592,
+    "kv_attn_kernel<wdrz::Bf16, 1, false, true>": 491847936,
+    "kv_mq_kernel<wdrz::Bf16, true, 8, 4>": 75279872,
+    "kv_mq_kernel<wdrz::Bf16, false, 8, 4>": 493158656,
     "dtw_rowcol_kernel<6>": 430080000,
     "dtw_seg_kernel": 430080000 + 43008000,
     "dtw_qk_kernel<wdrz::Bf16>": 430080000 + 2 * 16 * 10 * (448 + 1500) * 64,
