@@ -12,9 +12,9 @@
 // unit roundoff. 48 v_mfma_f32_32x32x16_bf16 of 32 cycles then do the work of 64
 // v_mfma_f32_32x32x2_f32 of 64 cycles per 32 x 32 step, and, unlike beside those, the softmax's VALU
 // instructions issue meanwhile. Measured, one encoder layer (B=1 H=20 L=1500): 110.6 -> 70.4 us, B=16
-// 1641 -> 1081; causal 448 x 448, B=16: 176 -> 109; error against 64 bits 5.3e-7 -> 4.5e-7. Bound now:
-// the MFMAs (24 for S^T, 24 for O^T, in two wavefronts per SIMD) and the split of K, V and P on the
-// VALU (11 instructions a pair).
+// 1641 -> 1081; causal 448 x 448, B=16: 176 -> 109; error against 64 bits 5.3e-7 -> 4.5e-7. Bound now,
+// by counters: VALU issue (softmax, and the split of K, V and P, 11 instructions a pair) takes 56% and the
+// MFMAs (24 for S^T, 24 for O^T a step) 47% of the SIMDs' busy cycles, 20% both at once.
 // Where the split falls short, the workgroup repeats its queries on the fp32 matrix cores (f32_tile),
 // whose result stands. Infinities and NaN do not survive it (inf - inf): they give NaN output. Below
 // 2^-110 the third part is below the smallest bf16 value and up to 2^-134 is lost: in V that shows

@@ -22,10 +22,11 @@
 // Why an FFT: the direct transform on the fp32 matrix cores (a [32 x 400] x [400 x 512] product
 // per 32 frames, the form before this one) took 240 us for 16 windows of 30 s and 50 us for one,
 // after an init launch that rebuilt its tables (3.3 us); the 55 MB this must move take 11 us. Now
-// 60 us for 16 windows and 14 us for one (a whole call 237 -> 72 and 53.6 -> 16.5 us), and nearer
-// to 64-bit results (3.6e-7 against 5.3e-7). What bounds it: half of a wavefront's cycles are VALU
-// issue (~1700 instructions per 6 frames, a third of them the filterbank and log10), half waits
-// for samples, LDS and the other wavefronts of its phase; no part's removal takes more than a sixth
+// 62-67 us for 16 windows and 14-15 us for one (a whole call 237 -> 71 and 53.6 -> 16.4 us), and nearer
+// to 64-bit results (3.6e-7 against 5.3e-7). What bounds it, by counters (16 windows): VALU issue
+// takes 46% of the SIMDs' busy cycles (1940 instructions per wavefront, i.e. per 6 frames) with 1.8
+// wavefronts on a SIMD on average; a wavefront issues them for a quarter of its time and waits for
+// half of it, for samples, LDS and the other wavefronts at a barrier. No part's removal takes more than a sixth
 // (transforms' arithmetic 3 us, filterbank loop 12, filter weights 3, stores 4 of the call's 76 us
 // when it was measured).
 #include <hip/hip_runtime.h>
